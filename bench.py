@@ -634,9 +634,9 @@ def bench_mlp(torch, ctx, clock):
                         "mfma_frac": f_tf / BF16_PEAK_TF},
             "backward": {"kernel_ms": b_ms, "moves_per_s": B / (b_ms / 1e3), "tflops": b_tf,
                          "mfma_frac": b_tf / BF16_PEAK_TF},
-            "note": "forward 41,216 flop/move, backward 73,984 (weight and input gradients, "
-                    "after its own forward); the GEMMs are 16x16 BF16 MFMA tiles of one wave, "
-                    "so at 128 hidden units the launches are latency-bound"}
+            "note": "forward 41,216 flop/move, backward 73,984 (weight and input gradients; its "
+                    "time includes its own forward); one fused launch each way with the "
+                    "activations on chip, bound by the FP32 erf / exp of GELU"}
 
 
 def bench_config0(ctx):

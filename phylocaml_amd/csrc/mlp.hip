@@ -159,6 +159,303 @@ __global__ void k_adam(float* __restrict__ p, const float* __restrict__ g, float
   p[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
 }
 
+// ---------------------------------------------------------------------------
+// Fused pass for small networks (n_in <= 64, H = 64 or 128): forward, or
+// forward + backward, of 32 rows of the batch at a time with every activation
+// on chip.
+//
+// A block is H / 16 waves; wave w owns hidden units 16w .. 16w+15 of both
+// layers and holds its slices of W1, W2^T and W2 as BF16 MFMA operands in
+// registers for the whole launch.  Products are formed transposed (A = weights,
+// B = activations), so a lane holds 4 units (16w + 4q + v) of one row (lane
+// l: row l % 16 of each 16-row group, q = l / 16): GELU, its derivative, the
+// loss and the bias / output-layer sums run in FP32 registers, and only the
+// BF16 operands of the next product pass through LDS.  Weight gradients
+// contract over the rows (one K = 32 MFMA step a tile) from unit-major copies,
+// accumulate in registers over the block's tiles and leave as one partial
+// per block, summed in a fixed order by k_mlp_sum.
+//
+// One wave per 16x16 tile with activations in memory (the k_gemm path below)
+// spent 219 us on 65,536 rows forward and 1.25 ms backward, in strided 4-byte
+// loads and 19 launches; here 20 us forward (one launch) and 89 us forward and
+// backward (two launches); 1,024 rows forward and backward take 18 us.  The
+// bound is the VALU: two erff a row and hidden unit (ocml's two branches, ~40
+// instructions each) forward, two erff and two expf more backward.
+// ---------------------------------------------------------------------------
+constexpr int kMlpRows = 32;     // rows of a tile (the K of the weight gradients)
+constexpr int kMlpMaxIn = 64;
+
+struct MlpArgs {
+  const float *X, *T, *W1, *b1, *W2, *b2, *w3, *b3;
+  float* y;      // forward: outputs (backward: nullptr)
+  float* part;   // backward: [blocks][n_params] gradient partials
+  double* lpart; // backward: [blocks] loss partials
+  int64_t B, n_params;
+  int n_in, vec4;  // vec4: rows of X can be read 16 bytes at a time
+};
+
+__device__ __forceinline__ f32x4 mfma16(const bf16x8 a, const bf16x8 b, const f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// sum over the 16 lanes of a row (every lane gets it)
+__device__ __forceinline__ float row16_sum(float v) {
+#pragma unroll
+  for (int off = 1; off < 16; off <<= 1) v += __shfl_xor(v, off, 64);
+  return v;
+}
+
+// W = waves per block = H / 16; KC = 32-feature chunks of the input
+template <int W, int KC, bool BWD>
+__global__ __launch_bounds__(64 * W) void k_mlp_fused(MlpArgs a) {
+  constexpr int H = 16 * W, HC = H / 32, G = kMlpRows / 16;
+  constexpr int RS = H + 8;         // row-major stride (bf16): 16-byte rows, staggered banks
+  constexpr int US = kMlpRows + 8;  // unit-major stride
+  __shared__ __attribute__((aligned(16))) __bf16 hr[kMlpRows * RS];  // H1, then dZ2, [row][unit]
+  __shared__ float ys[W][kMlpRows];
+  __shared__ __attribute__((aligned(16))) __bf16 ht[BWD ? H * US : 8];   // H1 [unit][row]
+  __shared__ __attribute__((aligned(16))) __bf16 d2t[BWD ? H * US : 8];  // dZ2 [unit][row]
+  __shared__ __attribute__((aligned(16))) __bf16 d1t[BWD ? H * US : 8];  // dZ1 [unit][row]
+  __shared__ __attribute__((aligned(16))) __bf16 xt[BWD ? 32 * KC * US : 8];  // X [feature][row]
+  const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int q = l >> 4, c = l & 15;
+  const int u0 = 16 * w + 4 * q;  // the lane's 4 units
+
+  bf16x8 a1[KC], a2[HC], a2t[BWD ? HC : 1];
+#pragma unroll
+  for (int k = 0; k < KC; ++k)
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      const int i = 32 * k + 8 * q + v;
+      a1[k][v] = (__bf16)(i < a.n_in ? a.W1[(int64_t)i * H + 16 * w + c] : 0.0f);
+    }
+#pragma unroll
+  for (int k = 0; k < HC; ++k)
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+      const int i = 32 * k + 8 * q + v;
+      a2[k][v] = (__bf16)a.W2[i * H + 16 * w + c];
+      if (BWD) a2t[k][v] = (__bf16)a.W2[(16 * w + c) * H + i];
+    }
+  float b1[4], b2[4], w3[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    b1[v] = a.b1[u0 + v];
+    b2[v] = a.b2[u0 + v];
+    w3[v] = a.w3[u0 + v];
+  }
+  const float b3 = a.b3[0];
+
+  f32x4 gW2[BWD ? W : 1], gW1[BWD ? 2 * KC : 1];
+  float gb1[4] = {0.f, 0.f, 0.f, 0.f}, gb2[4] = {0.f, 0.f, 0.f, 0.f}, gw3[4] = {0.f, 0.f, 0.f, 0.f}, gb3 = 0.f;
+  double loss = 0.0;
+#pragma unroll
+  for (int j = 0; j < (BWD ? W : 1); ++j) gW2[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < (BWD ? 2 * KC : 1); ++j) gW1[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int64_t tiles = (a.B + kMlpRows - 1) / kMlpRows;
+  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const int64_t row0 = tile * kMlpRows;
+    // layer 1; the activations' derivatives stay in registers
+    float g1[G][4];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int64_t row = row0 + 16 * g + c;
+      const float* x = a.X + (row < a.B ? row : a.B - 1) * a.n_in;
+      f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < KC; ++k) {
+        const int i0 = 32 * k + 8 * q;
+        float xv[8];
+        if (a.vec4) {  // n_in is a multiple of 4 and the rows are 16-byte aligned
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            float4 t4 = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (i0 + 4 * h < a.n_in) t4 = *reinterpret_cast<const float4*>(x + i0 + 4 * h);
+            xv[4 * h] = t4.x;
+            xv[4 * h + 1] = t4.y;
+            xv[4 * h + 2] = t4.z;
+            xv[4 * h + 3] = t4.w;
+          }
+        } else {
+#pragma unroll
+          for (int v = 0; v < 8; ++v) xv[v] = i0 + v < a.n_in ? x[i0 + v] : 0.0f;
+        }
+        bf16x8 b;
+#pragma unroll
+        for (int v = 0; v < 8; ++v) b[v] = (__bf16)xv[v];
+        z = mfma16(a1[k], b, z);
+        if (BWD && w == 0) {  // unit-major copy for dW1; rows past the batch meet dZ1 = 0
+#pragma unroll
+          for (int v = 0; v < 8; ++v) xt[(i0 + v) * US + 16 * g + c] = b[v];
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float zv = z[v] + b1[v];
+        const __bf16 h = (__bf16)gelu(zv);
+        hr[(16 * g + c) * RS + u0 + v] = h;
+        if (BWD) {
+          ht[(u0 + v) * US + 16 * g + c] = h;
+          g1[g][v] = gelu_grad(zv);
+        }
+      }
+    }
+    __syncthreads();
+    // layer 2 and the output layer
+    float z2[G][4];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < HC; ++k)
+        z = mfma16(a2[k], *reinterpret_cast<const bf16x8*>(&hr[(16 * g + c) * RS + 32 * k + 8 * q]), z);
+      float s = 0.f;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        z2[g][v] = z[v] + b2[v];
+        s += gelu(z2[g][v]) * w3[v];
+      }
+      s += __shfl_xor(s, 16, 64);
+      s += __shfl_xor(s, 32, 64);
+      if (q == 0) ys[w][16 * g + c] = s;
+    }
+    __syncthreads();
+    if (!BWD) {
+      // hr is rewritten only after this barrier (every wave has read it), ys
+      // only after the next tile's first barrier
+      if (threadIdx.x < kMlpRows && row0 + threadIdx.x < a.B) {
+        float s = 0.f;
+#pragma unroll
+        for (int k = 0; k < W; ++k) s += ys[k][threadIdx.x];
+        a.y[row0 + threadIdx.x] = s + b3;
+      }
+      continue;
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const int64_t row = row0 + 16 * g + c;
+      float s = 0.f;
+#pragma unroll
+      for (int k = 0; k < W; ++k) s += ys[k][16 * g + c];
+      const float d = row < a.B ? (s + b3) - a.T[row] : 0.0f;
+      const float dy = d / (float)a.B;
+      if (w == 0 && q == 0) {
+        loss += 0.5 * (double)d * (double)d / (double)a.B;
+        gb3 += dy;
+      }
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float zv = z2[g][v];
+        gw3[v] += gelu(zv) * dy;
+        const float dz = dy * w3[v] * gelu_grad(zv);
+        gb2[v] += dz;
+        const __bf16 h = (__bf16)dz;
+        hr[(16 * g + c) * RS + u0 + v] = h;
+        d2t[(u0 + v) * US + 16 * g + c] = h;
+      }
+    }
+    __syncthreads();
+    // dZ1 = (W2 dZ2) * gelu'(Z1)
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < HC; ++k)
+        z = mfma16(a2t[k], *reinterpret_cast<const bf16x8*>(&hr[(16 * g + c) * RS + 32 * k + 8 * q]), z);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float dz = z[v] * g1[g][v];
+        gb1[v] += dz;
+        d1t[(u0 + v) * US + 16 * g + c] = (__bf16)dz;
+      }
+    }
+    // dW2 (units of layer 1 of this wave x every unit of layer 2)
+    {
+      const bf16x8 ah = *reinterpret_cast<const bf16x8*>(&ht[(16 * w + c) * US + 8 * q]);
+#pragma unroll
+      for (int j = 0; j < W; ++j)
+        gW2[j] = mfma16(ah, *reinterpret_cast<const bf16x8*>(&d2t[(16 * j + c) * US + 8 * q]), gW2[j]);
+    }
+    __syncthreads();  // d1t written; hr, ht, d2t read
+    // dW1 (every feature x the units of this wave)
+    {
+      const bf16x8 bd = *reinterpret_cast<const bf16x8*>(&d1t[(16 * w + c) * US + 8 * q]);
+#pragma unroll
+      for (int j = 0; j < 2 * KC; ++j)
+        gW1[j] = mfma16(*reinterpret_cast<const bf16x8*>(&xt[(16 * j + c) * US + 8 * q]), bd, gW1[j]);
+    }
+    __syncthreads();  // xt read
+  }
+  if (!BWD) return;
+  // the block's partial gradient, laid out as the parameters
+  float* p = a.part + (int64_t)blockIdx.x * a.n_params;
+#pragma unroll
+  for (int j = 0; j < 2 * KC; ++j)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int i = 16 * j + 4 * q + v;
+      if (i < a.n_in) p[(int64_t)i * H + 16 * w + c] = gW1[j][v];
+    }
+  p += (int64_t)a.n_in * H;
+  float* pW2 = p + H;
+#pragma unroll
+  for (int j = 0; j < W; ++j)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) pW2[(int64_t)(u0 + v) * H + 16 * j + c] = gW2[j][v];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {
+    const float s1 = row16_sum(gb1[v]), s2 = row16_sum(gb2[v]), s3 = row16_sum(gw3[v]);
+    if (c == 0) {
+      p[u0 + v] = s1;
+      pW2[(int64_t)H * H + u0 + v] = s2;
+      pW2[(int64_t)H * H + H + u0 + v] = s3;
+    }
+  }
+  if (w == 0) {
+    const float s = row16_sum(q == 0 ? gb3 : 0.f);
+    double e = q == 0 ? loss : 0.0;
+#pragma unroll
+    for (int off = 1; off < 16; off <<= 1) e += __shfl_xor(e, off, 64);
+    if (l == 0) {
+      pW2[(int64_t)H * H + 2 * H] = s;
+      a.lpart[blockIdx.x] = e;
+    }
+  }
+}
+
+// Sums of the per-block partials in a fixed order: 64 parameters a block,
+// the partials dealt to its 4 waves.  The last block of the grid sums the
+// loss.  out2 (nullable) receives a second copy of the gradients.
+__global__ __launch_bounds__(256) void k_mlp_sum(const float* __restrict__ part, int parts, int64_t n,
+                                                 const double* __restrict__ lpart, float* __restrict__ out,
+                                                 float* __restrict__ out2, double* __restrict__ loss) {
+  __shared__ float sh[4][64];
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  if (blockIdx.x == gridDim.x - 1) {
+    if (threadIdx.x == 0 && loss) {
+      double e = 0.0;
+      for (int z = 0; z < parts; ++z) e += lpart[z];
+      *loss = e;
+    }
+    return;
+  }
+  const int64_t i = (int64_t)blockIdx.x * 64 + l;
+  float s = 0.f;
+  if (i < n) {
+#pragma unroll 8
+    for (int z = w; z < parts; z += 4) s += part[(int64_t)z * n + i];
+  }
+  sh[w][l] = s;
+  __syncthreads();
+  if (w == 0 && i < n) {
+    s = (sh[0][l] + sh[1][l]) + (sh[2][l] + sh[3][l]);
+    out[i] = s;
+    if (out2) out2[i] = s;
+  }
+}
+
 struct Views {
   float *W1, *b1, *W2, *b2, *w3, *b3;
 };
@@ -285,6 +582,92 @@ int backward(phy_ctx* ctx, phy_mlp* m, const float* X, const float* t, int64_t B
   return PHY_OK;
 }
 
+// The fused pass covers networks of up to 64 inputs with 64 or 128 hidden
+// units (its weights fit a block's registers); other sizes take the GEMMs.
+bool fused_fits(const phy_mlp* m) { return m->n_in <= kMlpMaxIn && (m->H == 64 || m->H == 128); }
+
+// blocks of a fused launch, at most one per tile of rows: backward one a CU
+// (each leaves a partial gradient, 84 KB at H = 128), forward three (what its
+// registers keep resident; 65,536 rows: 28.5 / 22.1 / 20.3 / 22.4 us at
+// 1 / 2 / 3 / 4 a CU)
+int fused_blocks(const phy_ctx* ctx, int64_t B, bool bwd) {
+  int n_cu = 256;
+  (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, ctx->device);
+  return (int)std::min<int64_t>((B + kMlpRows - 1) / kMlpRows, (int64_t)n_cu * (bwd ? 1 : 3));
+}
+
+MlpArgs fused_args(const phy_mlp* m, const float* X, const float* T, int64_t B) {
+  const Views p = views(m->params, m->n_in, m->H);
+  MlpArgs a{};
+  a.X = X;
+  a.T = T;
+  a.W1 = p.W1;
+  a.b1 = p.b1;
+  a.W2 = p.W2;
+  a.b2 = p.b2;
+  a.w3 = p.w3;
+  a.b3 = p.b3;
+  a.B = B;
+  a.n_params = m->n_params;
+  a.n_in = m->n_in;
+  a.vec4 = m->n_in % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0;
+  return a;
+}
+
+template <bool BWD>
+void fused_launch(phy_ctx* ctx, const phy_mlp* m, int blocks, const MlpArgs& a) {
+  const bool wide = m->n_in > 32;
+  const dim3 g((unsigned)blocks), t((unsigned)(4 * m->H));
+  if (m->H == 128) {
+    if (wide)
+      hipLaunchKernelGGL((k_mlp_fused<8, 2, BWD>), g, t, 0, ctx->stream, a);
+    else
+      hipLaunchKernelGGL((k_mlp_fused<8, 1, BWD>), g, t, 0, ctx->stream, a);
+  } else {
+    if (wide)
+      hipLaunchKernelGGL((k_mlp_fused<4, 2, BWD>), g, t, 0, ctx->stream, a);
+    else
+      hipLaunchKernelGGL((k_mlp_fused<4, 1, BWD>), g, t, 0, ctx->stream, a);
+  }
+}
+
+int ensure_ws(phy_ctx* ctx, phy_mlp* m, int64_t need) {
+  if (m->ws_floats >= need) return PHY_OK;
+  if (m->ws) PHY_HIP(ctx, hipFree(m->ws));
+  m->ws = nullptr;
+  m->ws_floats = 0;
+  PHY_HIP(ctx, hipMalloc((void**)&m->ws, sizeof(float) * (size_t)need));
+  m->ws_floats = need;
+  return PHY_OK;
+}
+
+int fused_forward(phy_ctx* ctx, phy_mlp* m, const float* X, int64_t B, float* y) {
+  MlpArgs a = fused_args(m, X, nullptr, B);
+  a.y = y;
+  KernelSpan span(ctx, "mlp_forward");
+  fused_launch<false>(ctx, m, fused_blocks(ctx, B, false), a);
+  PHY_LAUNCHED(ctx);
+  return PHY_OK;
+}
+
+int fused_backward(phy_ctx* ctx, phy_mlp* m, const float* X, const float* T, int64_t B, float* d_grads,
+                   double* d_loss) {
+  const int blocks = fused_blocks(ctx, B, true);
+  // loss partials (8-byte aligned) ahead of the gradient partials
+  const int rc = ensure_ws(ctx, m, 2 * (int64_t)blocks + blocks * m->n_params);
+  if (rc) return rc;
+  MlpArgs a = fused_args(m, X, T, B);
+  a.lpart = reinterpret_cast<double*>(m->ws);
+  a.part = m->ws + 2 * (int64_t)blocks;
+  KernelSpan span(ctx, "mlp_backward");
+  fused_launch<true>(ctx, m, blocks, a);
+  PHY_LAUNCHED(ctx);
+  hipLaunchKernelGGL(k_mlp_sum, dim3((unsigned)((m->n_params + 63) / 64 + 1)), dim3(256), 0, ctx->stream, a.part,
+                     blocks, m->n_params, a.lpart, m->grads, d_grads, d_loss);
+  PHY_LAUNCHED(ctx);
+  return PHY_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -355,6 +738,7 @@ int phy_mlp_forward(phy_ctx* ctx, phy_mlp* m, const float* d_x, int64_t B, float
   if (!ctx || !m || !d_x || !d_y || B < 0) return PHY_EINVAL;
   if (B == 0) return PHY_OK;
   if (B > (1 << 30)) return set_err(ctx, PHY_ERANGE, "mlp: batch too large");
+  if (fused_fits(m)) return fused_forward(ctx, m, d_x, B, d_y);
   int rc = ensure_cap(m, B);
   if (rc) return rc;
   return forward(ctx, m, d_x, B, d_y);
@@ -364,6 +748,7 @@ int phy_mlp_backward(phy_ctx* ctx, phy_mlp* m, const float* d_x, const float* d_
                      float* d_grads, double* d_loss) {
   if (!ctx || !m || !d_x || !d_t || B < 1) return PHY_EINVAL;
   if (B > (1 << 30)) return set_err(ctx, PHY_ERANGE, "mlp: batch too large");
+  if (fused_fits(m)) return fused_backward(ctx, m, d_x, d_t, B, d_grads, d_loss);
   int rc = ensure_cap(m, B);
   if (rc) return rc;
   {
@@ -376,13 +761,7 @@ int phy_mlp_backward(phy_ctx* ctx, phy_mlp* m, const float* d_x, const float* d_
     const int64_t rows = std::max<int64_t>(64, (B + 1023) / 1024);
     const int64_t need = std::max({part(H, 1), part(H, H), part(m->n_in, H),
                                    ((B + rows - 1) / rows) * (int64_t)H});
-    if (m->ws_floats < need) {
-      if (m->ws) PHY_HIP(ctx, hipFree(m->ws));
-      m->ws = nullptr;
-      m->ws_floats = 0;
-      PHY_HIP(ctx, hipMalloc((void**)&m->ws, sizeof(float) * (size_t)need));
-      m->ws_floats = need;
-    }
+    if ((rc = ensure_ws(ctx, m, need))) return rc;
   }
   if (d_loss && (rc = phy_zero_u64(ctx, reinterpret_cast<uint64_t*>(d_loss), 1))) return rc;
   rc = backward(ctx, m, d_x, d_t, B, d_loss);
