@@ -2,24 +2,36 @@
 //
 // Many independent trees of uneven taxon and pattern counts, each with its own
 // GTR-20 model and Gamma rates, are evaluated in one persistent launch:
-// workgroups take (tree, pattern tile) items from an atomic queue until it is
+// workgroups take (tree, pattern tile) items from atomic queues until they are
 // empty (every workgroup reaches the exit).  A workgroup of WAVES waves owns
 // 16*WAVES patterns of one tree and walks that tree's post-order program
 // (phy_topo_create's Sethi-Ullman order); the waves stay in lock step, so the
 // transition-matrix operands of the node being computed are staged once into
 // LDS and shared.
 //
-// Per node, child partial x (16 patterns x 20 states, per rate) times P^T:
-//   D[i][p] = sum_j P_r[i][j] x[j][p]     v_mfma_f32_16x16x32_bf16
-// with A = P (16 output states x 32 source states, zero padded) and B = x (32
-// source states x 16 patterns).  The output rows are a permutation rho of the
-// states chosen so that lane l (pattern l%16, quarter q = l/16) receives
-// states 8q..8q+7 -- exactly the k-slice that lane supplies as B operand of
-// the next product:  rho(4q+v) = 8q+v (block 0), rho(16+4q+v) = 8q+4+v
-// (block 1).  Partials therefore never move between lanes; combining the two
-// children, per-pattern power-of-two rescaling and the root sum are FP32 /
-// FP64 VALU work on 32 values per lane.  Spilled partials are stored as the
-// BF16 operand they will be used as (no extra rounding).
+// Per node, child partial x (16 patterns x 20 states, R rates) times P^T with
+// v_mfma_f32_16x16x32_bf16, A = P, B = x (columns = patterns).  The 20 states
+// of a rate split into 16 + 4: R main tiles of 16 output states, and one tile
+// whose 16 output rows are the last 4 states of up to 4 rates (row 4 rho + v =
+// rate rho, state 16 + v).  Lane l (pattern l % 16, quarter q = l / 16) then
+// holds states 4q .. 4q+3 of every rate and states 16 .. 19 of rate q: 4R + 4
+// values with no padding at R = 4.  The k index of a product is free, so its
+// slots are laid out as the lanes hold them -- slots 8q .. 8q+7 of the main
+// product of rate r are the lane's 4 states of rate r and its 4 extra states
+// (A is zero there unless q = r) -- and partials never move between lanes.
+// The extra tile takes R products over the same operands (A holds the rows of
+// rate r only), so a child is 2R products of R operands.
+// (Padding each rate to 32 states gave 8R values a lane, 12 of every 32 of
+// them zero: 196 VGPRs and two waves per SIMD against 156 and three here.
+// With the rest of the node loop below, 256 trees of 16-256 taxa and
+// 1,000-20,000 patterns take 8.0 ms against 17.1 at 8 groups per tile and 8.3
+// against 16.2 at 4.  Bound: VALU issue ~60% and the node's LDS reads and
+// barrier; MFMA busy ~27%.)
+// Combining the two children, per-pattern power-of-two rescaling and the root
+// sum are FP32 / FP64 VALU work on 4R + 4 values per lane.  A wave may own G
+// groups of 16 patterns, which share each P operand it reads from LDS.
+// Spilled partials are stored as the BF16 operand they will be used as (no
+// extra rounding).
 //
 // Precision: MFMA inputs are BF16 (8-bit mantissa), accumulation, partials and
 // exponents FP32 / int32, the root log-sum FP64.  P(t) = U diag(exp(lambda t))
@@ -41,11 +53,19 @@ namespace {
 constexpr int KAA = 20;
 constexpr int OPB = 64;  // uint4 (16 B) per lane-ordered operand block (1 KiB)
 
+// Work queues, one per XCD (workgroups are dealt round-robin to the 8 XCDs, so
+// blockIdx % 8 names a workgroup's XCD).  The tiles of a tree share its P
+// operands (7 KiB a branch at R = 4, ~2 MB for 128 taxa), which one XCD's 4 MB
+// L2 holds and eight would each fetch: with one queue for all, the 256 trees
+// above took 22.7 ms at 4 groups per tile, with these 9.4 (98% L2 hits).
+// A workgroup whose queue is empty takes from the next one, so the placement
+// is only a preference.
+constexpr int kQueues = 8;
+constexpr int kCounterPitch = 32;  // uint32: a 128-byte line per counter
+
 struct AADev {
   const int4* prog;
   const int64_t* prog_off;  // entries
-  const int32_t* fifo;
-  const int64_t* fifo_off;
   const int32_t* n_leaves;
   const uint8_t* tips;
   const int64_t* tips_off;  // bytes
@@ -56,107 +76,152 @@ struct AADev {
   const int64_t* pop_off;   // uint4 units
   const double* pi;         // [T][20]
   const double* probs;      // [T][R]
-  const int2* items;        // (tree, tile)
-  int n_items;
+  const int2* items;        // (tree, tile), queue by queue
+  int q_off[kQueues + 1];   // first item of each queue
   double* part;
   const int64_t* part_off;
-  unsigned* counter;
+  unsigned* counter;        // items taken from each queue
   int depth;                // LDS stack entries per wave
 };
 
-// source state of output row i of block b
-__host__ __device__ __forceinline__ int rho(int b, int i) {
-  const int q = i >> 2, v = i & 3;
-  return 8 * q + 4 * b + v;
-}
+// operand blocks (1 KiB) of one branch: R main products, R of the extra tile
+constexpr int aa_blocks(int R) { return 2 * R; }
 
-// --- P operands: one wave per (tree, branch, rate), four to a workgroup ---
-constexpr int kPopsPerBlock = 4;
+// --- P operands: a block of R waves takes `per` consecutive branches,
+// wave r forming P(rate_r t) in FP64 from U and Ui staged in LDS (a 2 x 4
+// tile of entries per lane), then the waves write the branch's operand blocks.
+// (One wave per (branch, rate) reading U and Ui from memory for every entry:
+// 425 us for 64 trees of 16-256 taxa, here 93.) ---
+// Branches per block: up to 8 share a tree's staged U and Ui, fewer when that
+// would leave CUs without a block.
+constexpr int kPopsPerBlock = 8;
 
-__global__ __launch_bounds__(64 * kPopsPerBlock) void k_aa_pops(
+template <int R>
+__global__ __launch_bounds__(64 * R) void k_aa_pops(
     const double* __restrict__ eig,  // [T][U 400|lam 20|Ui 400]
     const double* __restrict__ rates,  // [T][R]
     const double* __restrict__ blen,   // flat
     const int64_t* __restrict__ blen_off,
     const int32_t* __restrict__ br_tree,  // flat branch -> tree
-    int R, int64_t n_pairs, const int64_t* __restrict__ pop_off, uint4* __restrict__ pops) {
-  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
-  const int64_t pair = (int64_t)blockIdx.x * kPopsPerBlock + wv;
-  const bool valid = pair < n_pairs;
-  const int64_t pc = valid ? pair : n_pairs - 1;  // an idle wave reads in bounds, writes nothing
-  const int64_t gb = pc / R;  // flat branch index
-  const int r = (int)(pc % R);
-  const int t = br_tree[gb];
-  const int64_t b = gb - blen_off[t];
-  const double* U = eig + (size_t)t * (2 * KAA * KAA + KAA);
-  const double* lam = U + KAA * KAA;
-  const double* Ui = lam + KAA;
-  const double rt = rates[(size_t)t * R + r] * blen[gb];
-  __shared__ double ex[kPopsPerBlock][KAA];
-  __shared__ double P[kPopsPerBlock][KAA * KAA];
-  if (l < KAA) ex[wv][l] = exp(lam[l] * rt);
-  __syncthreads();
-  for (int e = l; e < KAA * KAA; e += 64) {
-    const int i = e / KAA, j = e % KAA;
-    double s = 0.0;
-    for (int m = 0; m < KAA; ++m) s += U[i * KAA + m] * ex[wv][m] * Ui[m * KAA + j];
-    if (!(rt >= 1e-10)) s = (i == j) ? 1.0 : 0.0;  // compose rule, lib/mlmodel.c:339-341
-    P[wv][e] = s;
-  }
-  __syncthreads();
-  if (!valid) return;
-  uint4* dst = pops + pop_off[t] + ((b * R + r) * 2) * OPB;
-  for (int blk = 0; blk < 2; ++blk) {
-    // lane l: output row l%16 -> state rho(blk, l%16); k = 8*(l/16) + v
-    const int srow = rho(blk, l & 15);
-    bf16x8 a;
-#pragma unroll
-    for (int v = 0; v < 8; ++v) {
-      const int k = 8 * (l >> 4) + v;
-      const float val = (srow < KAA && k < KAA) ? (float)P[wv][srow * KAA + k] : 0.0f;
-      a[v] = (__bf16)val;
+    int64_t n_branches, int per, const int64_t* __restrict__ pop_off, uint4* __restrict__ pops) {
+  constexpr int NB = aa_blocks(R), KK = KAA * KAA;
+  const int r = threadIdx.x >> 6, l = threadIdx.x & 63;
+  __shared__ double U[KK], Ui[KK], ex[R][KAA], P[R][KK];
+  int staged = -1;
+  const int64_t b0 = (int64_t)blockIdx.x * per;
+  const int64_t b1 = b0 + per < n_branches ? b0 + per : n_branches;
+  for (int64_t gb = b0; gb < b1; ++gb) {  // flat branch index (block-uniform)
+    const int t = br_tree[gb];
+    const int64_t b = gb - blen_off[t];
+    const double* E = eig + (size_t)t * (2 * KK + KAA);
+    const double rt = rates[(size_t)t * R + r] * blen[gb];
+    if (t != staged) {  // the previous branch's reads ended before its last barrier
+      for (int e = threadIdx.x; e < KK; e += 64 * R) {
+        U[e] = E[e];
+        Ui[e] = E[KK + KAA + e];
+      }
+      staged = t;
     }
-    dst[blk * OPB + l] = *reinterpret_cast<uint4*>(&a);
+    if (l < KAA) ex[r][l] = exp(E[KK + l] * rt);
+    __syncthreads();
+    if (l < 50) {  // rows i0, i0 + 1, columns j0 .. j0 + 3
+      const int i0 = 2 * (l / 5), j0 = 4 * (l % 5);
+      double s[2][4] = {};
+      for (int m = 0; m < KAA; ++m) {
+        const double e = ex[r][m], u0 = U[i0 * KAA + m] * e, u1 = U[(i0 + 1) * KAA + m] * e;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const double v = Ui[m * KAA + j0 + j];
+          s[0][j] += u0 * v;
+          s[1][j] += u1 * v;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          double v = s[i][j];
+          if (!(rt >= 1e-10)) v = (i0 + i == j0 + j) ? 1.0 : 0.0;  // compose rule, lib/mlmodel.c:339-341
+          P[r][(i0 + i) * KAA + j0 + j] = v;
+        }
+    }
+    __syncthreads();
+    uint4* dst = pops + pop_off[t] + b * (NB * OPB);
+    const int row = l & 15, q = l >> 4;
+    for (int blk = r; blk < NB; blk += R) {
+      bf16x8 a;
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        // main: state `row` of rate `br`; extra tile: state 16 + row % 4 of
+        // rate row / 4, zero unless that is `br`
+        const int br = blk % R;
+        const int st = blk < R ? row : (row >> 2) == br ? 16 + (row & 3) : -1;
+        double val = 0.0;
+        if (st >= 0) {
+          if (v < 4) val = P[br][st * KAA + 4 * q + v];
+          else if (q == br) val = P[br][st * KAA + 16 + v - 4];
+        }
+        a[v] = (__bf16)(float)val;
+      }
+      dst[blk * OPB + l] = *reinterpret_cast<uint4*>(&a);
+    }
   }
 }
 
-__device__ __forceinline__ bf16x8 to_bf16x8(const float* x) {
-  bf16x8 r;
+// four values as packed BF16
+__device__ __forceinline__ uint2 pack4(const float* x) {
+  typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+  bf16x4 r;
 #pragma unroll
-  for (int v = 0; v < 8; ++v) r[v] = (__bf16)x[v];
-  return r;
+  for (int v = 0; v < 4; ++v) r[v] = (__bf16)x[v];
+  return *reinterpret_cast<const uint2*>(&r);
+}
+__device__ __forceinline__ bf16x8 operand(const uint2 lo, const uint2 hi) {
+  const uint4 u = make_uint4(lo.x, lo.y, hi.x, hi.y);
+  return *reinterpret_cast<const bf16x8*>(&u);
 }
 
+// a lane's slots of a tip: states 4q .. 4q+3, then 16 .. 19
 __device__ __forceinline__ bf16x8 tip_operand(uint32_t code, int q) {
   bf16x8 r;
 #pragma unroll
   for (int v = 0; v < 8; ++v) {
-    const int s = 8 * q + v;
-    const bool on = (code < (uint32_t)KAA) ? (s == (int)code) : (s < KAA);
-    r[v] = (__bf16)(on ? 1.0f : 0.0f);
+    const int s = v < 4 ? 4 * q + v : 12 + v;
+    r[v] = (__bf16)((code >= (uint32_t)KAA || s == (int)code) ? 1.0f : 0.0f);
   }
   return r;
 }
 
-template <int WAVES, int R, int LV>
-__global__ __launch_bounds__(64 * WAVES) void k_aa_prune(AADev a) {
-  constexpr int NT = 64 * WAVES;
-  constexpr int STAGE = 2 * R * 2 * OPB;  // uint4 per node: [c][r][blk][lane]
-  constexpr int NBLK = 2 * R * 2;         // 1 KiB operand blocks per node
-  __shared__ uint4 stage[2][STAGE];       // double buffer: node i and node i+1
-  __shared__ uint4 tipop[(KAA + 1) * 4];  // B operand of a tip: [code 0..20][quarter]
+// 16-byte units of one LDS stack level of a 16-pattern group: R + 1 packed
+// quadruples a lane, and 16 exponents
+constexpr int aa_level(int R) { return (R + 1) * 32 + 4; }
+
+// a partial as BF16 operands, with its exponent
+template <int R>
+struct AAVec {
+  uint2 own[R], ext;
+  int e;
+};
+
+// TW: 16-pattern groups of a tile; G: groups of a wave
+template <int TW, int G, int R, int LV>
+__global__ __launch_bounds__(64 * (TW / G)) void k_aa_prune(AADev a) {
+  static_assert(TW % G == 0, "whole groups per wave");
+  constexpr int NW = TW / G, NT = 64 * NW;
+  constexpr int NB = aa_blocks(R);
+  constexpr int NBLK = 2 * NB;              // 1 KiB operand blocks per node
+  __shared__ uint4 stage[2][NBLK * OPB];    // double buffer: node i and node i+1
+  __shared__ uint4 tipop[(KAA + 1) * 4];    // B operand of a tip: [code 0..20][quarter]
   __shared__ int s_item;
   extern __shared__ uint4 dyn[];
   // the wave index is uniform: readfirstlane keeps the operand DMA loop scalar
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & 63,
             q = l >> 4, pl = l & 15;
-  // per-wave stack: the bottom LV levels in registers (selected by the
-  // uniform stack pointer with value selects), the rest in LDS:
-  // (depth - LV) x (R operands of 64 lanes) + exponents
+  // per-group stack: the bottom LV levels in registers (selected by the
+  // uniform stack pointer with value selects), the rest in LDS
   const int rows = a.depth > LV ? a.depth - LV : 0;
-  uint4* stk = dyn + (size_t)wave * rows * (R * 64 + 16);
-  uint4 rs[LV > 0 ? LV : 1][R];
-  int rse[LV > 0 ? LV : 1];
+  uint4* stk = dyn + (size_t)wave * G * rows * aa_level(R);
+  AAVec<R> rs[LV > 0 ? LV : 1][G];
   // the 21 tip operands (a state 0..19, or missing = all 20 states) for each
   // quarter of the lanes, built once; a tip child is then one LDS read
   for (int e = tid; e < (KAA + 1) * 4; e += NT) {
@@ -164,215 +229,253 @@ __global__ __launch_bounds__(64 * WAVES) void k_aa_prune(AADev a) {
     tipop[e] = *reinterpret_cast<const uint4*>(&b);
   }
 
+  bool own_empty = false;
   for (;;) {
     __syncthreads();
-    if (tid == 0) s_item = (int)atomicAdd(a.counter, 1u);
+    if (tid < 64) {
+      const int own = (int)(blockIdx.x % kQueues);
+      auto take = [&](int xq) {
+        int k = 0;
+        if (l == 0) k = (int)atomicAdd(a.counter + xq * kCounterPitch, 1u);
+        k = a.q_off[xq] + __builtin_amdgcn_readfirstlane(k);
+        return k < a.q_off[xq + 1] ? k : -1;
+      };
+      int item = own_empty ? -1 : take(own);
+      own_empty = item < 0;
+      // one parallel look at every queue before each attempt: counters only
+      // grow, so an attempt that fails leaves one queue less
+      while (item < 0) {
+        const int x = l < kQueues ? l : 0;
+        const unsigned taken = __hip_atomic_load(a.counter + x * kCounterPitch, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+        const bool left = l < kQueues && (int)taken < a.q_off[x + 1] - a.q_off[x];
+        const unsigned m = (unsigned)__ballot(left);
+        if (!m) break;
+        const unsigned after = m & ~((2u << own) - 1u);  // the next queue that has items, cyclically
+        item = take(__builtin_ctz(after ? after : m));
+      }
+      if (l == 0) s_item = item;
+    }
     __syncthreads();
     // uniform in fact; readfirstlane tells the compiler, so everything
-    // derived from the item (tree offsets, fifo ids, operand addresses) is
+    // derived from the item (tree offsets, operand addresses) is
     // scalar
     const int item = __builtin_amdgcn_readfirstlane(s_item);
-    if (item >= a.n_items) break;
+    if (item < 0) break;
     const int2 it = a.items[item];
     const int t = __builtin_amdgcn_readfirstlane(it.x), tile = __builtin_amdgcn_readfirstlane(it.y);
     const int64_t pitch = a.pitch[t];
-    const int64_t p = (int64_t)tile * (16 * WAVES) + wave * 16 + pl;  // < pitch by construction
+    // pattern of group 0; group g is 16 g further, all < pitch by construction
+    const int64_t p = (int64_t)tile * (16 * TW) + wave * (16 * G) + pl;
     const int N = a.n_leaves[t];
     const int4* prog = a.prog + a.prog_off[t];
-    const int32_t* fifo = a.fifo + a.fifo_off[t];
     const uint8_t* tips = a.tips + a.tips_off[t];
     const uint4* pops = a.pops + a.pop_off[t];
     int sp = 0;
-    float acc[R][8];
-    int acc_e = 0;
+    float acc[G][R + 1][4];  // [r]: states 4q+v of rate r; [R]: states 16+v of rate q
+    int acc_e[G];
 #pragma unroll
-    for (int r = 0; r < R; ++r)
+    for (int g = 0; g < G; ++g) {
+      acc_e[g] = 0;
 #pragma unroll
-      for (int v = 0; v < 8; ++v) acc[r][v] = 0.f;
+      for (int r = 0; r <= R; ++r)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[g][r][v] = 0.f;
+    }
 
     // Every global load issued while node i computes (the operand DMA of node
-    // i+1, the tip codes of node i+1, fifo id refills) is consumed at node i+1
+    // i+1, the tip codes of node i+1) is consumed at node i+1
     // or later, after the node's closing vmcnt(0) and barrier.  Nothing loaded
     // from global memory is waited on in the middle of a node, so the DMA
     // latency overlaps a whole node of MFMA and VALU work.
     //
     // operands of a node's two children straight into LDS (global_load_lds,
     // 16 B per lane: one 1 KiB block per wave instruction), no registers
+    // a wave copies consecutive blocks of one child (of both if it is alone),
+    // four to an address
     auto dma_stage = [&](const int4 o, int buf) {
+      constexpr int HW = NW > 1 ? NW / 2 : 1;     // waves per child
+      constexpr int CH = (NB + HW - 1) / HW;      // blocks per wave and child
+      const int first = (wave % HW) * CH;
 #pragma unroll
-      for (int k = 0; k < (NBLK + WAVES - 1) / WAVES; ++k) {
-        const int bk = wave + k * WAVES;  // uniform
-        if (NBLK % WAVES != 0 && bk >= NBLK) break;
-        const int c = bk / (R * 2), rem = bk % (R * 2);
-        const int child = c ? o.z : o.y;
-        const uint4* src = pops + ((size_t)child * R * 2 + rem) * OPB + l;
-        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                         (__attribute__((address_space(3))) void*)(&stage[buf][bk * OPB]),
-                                         16, 0, 0);
+      for (int cc = 0; cc < (NW > 1 ? 1 : 2); ++cc) {
+        const int c = NW > 1 ? wave / HW : cc;
+        const uint32_t child = (uint32_t)(c ? o.z : o.y) * (NB * OPB);
+#pragma unroll
+        for (int k = 0; k < CH; k += 4) {
+          if (NB % CH != 0 || HW * CH > NB)
+            if (first + k >= NB) break;
+          const uint4* src = pops + child + (first + k) * OPB + l;
+          uint4* dst = &stage[buf][(c * NB + first + k) * OPB];
+          static_for<0, (CH < 4 ? CH : 4)>([&](auto j) {
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                             (__attribute__((address_space(3))) void*)dst, 16,
+                                             decltype(j)::value * 1024, 0);
+          });
+        }
       }
     };
-    // leaf ids of the stream, 128 at a time in two lane vectors (entries
-    // fbase .. fbase+127; the tree's fifo is padded by 128 ids)
-    int fbase = 0, fpos = 0;
-    int fcur = fifo[l], fnx = fifo[64 + l];
-    auto fid = [&](int pos) -> int {
-      const int k = pos - fbase;  // uniform, 0 <= k < 128
-      return k < 64 ? __builtin_amdgcn_readlane(fcur, k) : __builtin_amdgcn_readlane(fnx, k - 64);
+    // tip codes of a node's leaf children (row 0 for a child that is no leaf)
+    auto leaf_codes = [&](const int4 o, uint32_t* ca, uint32_t* cb) {
+      const uint8_t* ta = tips + (int64_t)((o.w & 3) == SRC_LEAF ? o.y : 0) * pitch;
+      const uint8_t* tb = tips + (int64_t)(((o.w >> 2) & 3) == SRC_LEAF ? o.z : 0) * pitch;
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        ca[g] = ta[p + 16 * g];
+        cb[g] = tb[p + 16 * g];
+      }
     };
-    auto tip_at = [&](int pos) -> uint32_t { return tips[(size_t)fid(pos) * pitch + p]; };
-    // tip codes of a node's leaf children: the first leaf of the stream goes
-    // to child a when a is a leaf, else to child b
-    auto leaf_codes = [&](const int4 o, int pos, uint32_t& ca, uint32_t& cb) {
-      ca = tip_at(pos);
-      cb = tip_at(pos + ((o.w & 3) == SRC_LEAF ? 1 : 0));
-    };
-    uint32_t code_a, code_b;
+    uint32_t code_a[G], code_b[G];
     {
       const int4 o0 = prog[0];
-      leaf_codes(o0, 0, code_a, code_b);
+      leaf_codes(o0, code_a, code_b);
       dma_stage(o0, 0);
     }
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the DMA has landed
     __syncthreads();
 
+    auto packed = [&](int g) {
+      AAVec<R> u;
+#pragma unroll
+      for (int r = 0; r < R; ++r) u.own[r] = pack4(acc[g][r]);
+      u.ext = pack4(acc[g][R]);
+      u.e = acc_e[g];
+      return u;
+    };
+    auto select = [&](bool hit, AAVec<R>& d, const AAVec<R>& x) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        d.own[r].x = hit ? x.own[r].x : d.own[r].x;
+        d.own[r].y = hit ? x.own[r].y : d.own[r].y;
+      }
+      d.ext.x = hit ? x.ext.x : d.ext.x;
+      d.ext.y = hit ? x.ext.y : d.ext.y;
+      d.e = hit ? x.e : d.e;
+    };
+
     for_each_entry_ahead(prog, N - 1, [&](int i, const int4 op, const int4 on) {
       const int buf = i & 1;
       const bool more = i + 1 < N - 1;
       const int fl = op.w;
-      const int nl = ((fl & 3) == SRC_LEAF ? 1 : 0) + (((fl >> 2) & 3) == SRC_LEAF ? 1 : 0);
-      if (fpos - fbase >= 64) {  // fnx landed at least one node ago
-        fbase += 64;
-        fcur = fnx;
-        fnx = fifo[fbase + 64 + l];
-      }
       if (more) dma_stage(on, buf ^ 1);  // in flight while node i computes
-      const uint32_t ca = code_a, cb = code_b;
-      leaf_codes(on, fpos + nl, code_a, code_b);  // node i+1's tips, used there
-      fpos += nl;
-      const uint4* cur = stage[buf];
+      uint32_t ca[G], cb[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        ca[g] = code_a[g];
+        cb[g] = code_b[g];
+      }
+      leaf_codes(on, code_a, code_b);  // node i+1's tips, used there
+      auto pop = [&](int c, int blk) {
+        const uint4 u = stage[buf][(c * NB + blk) * OPB + l];
+        return *reinterpret_cast<const bf16x8*>(&u);
+      };
       if (fl & DOWN_SPILL) {
-        if (sp < LV) {
-          uint4 u[R];
 #pragma unroll
-          for (int r = 0; r < R; ++r) {
-            bf16x8 b = to_bf16x8(acc[r]);
-            u[r] = *reinterpret_cast<uint4*>(&b);
+        for (int g = 0; g < G; ++g) {
+          const AAVec<R> u = packed(g);
+          if (sp < LV) {
+            static_for<0, LV>([&](auto lv) { select(sp == lv, rs[lv][g], u); });
+          } else {
+            uint2* s = reinterpret_cast<uint2*>(stk + (size_t)((sp - LV) * G + g) * aa_level(R));
+#pragma unroll
+            for (int r = 0; r < R; ++r) s[r * 64 + l] = u.own[r];
+            s[R * 64 + l] = u.ext;
+            if (q == 0) reinterpret_cast<int*>(s + (R + 1) * 64)[pl] = u.e;
           }
-          static_for<0, LV>([&](auto lv) {
-            const bool hit = sp == lv;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-              rs[lv][r].x = hit ? u[r].x : rs[lv][r].x;
-              rs[lv][r].y = hit ? u[r].y : rs[lv][r].y;
-              rs[lv][r].z = hit ? u[r].z : rs[lv][r].z;
-              rs[lv][r].w = hit ? u[r].w : rs[lv][r].w;
-            }
-            rse[lv] = hit ? acc_e : rse[lv];
-          });
-        } else {
-          uint4* s = stk + (size_t)(sp - LV) * (R * 64 + 16);
-#pragma unroll
-          for (int r = 0; r < R; ++r) {
-            bf16x8 b = to_bf16x8(acc[r]);
-            s[r * 64 + l] = *reinterpret_cast<uint4*>(&b);
-          }
-          if (q == 0) reinterpret_cast<int*>(s + R * 64)[pl] = acc_e;
         }
         ++sp;
       }
-      float xa[R][8];
-      int ea = 0, eb = 0;
+      float xa[G][R + 1][4];
+      int ea[G];
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
         const int src = c ? ((fl >> 2) & 3) : (fl & 3);
-        bf16x8 bop[R];
-        int e = 0;
+        AAVec<R> x[G];
         if (src == SRC_LEAF) {
-          const uint4 tu = tipop[min(c ? cb : ca, (uint32_t)KAA) * 4 + q];
-          const bf16x8 tb = *reinterpret_cast<const bf16x8*>(&tu);
 #pragma unroll
-          for (int r = 0; r < R; ++r) bop[r] = tb;
+          for (int g = 0; g < G; ++g) {
+            const uint4 tu = tipop[min(c ? cb[g] : ca[g], (uint32_t)KAA) * 4 + q];
+#pragma unroll
+            for (int r = 0; r < R; ++r) x[g].own[r] = make_uint2(tu.x, tu.y);
+            x[g].ext = make_uint2(tu.z, tu.w);
+            x[g].e = 0;
+          }
         } else if (src == SRC_ACC) {
 #pragma unroll
-          for (int r = 0; r < R; ++r) bop[r] = to_bf16x8(acc[r]);
-          e = acc_e;
+          for (int g = 0; g < G; ++g) x[g] = packed(g);
         } else {
           --sp;
-          if (sp < LV) {
-            uint4 u[R];
 #pragma unroll
-            for (int r = 0; r < R; ++r) u[r] = rs[0][r];
-            e = rse[0];
-            static_for<1, LV>([&](auto lv) {
-              const bool hit = sp == lv;
+          for (int g = 0; g < G; ++g) {
+            if (sp < LV) {
+              x[g] = rs[0][g];
+              static_for<1, LV>([&](auto lv) { select(sp == lv, x[g], rs[lv][g]); });
+            } else {
+              const uint2* s = reinterpret_cast<const uint2*>(stk + (size_t)((sp - LV) * G + g) * aa_level(R));
 #pragma unroll
-              for (int r = 0; r < R; ++r) {
-                u[r].x = hit ? rs[lv][r].x : u[r].x;
-                u[r].y = hit ? rs[lv][r].y : u[r].y;
-                u[r].z = hit ? rs[lv][r].z : u[r].z;
-                u[r].w = hit ? rs[lv][r].w : u[r].w;
-              }
-              e = hit ? rse[lv] : e;
-            });
-#pragma unroll
-            for (int r = 0; r < R; ++r) bop[r] = *reinterpret_cast<const bf16x8*>(&u[r]);
-          } else {
-            const uint4* s = stk + (size_t)(sp - LV) * (R * 64 + 16);
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-              const uint4 u = s[r * 64 + l];
-              bop[r] = *reinterpret_cast<const bf16x8*>(&u);
+              for (int r = 0; r < R; ++r) x[g].own[r] = s[r * 64 + l];
+              x[g].ext = s[R * 64 + l];
+              x[g].e = reinterpret_cast<const int*>(s + (R + 1) * 64)[pl];
             }
-            e = reinterpret_cast<const int*>(s + R * 64)[pl];
           }
         }
+        auto combine = [&](int g, int r, const f32x4 d) {
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            if (c == 0) xa[g][r][v] = d[v];
+            else acc[g][r][v] = xa[g][r][v] * d[v];
+          }
+        };
+        f32x4 d[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) d[g] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-          f32x4 d0 = {0.f, 0.f, 0.f, 0.f}, d1 = {0.f, 0.f, 0.f, 0.f};
-          const uint4 a0 = cur[((c * R + r) * 2 + 0) * OPB + l];
-          const uint4 a1 = cur[((c * R + r) * 2 + 1) * OPB + l];
-          d0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(&a0), bop[r], d0, 0, 0, 0);
-          d1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(&a1), bop[r], d1, 0, 0, 0);
-          if (c == 0) {
+          const bf16x8 Am = pop(c, r), Ax = pop(c, R + r);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              xa[r][v] = d0[v];
-              xa[r][4 + v] = d1[v];
-            }
-          } else {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-              acc[r][v] = xa[r][v] * d0[v];
-              acc[r][4 + v] = xa[r][4 + v] * d1[v];
-            }
+          for (int g = 0; g < G; ++g) {
+            const bf16x8 b = operand(x[g].own[r], x[g].ext);
+            combine(g, r, __builtin_amdgcn_mfma_f32_16x16x32_bf16(Am, b, f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0));
+            d[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ax, b, d[g], 0, 0, 0);
           }
         }
-        if (c == 0) ea = e; else eb = e;
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          combine(g, R, d[g]);
+          if (c == 0) ea[g] = x[g].e;
+          else acc_e[g] = ea[g] + x[g].e;
+        }
       }
-      acc_e = ea + eb;
-      // per-pattern rescale: lanes l, l^16, l^32, l^48 share pattern pl
-      float mx = 0.f;
+      // Rescale, except at a node of two leaves: its values are products of two
+      // entries of P (>= ~1e-15 each: a branch below 1e-10 is the identity), far
+      // inside the range, and its parent tests again.
+      if ((fl & 15) != (SRC_LEAF | SRC_LEAF << 2))
 #pragma unroll
-      for (int r = 0; r < R; ++r)
+      for (int g = 0; g < G; ++g) {
+        // per-pattern rescale: lanes l, l^16, l^32, l^48 share pattern pl
+        float mx = 0.f;
 #pragma unroll
-        for (int v = 0; v < 8; ++v) mx = fmaxf(mx, acc[r][v]);
-      // with lanes l ^ 16 and l ^ 32 (v_permlane16/32_swap: no LDS round trip)
-      {
-        const unsigned u = __float_as_uint(mx);
-        const auto s16 = __builtin_amdgcn_permlane16_swap(u, u, false, false);
-        mx = fmaxf(__uint_as_float(s16[0]), __uint_as_float(s16[1]));
-        const unsigned u2 = __float_as_uint(mx);
-        const auto s32 = __builtin_amdgcn_permlane32_swap(u2, u2, false, false);
-        mx = fmaxf(__uint_as_float(s32[0]), __uint_as_float(s32[1]));
-      }
-      if (mx < 0x1p-24f && mx > 0.f) {
-        int ex;
-        (void)frexpf(mx, &ex);
+        for (int r = 0; r <= R; ++r)
 #pragma unroll
-        for (int r = 0; r < R; ++r)
+          for (int v = 0; v < 4; ++v) mx = fmaxf(mx, acc[g][r][v]);
+        // with lanes l ^ 16 and l ^ 32 (v_permlane16/32_swap: no LDS round trip);
+        // the values are not negative, so their bits compare as integers
+        {
+          unsigned u = __float_as_uint(mx);
+          const auto s16 = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+          u = s16[0] > s16[1] ? s16[0] : s16[1];
+          const auto s32 = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+          mx = __uint_as_float(s32[0] > s32[1] ? s32[0] : s32[1]);
+        }
+        if (mx < 0x1p-24f && mx > 0.f) {
+          int ex;
+          (void)frexpf(mx, &ex);
 #pragma unroll
-          for (int v = 0; v < 8; ++v) acc[r][v] = ldexpf(acc[r][v], -ex);
-        acc_e += ex;
+          for (int r = 0; r <= R; ++r)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) acc[g][r][v] = ldexpf(acc[g][r][v], -ex);
+          acc_e[g] += ex;
+        }
       }
       __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): node i+1 operands and tips landed
       __syncthreads();
@@ -380,24 +483,30 @@ __global__ __launch_bounds__(64 * WAVES) void k_aa_prune(AADev a) {
     // root: L_p = sum_r prob_r sum_i pi_i L[r][i]
     const double* pi = a.pi + (size_t)t * KAA;
     const double* pr = a.probs + (size_t)t * R;
-    double s = 0.0;
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      double sr = 0.0;
+    for (int g = 0; g < G; ++g) {
+      double s = 0.0;
 #pragma unroll
-      for (int v = 0; v < 8; ++v) {
-        const int st = 8 * q + v;
-        if (st < KAA) sr += pi[st] * (double)acc[r][v];
+      for (int r = 0; r < R; ++r) {
+        double sr = 0.0;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) sr += pi[4 * q + v] * (double)acc[g][r][v];
+        s += pr[r] * sr;
       }
-      s += pr[r] * sr;
-    }
-    s += __shfl_xor(s, 16, 64);
-    s += __shfl_xor(s, 32, 64);
-    const uint32_t w = a.wts[a.w_off[t] + p];
-    double contrib = (q == 0 && w) ? (double)w * (log(s) + (double)acc_e * 0.6931471805599453) : 0.0;
+      if (q < R) {
+        double sr = 0.0;
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) contrib += __shfl_xor(contrib, off, 64);
-    if (l == 0) a.part[a.part_off[t] + (int64_t)tile * WAVES + wave] = contrib;
+        for (int v = 0; v < 4; ++v) sr += pi[16 + v] * (double)acc[g][R][v];
+        s += pr[q] * sr;
+      }
+      s += __shfl_xor(s, 16, 64);
+      s += __shfl_xor(s, 32, 64);
+      const uint32_t w = a.wts[a.w_off[t] + p + 16 * g];
+      double contrib = (q == 0 && w) ? (double)w * (log(s) + (double)acc_e[g] * 0.6931471805599453) : 0.0;
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) contrib += __shfl_xor(contrib, off, 64);
+      if (l == 0) a.part[a.part_off[t] + (int64_t)tile * TW + wave * G + g] = contrib;
+    }
   }
 }
 
@@ -428,7 +537,7 @@ __global__ void k_aa_reduce(const double* __restrict__ part, const int64_t* __re
   }
 }
 
-__global__ void k_zero_u32(unsigned* p) { *p = 0u; }
+__global__ void k_zero_u32(unsigned* p) { p[threadIdx.x * kCounterPitch] = 0u; }
 
 }  // namespace
 
@@ -439,13 +548,14 @@ struct phy_aa_batch {
   std::vector<int32_t> n_leaves;
   std::vector<int64_t> n_pat, pitch;
   int64_t n_items = 0;
+  int32_t q_off[kQueues + 1] = {};
   int64_t n_branches = 0, pattern_nodes = 0;
   std::vector<void*> bufs;  // owned device allocations
   // device arrays
   int4* prog = nullptr;
-  int64_t *prog_off = nullptr, *fifo_off = nullptr, *tips_off = nullptr, *pitch_d = nullptr,
+  int64_t *prog_off = nullptr, *tips_off = nullptr, *pitch_d = nullptr,
           *w_off = nullptr, *pop_off = nullptr, *part_off = nullptr, *blen_off = nullptr;
-  int32_t *fifo = nullptr, *nl = nullptr, *br_tree = nullptr;
+  int32_t *nl = nullptr, *br_tree = nullptr;
   uint8_t* tips = nullptr;
   uint32_t* wts = nullptr;
   uint4* pops = nullptr;
@@ -469,26 +579,69 @@ int upload(phy_aa_batch* b, T** dst, const std::vector<T>& src) {
   return PHY_OK;
 }
 
-size_t lds_bytes(int waves, int R, int depth, int lv) {
-  return (size_t)waves * (depth > lv ? depth - lv : 0) * (R * 64 + 16) * sizeof(uint4);
+// Order the items (given tree by tree) into the queues: trees by decreasing
+// taxa, so that every queue runs its longest items first, each to the queue
+// with the least work so far (a tile costs its tree's taxa).  A tree of more
+// than 1/32 of the whole work is dealt in runs of tiles that small, so that
+// few or uneven trees still spread over the chip.
+void deal_items(const std::vector<int32_t>& n_leaves, std::vector<int2>& items, int32_t* q_off) {
+  const size_t T = n_leaves.size();
+  std::vector<int64_t> first(T + 1, 0);
+  int64_t total = 0;
+  for (const int2& it : items) {
+    ++first[it.x + 1];
+    total += n_leaves[it.x];
+  }
+  for (size_t t = 0; t < T; ++t) first[t + 1] += first[t];
+  std::vector<int32_t> order(T);
+  std::iota(order.begin(), order.end(), 0);
+  std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) { return n_leaves[x] > n_leaves[y]; });
+  std::vector<int2> q[kQueues];
+  int64_t load[kQueues] = {};
+  for (const int32_t t : order) {
+    const int64_t run = std::max<int64_t>(1, total / 32 / n_leaves[t]);
+    for (int64_t k = first[t]; k < first[t + 1]; k += run) {
+      const int x = (int)(std::min_element(load, load + kQueues) - load);
+      const int64_t end = std::min(k + run, first[t + 1]);
+      q[x].insert(q[x].end(), items.begin() + k, items.begin() + end);
+      load[x] += (end - k) * n_leaves[t];
+    }
+  }
+  items.clear();
+  for (int x = 0; x < kQueues; ++x) {
+    q_off[x] = (int32_t)items.size();
+    items.insert(items.end(), q[x].begin(), q[x].end());
+  }
+  q_off[kQueues] = (int32_t)items.size();
 }
 
-// stack levels kept in registers: 3 for stacks of 3 or more levels (frees
-// LDS for a second workgroup per CU), else none (fewer VGPRs).
+size_t lds_bytes(int waves, int R, int depth, int lv) {
+  return (size_t)waves * (depth > lv ? depth - lv : 0) * aa_level(R) * sizeof(uint4);
+}
+
+// Groups of 16 patterns per wave: two where a tile has 8 (the waves of a
+// workgroup then share its operand copies less often but read each operand
+// from LDS once for 32 patterns: 8.0 against 12.1 ms for the 256 trees above),
+// else one (at 4 groups per tile two waves would copy the 16 KiB of a node:
+// 15.1 against 8.3 ms).
+constexpr int aa_groups(int waves) { return waves == 8 ? 2 : 1; }
+
+// Stack levels kept in registers: none for stacks of 1 or 2 levels (fewer
+// VGPRs), else 3, or 4 with one group per wave for stacks of 5 or more (at 5
+// levels three workgroups of 4 waves then fit a CU's LDS instead of two, and
+// the registers still allow three waves per SIMD: 8.3 against 10.9 ms).
 // PHY_AA_REG=0|3 overrides.
-int aa_register_levels(int depth) {
+int aa_register_levels(int depth, int waves) {
   const char* s = getenv("PHY_AA_REG");
   if (s && (s[0] == '0' || s[0] == '3') && s[1] == 0) return s[0] - '0';
-  return depth >= 3 ? 3 : 0;
+  return depth >= 5 && aa_groups(waves) == 1 ? 4 : depth >= 3 ? 3 : 0;
 }
 
-template <int WAVES, int R, int LV>
+template <int TW, int G, int R, int LV>
 int launch(phy_ctx* ctx, phy_aa_batch* b) {
   AADev a;
   a.prog = b->prog;
   a.prog_off = b->prog_off;
-  a.fifo = b->fifo;
-  a.fifo_off = b->fifo_off;
   a.n_leaves = b->nl;
   a.tips = b->tips;
   a.tips_off = b->tips_off;
@@ -500,34 +653,44 @@ int launch(phy_ctx* ctx, phy_aa_batch* b) {
   a.pi = b->pi;
   a.probs = b->probs;
   a.items = b->items;
-  a.n_items = (int)b->n_items;
+  for (int k = 0; k <= kQueues; ++k) a.q_off[k] = b->q_off[k];
   a.part = b->part;
   a.part_off = b->part_off;
   a.counter = b->counter;
   a.depth = std::max(1, b->depth);
-  const size_t lds = lds_bytes(WAVES, R, a.depth, LV);
+  const size_t lds = lds_bytes(TW, R, a.depth, LV);
+  constexpr int NT = 64 * (TW / G);
   int dev = 0, n_cu = 256;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev);
   int per_cu = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_aa_prune<WAVES, R, LV>, 64 * WAVES, lds) != hipSuccess || per_cu < 1)
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (k_aa_prune<TW, G, R, LV>), NT, lds) != hipSuccess || per_cu < 1)
     per_cu = 1;
   const int64_t grid = std::min<int64_t>((int64_t)n_cu * per_cu, b->n_items);
   KernelSpan span(ctx, "aa_prune");
-  hipLaunchKernelGGL((k_aa_prune<WAVES, R, LV>), dim3((unsigned)std::max<int64_t>(grid, 1)), dim3(64 * WAVES), lds,
+  hipLaunchKernelGGL((k_aa_prune<TW, G, R, LV>), dim3((unsigned)std::max<int64_t>(grid, 1)), dim3(NT), lds,
                      ctx->stream, a);
   PHY_LAUNCHED(ctx);
   return PHY_OK;
 }
 
+template <int TW, int R>
+int launch_l(phy_ctx* ctx, phy_aa_batch* b) {
+  constexpr int G = aa_groups(TW);
+  switch (aa_register_levels(std::max(1, b->depth), TW)) {
+    case 0: return launch<TW, G, R, 0>(ctx, b);
+    case 3: return launch<TW, G, R, 3>(ctx, b);
+    default: return launch<TW, G, R, G == 1 ? 4 : 3>(ctx, b);
+  }
+}
+
 template <int R>
 int launch_w(phy_ctx* ctx, phy_aa_batch* b) {
-  const bool reg = aa_register_levels(std::max(1, b->depth)) == 3;
   switch (b->waves) {
-    case 1: return reg ? launch<1, R, 3>(ctx, b) : launch<1, R, 0>(ctx, b);
-    case 2: return reg ? launch<2, R, 3>(ctx, b) : launch<2, R, 0>(ctx, b);
-    case 4: return reg ? launch<4, R, 3>(ctx, b) : launch<4, R, 0>(ctx, b);
-    case 8: return reg ? launch<8, R, 3>(ctx, b) : launch<8, R, 0>(ctx, b);
+    case 1: return launch_l<1, R>(ctx, b);
+    case 2: return launch_l<2, R>(ctx, b);
+    case 4: return launch_l<4, R>(ctx, b);
+    case 8: return launch_l<8, R>(ctx, b);
     default: return set_err(ctx, PHY_ERANGE, "aa_batch: waves per workgroup must be 1, 2, 4 or 8");
   }
 }
@@ -556,8 +719,8 @@ int phy_aa_batch_create(phy_ctx* ctx, int32_t T, const int32_t* n_leaves, const 
   b->waves = waves;
   const int tile = 16 * waves;
   std::vector<int4> prog;
-  std::vector<int64_t> prog_off, fifo_off, tips_off, pitch, w_off, pop_off, part_off, blen_off;
-  std::vector<int32_t> fifo, nl, br_tree;
+  std::vector<int64_t> prog_off, tips_off, pitch, w_off, pop_off, part_off, blen_off;
+  std::vector<int32_t> nl, br_tree;
   std::vector<uint8_t> tipv;
   std::vector<uint32_t> wv;
   std::vector<double> eig, blv;
@@ -580,9 +743,6 @@ int phy_aa_batch_create(phy_ctx* ctx, int32_t T, const int32_t* n_leaves, const 
     for (size_t k = 0; k < topo->down_prog.size(); k += 4)
       prog.push_back(make_int4(topo->down_prog[k], topo->down_prog[k + 1], topo->down_prog[k + 2],
                                topo->down_prog[k + 3]));
-    fifo_off.push_back((int64_t)fifo.size());
-    fifo.insert(fifo.end(), topo->down_fifo.begin(), topo->down_fifo.end());
-    fifo.insert(fifo.end(), 128, 0);  // the kernel holds ids fbase .. fbase+127, fbase <= N
     phy_topo_destroy(topo);
     nl.push_back(N);
     const int64_t pp = (P + tile - 1) / tile * tile;
@@ -614,7 +774,7 @@ int phy_aa_batch_create(phy_ctx* ctx, int32_t T, const int32_t* n_leaves, const 
     for (int32_t v = 0; v < M; ++v) br_tree.push_back(t);
     b->n_branches += M;
     pop_off.push_back(pop_pos);
-    pop_pos += (int64_t)M * R * 2 * OPB;
+    pop_pos += (int64_t)M * aa_blocks(R) * OPB;
     part_off.push_back(part_pos);
     const int64_t tiles = pp / tile;
     part_pos += tiles * waves;
@@ -626,24 +786,19 @@ int phy_aa_batch_create(phy_ctx* ctx, int32_t T, const int32_t* n_leaves, const 
     b->pattern_nodes += P * (N - 1);
   }
   part_off.push_back(part_pos);
-  // largest trees first (longest items first), a tree's tiles kept together
-  std::stable_sort(items.begin(), items.end(), [&](const int2& x, const int2& y) {
-    const int nx = nl[x.x], ny = nl[y.x];
-    if (nx != ny) return nx > ny;
-    return x.x < y.x;
-  });
   b->n_items = (int64_t)items.size();
   if (b->n_items > 0x7fffffff) {
     delete b;
     return set_err(ctx, PHY_ERANGE, "aa_batch: too many work items");
   }
-  // static operand double buffer (2 x 2R x 2 KiB) plus the dynamic stack,
-  // within the device's LDS per workgroup
+  deal_items(nl, items, b->q_off);
+  // static operand double buffer (2 nodes x 2 children) plus the dynamic
+  // stack, within the device's LDS per workgroup
   int lds_max = 64 * 1024, dev = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-  const int lv = aa_register_levels(std::max(1, b->depth));
-  if (lds_bytes(waves, R, std::max(1, b->depth), lv) + (size_t)2 * 2 * R * 2 * OPB * sizeof(uint4) > (size_t)lds_max) {
+  const int lv = aa_register_levels(std::max(1, b->depth), waves);
+  if (lds_bytes(waves, R, std::max(1, b->depth), lv) + (size_t)2 * 2 * aa_blocks(R) * OPB * sizeof(uint4) > (size_t)lds_max) {
     delete b;
     return set_err(ctx, PHY_ERANGE, "aa_batch: LDS stack too deep for this many waves per workgroup");
   }
@@ -652,8 +807,6 @@ int phy_aa_batch_create(phy_ctx* ctx, int32_t T, const int32_t* n_leaves, const 
   int rc = PHY_OK;
   if (!rc) rc = upload(b, &b->prog, prog);
   if (!rc) rc = upload(b, &b->prog_off, prog_off);
-  if (!rc) rc = upload(b, &b->fifo, fifo);
-  if (!rc) rc = upload(b, &b->fifo_off, fifo_off);
   if (!rc) rc = upload(b, &b->nl, nl);
   if (!rc) rc = upload(b, &b->tips, tipv);
   if (!rc) rc = upload(b, &b->tips_off, tips_off);
@@ -672,7 +825,7 @@ int phy_aa_batch_create(phy_ctx* ctx, int32_t T, const int32_t* n_leaves, const 
   if (!rc) rc = upload(b, &b->items, items);
   if (!rc) rc = upload(b, &b->pops, std::vector<uint4>((size_t)pop_pos));
   if (!rc) rc = upload(b, &b->part, std::vector<double>((size_t)part_pos));
-  if (!rc) rc = upload(b, &b->counter, std::vector<unsigned>(4, 0u));
+  if (!rc) rc = upload(b, &b->counter, std::vector<unsigned>(kQueues * kCounterPitch, 0u));
   if (rc) {
     phy_aa_batch_destroy(b);
     return rc;
@@ -700,13 +853,22 @@ int phy_aa_batch_run(phy_ctx* ctx, phy_aa_batch* b, double* d_lnl) {
   if (!ctx || !b || !d_lnl) return PHY_EINVAL;
   if (b->ctx != ctx) return set_err(ctx, PHY_EINVAL, "aa_batch: built on another context");
   // 1. P operands for every (tree, branch, rate)
-  const int64_t n_pairs = b->n_branches * b->R;
-  const int64_t nwg = (n_pairs + kPopsPerBlock - 1) / kPopsPerBlock;
-  hipLaunchKernelGGL(k_aa_pops, dim3((unsigned)nwg), dim3(64 * kPopsPerBlock), 0, ctx->stream, b->eig,
-                     b->rates, b->blen, b->blen_off, b->br_tree, b->R, n_pairs, b->pop_off, b->pops);
+  int n_cu = 256;
+  (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, ctx->device);
+  const int per = (int)std::min<int64_t>(kPopsPerBlock, 1 + b->n_branches / (4 * n_cu));
+  const unsigned nwg = (unsigned)((b->n_branches + per - 1) / per);
+  auto pops = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(nwg), dim3(64 * b->R), 0, ctx->stream, b->eig, b->rates, b->blen, b->blen_off,
+                       b->br_tree, b->n_branches, per, b->pop_off, b->pops);
+  };
+  switch (b->R) {
+    case 1: pops(k_aa_pops<1>); break;
+    case 2: pops(k_aa_pops<2>); break;
+    default: pops(k_aa_pops<4>); break;
+  }
   PHY_LAUNCHED(ctx);
   // 2. the persistent pruning launch
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(1), 0, ctx->stream, b->counter);
+  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(kQueues), 0, ctx->stream, b->counter);
   PHY_LAUNCHED(ctx);
   int rc;
   switch (b->R) {

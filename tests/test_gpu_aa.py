@@ -140,3 +140,52 @@ def test_one_and_two_rate_classes(ctx, R, waves):
     for k, t in enumerate(trees):
         ov = _oracle(t)
         assert abs(got[k] - ov) <= 2e-3 * abs(ov), (k, got[k], ov)
+
+
+def _balanced(n):
+    """Children of a balanced tree of n = 2^k leaves (the deepest stack)."""
+    ch, level, nxt = [], list(range(n)), n
+    while len(level) > 1:
+        level2 = []
+        for a, b in zip(level[::2], level[1::2]):
+            ch += [a, b]
+            level2.append(nxt)
+            nxt += 1
+        level = level2
+    return np.array(ch, np.int32), nxt - 1
+
+
+@pytest.mark.parametrize("R", [1, 2, 4])
+def test_every_tile_gives_the_same_trees(ctx, R):
+    # one or two groups of 16 patterns per wave, 0 / 3 / 4 stack levels in
+    # registers (by the deepest tree of a batch) and the rest in LDS: the same
+    # operations per pattern, so the lnL differ by the order of an FP64 sum of
+    # <= 1,000 terms (1,000 x 2^-53 ~ 1e-13)
+    from dataclasses import replace
+
+    from phylocaml_amd import aa
+
+    rng = np.random.default_rng(61 + R)
+    rates = np.array({1: [1.0], 2: [0.3, 1.7], 4: [0.05, 0.4, 0.9, 2.65]}[R])
+    for name, shapes in (("shallow", [(2, 1), (3, 17), (5, 300)]),
+                         ("deep", [(128, 129), (2, 16), (64, 1), (33, 257), (16, 1000)])):
+        trees = []
+        for k, (n, p) in enumerate(shapes):
+            t = aa.synth_tree(7000 + 10 * R + k, n, p, n_sim=100)
+            if name == "deep" and n & (n - 1) == 0:
+                ch, root = _balanced(n)
+                t = replace(t, children=ch, root=root)
+            t.tips[rng.random(t.tips.shape) < 0.05] = 255
+            trees.append(replace(t, rates=rates, probs=np.full(R, 1.0 / R)))
+        got = {}
+        for waves in (1, 2, 4, 8):
+            print(f"aa {name} R={R} waves={waves}", flush=True)
+            b = aa.AABatch(ctx, trees, waves=waves)
+            b.run()
+            ctx.sync()
+            got[waves] = b.lnl.cpu().numpy()
+        for waves in (1, 2, 8):
+            assert np.allclose(got[waves], got[4], rtol=1e-12, atol=0)
+        for k, t in enumerate(trees):
+            ov = _oracle(t)
+            assert abs(got[4][k] - ov) <= 2e-3 * abs(ov), (k, got[4][k], ov)
