@@ -86,6 +86,14 @@ struct SplitProg {
   int32_t* d_meta = nullptr;  // prog_off | n_ops | fifo_off, parts + 1 each
 };
 
+// Split of a tree for the Fitch passes: the cut nodes of its parts (empty: no
+// split) and the programs of both passes.
+struct FitchSplit {
+  std::vector<int32_t> parts;
+  SplitProg down, up;
+  int32_t* d_part_parent = nullptr;
+};
+
 struct phy_topo {
   phy_ctx* ctx = nullptr;
   int32_t n_leaves = 0;
@@ -101,15 +109,16 @@ struct phy_topo {
   std::vector<int32_t> up_prog;
   std::vector<int32_t> up_fifo;    // node ids in load order (2N-1)
   int32_t up_depth = 0;
-  // device copies
+  // device copies, all in one allocation
+  void* d_programs = nullptr;
   int4* d_down_prog = nullptr;
   int32_t* d_down_fifo = nullptr;
   int4* d_up_prog = nullptr;
   int32_t* d_up_fifo = nullptr;
-  // split programs (empty parts: the tree is run whole)
-  std::vector<int32_t> parts;      // cut node of each part
-  SplitProg split_down, split_up;
-  int32_t* d_part_parent = nullptr;
+  // splits of the Fitch passes: `split` for passes over many sites, `fine`
+  // (about sqrt(N) parts, device only) for passes whose sites leave the chip
+  // idle, which are bound by the longest chain of nodes
+  FitchSplit split, fine;
   // split form of the fused pruning pass (its own cuts, fewer than the Fitch
   // passes take: every part adds a stored root partial per pattern):
   // psplit holds the part programs; the top program reads the cut nodes as

@@ -16,6 +16,7 @@
 //    child first and stacking the larger; each node's preliminary set is
 //    loaded exactly once, in a fixed order.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <functional>
 
@@ -358,6 +359,55 @@ std::vector<int32_t> choose_cuts(int32_t N, const std::vector<int32_t>& ch,
   return cuts;
 }
 
+// Programs of the Fitch passes split under at most `want` cut nodes of at
+// least `min_leaves` leaves (no parts when fewer than two are found).
+int compile_fitch_split(const phy_topo* t, int want, int32_t min_leaves, FitchSplit* out) {
+  const int32_t N = t->n_leaves, M = 2 * N - 1;
+  const std::vector<int32_t>& ch = t->children;
+  const Stop is_leaf = [N](int32_t v) { return v < N; };
+  *out = FitchSplit();
+  if (want < 2) return 0;
+  const std::vector<int32_t> cuts = choose_cuts(N, ch, t->subtree, t->root, want, min_leaves);
+  if (cuts.size() < 2) return 0;
+  std::vector<char> is_cut(M, 0);
+  for (int32_t c : cuts) is_cut[c] = 1;
+  const Stop stop_top = [N, &is_cut](int32_t v) { return v < N || is_cut[v]; };
+  SplitProg& sd = out->down;
+  SplitProg& su = out->up;
+  std::vector<int32_t> pg, ff;
+  int32_t d = 0, n_ops = 0;
+  auto add = [&](SplitProg& sp) {
+    sp.prog_off.push_back((int32_t)sp.prog.size() / 4);
+    sp.n_ops.push_back((int32_t)pg.size() / 4);
+    sp.fifo_off.push_back((int32_t)sp.fifo.size());
+    sp.prog.insert(sp.prog.end(), pg.begin(), pg.end());
+    std::vector<int32_t> pad(phy_fifo_padded(ff.size()), ff.empty() ? 0 : ff[0]);
+    std::copy(ff.begin(), ff.end(), pad.begin());
+    sp.fifo.insert(sp.fifo.end(), pad.begin(), pad.end());
+    sp.depth = std::max(sp.depth, d);
+    n_ops += (int32_t)pg.size() / 4;
+  };
+  // down: parts first, then the top (cut nodes read as leaves)
+  for (int32_t c : cuts) {
+    if (!compile_down(N, ch, c, is_leaf, &pg, &ff, &d)) return 4;
+    add(sd);
+  }
+  if (!compile_down(N, ch, t->root, stop_top, &pg, &ff, &d)) return 4;
+  add(sd);
+  if (n_ops != N - 1) return 5;
+  // up: the top first, then the parts (entered from the parent's final)
+  n_ops = 0;
+  compile_up(N, ch, t->subtree, t->root, stop_top, SRC_LEAF, &pg, &ff, &d);
+  add(su);
+  for (int32_t c : cuts) {
+    compile_up(N, ch, t->subtree, c, is_leaf, SRC_EXT, &pg, &ff, &d);
+    add(su);
+  }
+  if (n_ops != N - 1) return 6;
+  out->parts = cuts;
+  return 0;
+}
+
 }  // namespace
 
 void phy_compile_up_program(int32_t N, const std::vector<int32_t>& ch, const std::vector<int32_t>& size,
@@ -390,55 +440,13 @@ int phy_compile_topo(phy_topo* t) {
   if ((int32_t)t->up_prog.size() != 4 * (N - 1) || (int32_t)t->up_fifo.size() != M) return 3;
 
   // ---- split programs: parts under cut nodes run side by side ----
-  t->parts.clear();
   // default: up to 16 parts of >= 64 leaves on average; PHY_FITCH_PARTS
   // asks for a count (parts of >= 16 leaves)
   const char* env_parts = getenv("PHY_FITCH_PARTS");
   const int want = env_parts ? (int)std::min<int32_t>(std::max(1, std::min(kMaxParts, atoi(env_parts))), N / 16)
                              : (int)std::min<int32_t>(16, N / 64);
-  if (want >= 2) {
-    const std::vector<int32_t> cuts = choose_cuts(N, ch, t->subtree, t->root, want, 16);
-    if (cuts.size() >= 2) {
-      std::vector<char> is_cut(M, 0);
-      for (int32_t c : cuts) is_cut[c] = 1;
-      const Stop stop_top = [N, &is_cut](int32_t v) { return v < N || is_cut[v]; };
-      SplitProg& sd = t->split_down;
-      SplitProg& su = t->split_up;
-      sd = SplitProg();
-      su = SplitProg();
-      std::vector<int32_t> pg, ff;
-      int32_t d = 0, n_ops = 0;
-      auto add = [&](SplitProg& sp) {
-        sp.prog_off.push_back((int32_t)sp.prog.size() / 4);
-        sp.n_ops.push_back((int32_t)pg.size() / 4);
-        sp.fifo_off.push_back((int32_t)sp.fifo.size());
-        sp.prog.insert(sp.prog.end(), pg.begin(), pg.end());
-        std::vector<int32_t> pad(phy_fifo_padded(ff.size()), ff.empty() ? 0 : ff[0]);
-        std::copy(ff.begin(), ff.end(), pad.begin());
-        sp.fifo.insert(sp.fifo.end(), pad.begin(), pad.end());
-        sp.depth = std::max(sp.depth, d);
-        n_ops += (int32_t)pg.size() / 4;
-      };
-      // down: parts first, then the top (cut nodes read as leaves)
-      for (int32_t c : cuts) {
-        if (!compile_down(N, ch, c, is_leaf, &pg, &ff, &d)) return 4;
-        add(sd);
-      }
-      if (!compile_down(N, ch, t->root, stop_top, &pg, &ff, &d)) return 4;
-      add(sd);
-      if (n_ops != N - 1) return 5;
-      // up: the top first, then the parts (entered from the parent's final)
-      n_ops = 0;
-      compile_up(N, ch, t->subtree, t->root, stop_top, SRC_LEAF, &pg, &ff, &d);
-      add(su);
-      for (int32_t c : cuts) {
-        compile_up(N, ch, t->subtree, c, is_leaf, SRC_EXT, &pg, &ff, &d);
-        add(su);
-      }
-      if (n_ops != N - 1) return 6;
-      for (int32_t c : cuts) t->parts.push_back(c);
-    }
-  }
+  const int rc = compile_fitch_split(t, want, 16, &t->split);
+  if (rc) return rc;
 
   // ---- split form of the fused pruning pass ----
   // default: up to 16 parts of >= 128 leaves on average; PHY_PRUNE_PARTS
@@ -505,21 +513,51 @@ int phy_compile_topo(phy_topo* t) {
   return 0;
 }
 
-// device copies of a split program: programs, leaf streams and the offsets
-// [prog_off | n_ops | fifo_off], one per program each
-static hipError_t upload_split(SplitProg* sp) {
+static std::vector<int32_t> split_meta(const SplitProg& sp) {
   std::vector<int32_t> meta;
-  meta.insert(meta.end(), sp->prog_off.begin(), sp->prog_off.end());
-  meta.insert(meta.end(), sp->n_ops.begin(), sp->n_ops.end());
-  meta.insert(meta.end(), sp->fifo_off.begin(), sp->fifo_off.end());
-  hipError_t e = hipMalloc((void**)&sp->d_prog, sp->prog.size() * 4);
-  if (e == hipSuccess) e = hipMalloc((void**)&sp->d_fifo, sp->fifo.size() * 4);
-  if (e == hipSuccess) e = hipMalloc((void**)&sp->d_meta, meta.size() * 4);
-  if (e == hipSuccess) e = hipMemcpy(sp->d_prog, sp->prog.data(), sp->prog.size() * 4, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(sp->d_fifo, sp->fifo.data(), sp->fifo.size() * 4, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(sp->d_meta, meta.data(), meta.size() * 4, hipMemcpyHostToDevice);
-  return e;
+  meta.insert(meta.end(), sp.prog_off.begin(), sp.prog_off.end());
+  meta.insert(meta.end(), sp.n_ops.begin(), sp.n_ops.end());
+  meta.insert(meta.end(), sp.fifo_off.begin(), sp.fifo_off.end());
+  return meta;
 }
+
+// Device copies of every program of a topology, packed into one allocation and
+// one copy (a search makes a topology per accepted move): `put` queues an array
+// and the pointer that is to hold its device address.
+struct TopoUpload {
+  std::vector<int32_t> all;
+  std::vector<std::pair<size_t, void**>> at;
+
+  template <class T>
+  void put(const std::vector<int32_t>& v, T** dst) {
+    at.push_back({all.size(), (void**)dst});
+    all.insert(all.end(), v.begin(), v.end());
+    all.resize((all.size() + 63) / 64 * 64, 0);  // 256-byte aligned pieces
+  }
+  // programs, leaf streams and the offsets [prog_off | n_ops | fifo_off]
+  void put(SplitProg* sp) {
+    std::vector<int32_t> meta;
+    for (const auto* v : {&sp->prog_off, &sp->n_ops, &sp->fifo_off}) meta.insert(meta.end(), v->begin(), v->end());
+    put(sp->prog, &sp->d_prog);
+    put(sp->fifo, &sp->d_fifo);
+    put(meta, &sp->d_meta);
+  }
+  void put(const phy_topo* t, FitchSplit* f) {
+    if (f->parts.empty()) return;
+    put(&f->down);
+    put(&f->up);
+    std::vector<int32_t> pp;
+    for (int32_t c : f->parts) pp.push_back(t->parent[c]);
+    put(pp, &f->d_part_parent);
+  }
+  hipError_t run(void** d_all) {
+    hipError_t e = hipMalloc(d_all, all.size() * 4);
+    if (e != hipSuccess) return e;
+    e = hipMemcpy(*d_all, all.data(), all.size() * 4, hipMemcpyHostToDevice);
+    for (const auto& x : at) *x.second = static_cast<int32_t*>(*d_all) + x.first;
+    return e;
+  }
+};
 
 extern "C" {
 
@@ -567,38 +605,32 @@ int phy_topo_create(phy_ctx* ctx, int32_t N, const int32_t* children, int32_t ro
     *out = t;
     return PHY_OK;
   }
-  hipError_t e = hipSuccess;
+  // about sqrt(N) parts of sqrt(N) leaves under a top of as many nodes: the
+  // shortest chain of two launches (PHY_FITCH_PARTS keeps to its one split)
+  if (N >= 24 && !getenv("PHY_FITCH_PARTS")) {
+    const int want = std::min(kMaxParts, (int)std::lround(std::sqrt((double)N)));
+    if (compile_fitch_split(t, want, std::max(3, N / want / 2), &t->fine)) {
+      delete t;
+      return set_err(ctx, PHY_EINVAL, "topology: program compilation failed");
+    }
+  }
   std::vector<int32_t> dfifo(phy_fifo_padded(t->down_fifo.size()), t->down_fifo[0]);
   std::vector<int32_t> ufifo(phy_fifo_padded(t->up_fifo.size()), t->up_fifo[0]);
   std::copy(t->down_fifo.begin(), t->down_fifo.end(), dfifo.begin());
   std::copy(t->up_fifo.begin(), t->up_fifo.end(), ufifo.begin());
-  const size_t pd = t->down_prog.size() * sizeof(int32_t), fd = dfifo.size() * sizeof(int32_t);
-  const size_t pu = t->up_prog.size() * sizeof(int32_t), fu = ufifo.size() * sizeof(int32_t);
-  if (e == hipSuccess) e = hipMalloc((void**)&t->d_down_prog, pd);
-  if (e == hipSuccess) e = hipMalloc((void**)&t->d_down_fifo, fd);
-  if (e == hipSuccess) e = hipMalloc((void**)&t->d_up_prog, pu);
-  if (e == hipSuccess) e = hipMalloc((void**)&t->d_up_fifo, fu);
-  if (e == hipSuccess) e = hipMemcpy(t->d_down_prog, t->down_prog.data(), pd, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(t->d_down_fifo, dfifo.data(), fd, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(t->d_up_prog, t->up_prog.data(), pu, hipMemcpyHostToDevice);
-  if (e == hipSuccess) e = hipMemcpy(t->d_up_fifo, ufifo.data(), fu, hipMemcpyHostToDevice);
-  if (e == hipSuccess && !t->parts.empty()) {
-    std::vector<int32_t> pp(t->parts.size());
-    for (size_t k = 0; k < t->parts.size(); ++k) pp[k] = t->parent[t->parts[k]];
-    for (SplitProg* sp : {&t->split_down, &t->split_up})
-      if (e == hipSuccess) e = upload_split(sp);
-    if (e == hipSuccess) e = hipMalloc((void**)&t->d_part_parent, pp.size() * 4);
-    if (e == hipSuccess) e = hipMemcpy(t->d_part_parent, pp.data(), pp.size() * 4, hipMemcpyHostToDevice);
+  TopoUpload up;
+  up.put(t->down_prog, &t->d_down_prog);
+  up.put(dfifo, &t->d_down_fifo);
+  up.put(t->up_prog, &t->d_up_prog);
+  up.put(ufifo, &t->d_up_fifo);
+  up.put(t, &t->split);
+  up.put(t, &t->fine);
+  if (!t->pparts.empty()) {
+    up.put(&t->psplit);
+    up.put(t->ptop_prog, &t->d_ptop_prog);
+    up.put(t->ptop_fifo, &t->d_ptop_fifo);
   }
-  if (e == hipSuccess && !t->pparts.empty()) {
-    if (e == hipSuccess) e = upload_split(&t->psplit);
-    if (e == hipSuccess) e = hipMalloc((void**)&t->d_ptop_prog, t->ptop_prog.size() * 4);
-    if (e == hipSuccess) e = hipMalloc((void**)&t->d_ptop_fifo, t->ptop_fifo.size() * 4);
-    if (e == hipSuccess)
-      e = hipMemcpy(t->d_ptop_prog, t->ptop_prog.data(), t->ptop_prog.size() * 4, hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-      e = hipMemcpy(t->d_ptop_fifo, t->ptop_fifo.data(), t->ptop_fifo.size() * 4, hipMemcpyHostToDevice);
-  }
+  const hipError_t e = up.run(&t->d_programs);
   if (e != hipSuccess) {
     phy_topo_destroy(t);
     return set_err(ctx, PHY_EDEVICE, std::string("topology upload: ") + hipGetErrorString(e));
@@ -609,18 +641,7 @@ int phy_topo_create(phy_ctx* ctx, int32_t N, const int32_t* children, int32_t ro
 
 void phy_topo_destroy(phy_topo* t) {
   if (!t) return;
-  if (t->d_down_prog) (void)hipFree(t->d_down_prog);
-  if (t->d_down_fifo) (void)hipFree(t->d_down_fifo);
-  if (t->d_up_prog) (void)hipFree(t->d_up_prog);
-  if (t->d_up_fifo) (void)hipFree(t->d_up_fifo);
-  for (SplitProg* sp : {&t->split_down, &t->split_up, &t->psplit}) {
-    if (sp->d_prog) (void)hipFree(sp->d_prog);
-    if (sp->d_fifo) (void)hipFree(sp->d_fifo);
-    if (sp->d_meta) (void)hipFree(sp->d_meta);
-  }
-  if (t->d_part_parent) (void)hipFree(t->d_part_parent);
-  if (t->d_ptop_prog) (void)hipFree(t->d_ptop_prog);
-  if (t->d_ptop_fifo) (void)hipFree(t->d_ptop_fifo);
+  if (t->d_programs) (void)hipFree(t->d_programs);
   if (t->d_scratch) (void)hipFree(t->d_scratch);
   delete t;
 }
@@ -637,16 +658,16 @@ int phy_topo_programs(const phy_topo* t, int32_t* down_prog, int32_t* down_fifo,
 
 int phy_topo_split(const phy_topo* t, int32_t* n_parts, int32_t* cut_nodes) {
   if (!t) return PHY_EINVAL;
-  if (n_parts) *n_parts = (int32_t)t->parts.size();
-  if (cut_nodes) std::copy(t->parts.begin(), t->parts.end(), cut_nodes);
+  if (n_parts) *n_parts = (int32_t)t->split.parts.size();
+  if (cut_nodes) std::copy(t->split.parts.begin(), t->split.parts.end(), cut_nodes);
   return PHY_OK;
 }
 
 int phy_topo_split_program(const phy_topo* t, int32_t up, int32_t k, int32_t* prog, int32_t* n_ops,
                            int32_t* fifo, int32_t* n_fifo) {
-  if (!t || t->parts.empty()) return PHY_EINVAL;
-  const SplitProg& sp = up ? t->split_up : t->split_down;
-  if (k < 0 || k > (int32_t)t->parts.size()) return PHY_EINVAL;
+  if (!t || t->split.parts.empty()) return PHY_EINVAL;
+  const SplitProg& sp = up ? t->split.up : t->split.down;
+  if (k < 0 || k > (int32_t)t->split.parts.size()) return PHY_EINVAL;
   const int32_t n = sp.n_ops[k];
   // the fifo of program k ends where the next one's padded fifo begins; its
   // unpadded length is the number of operands the program reads

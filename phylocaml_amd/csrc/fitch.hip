@@ -15,9 +15,10 @@
 // preliminary set written once (down), every set read once and every final
 // set written once (up).  The operand stream (leaves for the down-pass, node
 // sets for the up-pass) is consumed in a fixed order and is prefetched a
-// batch ahead through registers into an LDS ring.  Trees of >= 128 leaves
-// run split: parts under cut nodes side by side (grid.y = part), plus a top
-// program, which multiplies the waves in flight by the number of parts.
+// batch ahead through registers into an LDS ring.  Larger trees run split:
+// parts under cut nodes side by side (grid.y = part), plus a top program,
+// which multiplies the waves in flight by the number of parts (pass_shape
+// chooses between a coarse and a fine split).
 #include <algorithm>
 #include <cstdlib>
 
@@ -204,6 +205,66 @@ __device__ __forceinline__ uint64_t weigh32(uint32_t e, const uint32_t* __restri
   return c;
 }
 
+// Weights of a lane's 8V sites as bit planes in the nibble layout: bit 0 of
+// nibble k of plane b is bit b of site k's weight, so the weight of the flagged
+// sites e of a word is sum_b popcount(e & plane_b) 2^b.  Up to kPlanes bits; a
+// wave with a heavier site adds its flagged sites one by one.  (That walk, a
+// dependent load per flagged site and node, took the down-pass of 301 taxa x
+// 50,021 weighted sites with node costs from 81 us unweighted to 210; with the
+// planes 36 and 42.)
+constexpr int kPlanes = 8;
+
+template <int V>
+struct WeightPlanes {
+  uint32_t p[kPlanes][V];
+  int n;  // planes in use in this wave; > kPlanes: none, walk the sites
+
+  __device__ __forceinline__ void load(const uint32_t* __restrict__ wt, int64_t word, int64_t n_sites, bool act) {
+    uint32_t any = 0;
+#pragma unroll
+    for (int b = 0; b < kPlanes; ++b)
+#pragma unroll
+      for (int i = 0; i < V; ++i) p[b][i] = 0;
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int64_t s = (word + i) * 8 + k;
+        const uint32_t w = act && s < n_sites ? wt[s] : 0u;
+        any |= w;
+#pragma unroll
+        for (int b = 0; b < kPlanes; ++b) p[b][i] |= ((w >> b) & 1u) << (4 * k);
+      }
+    n = 0;
+#pragma unroll
+    for (int b = 0; b < kPlanes; ++b)
+      if (__ballot((any >> b) & 1u)) n = b + 1;
+    if (__ballot(any >> kPlanes)) n = kPlanes + 1;
+  }
+  __device__ __forceinline__ uint32_t weigh(const uint32_t* e) const {
+    uint32_t c = 0;
+#pragma unroll
+    for (int b = 0; b < kPlanes; ++b) {
+      if (b >= n) break;
+      uint32_t m = 0;
+#pragma unroll
+      for (int i = 0; i < V; ++i) m += __popc(e[i] & p[b][i]);
+      c += m << b;
+    }
+    return c;
+  }
+};
+
+// sum over the wave (no overflow: at most 8V sites of weight < 2^kPlanes a lane)
+__device__ __forceinline__ uint32_t wave_sum32(uint32_t v) {
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, false);  // row_ror:8
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xF, 0xF, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xF, 0xF, false);
+  v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xF, 0xF, false);
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 0) + (uint32_t)__builtin_amdgcn_readlane((int)v, 16) +
+         (uint32_t)__builtin_amdgcn_readlane((int)v, 32) + (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+}
+
 // V 32-bit words (8 sites each) per thread, loaded and stored as one
 // 4V-byte access
 template <int V>
@@ -263,18 +324,25 @@ enum : int { MODE_WHOLE = 0, MODE_PART = 1, MODE_TOP = 2 };
   } while (0)
 
 // W = number of 32-bit words per node row; lane w owns words V*w .. V*w+V-1
-template <int BATCH, bool NODE_COST, int MODE, int V, bool NT>
+template <int BATCH, bool NODE_COST, int MODE, int V, bool NT, bool PACED>
 __global__ __launch_bounds__(256) void k_fitch_down(
     const int4* __restrict__ prog, int n_ops, const int32_t* __restrict__ fifo_ids,
     const int32_t* __restrict__ meta, int n_parts, uint4* __restrict__ scratch, int narrow,
     uint32_t* __restrict__ sets32, int64_t stride, int64_t W, int64_t n_sites, int N,
     const uint32_t* __restrict__ wt, uint32_t* __restrict__ site_cost,
-    unsigned long long* __restrict__ node_cost, unsigned long long* __restrict__ total) {
+    unsigned long long* __restrict__ node_cost, unsigned long long* __restrict__ total, int nc_off) {
   using T = Words<V>;
   extern __shared__ uint4 lds_dyn[];
   const int tid = threadIdx.x, bd = blockDim.x;
   const int part = MODE == MODE_PART ? (int)blockIdx.y : n_parts;
   if (MODE != MODE_WHOLE) SPLIT_SELECT(part);
+  // node costs of the block, at byte nc_off of the LDS (nc_off < 0: a program
+  // too long for that, each wave adds to node_cost at every node)
+  unsigned long long* ncl = reinterpret_cast<unsigned long long*>(reinterpret_cast<char*>(lds_dyn) + nc_off);
+  if (NODE_COST && nc_off >= 0) {
+    for (int k = tid; k < n_ops; k += bd) ncl[k] = 0;
+    __syncthreads();
+  }
   const int64_t L = W / V;                           // lanes (W is a multiple of V)
   const int64_t w = (int64_t)blockIdx.x * bd + tid;  // lane index
   const bool act = w < L;
@@ -285,6 +353,9 @@ __global__ __launch_bounds__(256) void k_fitch_down(
   T* stk = ring + (size_t)2 * BATCH * bd;
   OperandRing<BATCH, SetLoad<V, NT>, T> leaves;
   leaves.init(ring, fifo_ids, SetLoad<V, NT>{sets, strideT, wc}, bd, tid);
+
+  WeightPlanes<V> planes;
+  if (NODE_COST && wt) planes.load(wt, wc * V, n_sites, act);
 
   uint32_t cnt[V];  // nibble counters, flushed every 15 nodes
   uint32_t site[8 * V];
@@ -299,7 +370,7 @@ __global__ __launch_bounds__(256) void k_fitch_down(
   int since = 0;
   T acc = {};
   int sp = 0;
-  for_each_entry(prog, n_ops, [&](int, const int4 op) {
+  for_each_entry<PACED>(prog, n_ops, [&](int i_op, const int4 op) {
     const int fl = op.w;
     if (fl & DOWN_SPILL) {
       stk[sp * bd + tid] = acc;
@@ -322,16 +393,26 @@ __global__ __launch_bounds__(256) void k_fitch_down(
     }
     if (act) st_row<V, NT>(sets + (int64_t)op.x * strideT + w, acc);
     if (NODE_COST) {
-      uint64_t c = 0;
-      if (act) {
+      uint32_t m[V];
 #pragma unroll
-        for (int i = 0; i < V; ++i) {
-          const uint32_t m = e[i] & vm[i];
-          c += wt ? weigh32(m, wt, w * V + i) : (uint64_t)__popc(m);
+      for (int i = 0; i < V; ++i) m[i] = act ? e[i] & vm[i] : 0u;
+      uint64_t c = 0;
+      if (wt && planes.n > kPlanes) {  // wave-uniform
+#pragma unroll
+        for (int i = 0; i < V; ++i) c += weigh32(m[i], wt, w * V + i);
+        c = wave_sum(c);
+      } else {
+        uint32_t c32 = 0;
+        if (wt) {
+          c32 = planes.weigh(m);
+        } else {
+#pragma unroll
+          for (int i = 0; i < V; ++i) c32 += __popc(m[i]);
         }
+        c = wave_sum32(c32);
       }
-      c = wave_sum(c);
-      if ((tid & 63) == 0 && c) atomicAdd(&node_cost[op.x - N], (unsigned long long)c);
+      if ((tid & 63) == 0 && c)
+        atomicAdd(nc_off >= 0 ? ncl + i_op : node_cost + (op.x - N), (unsigned long long)c);
     }
     if (++since == 15) {
 #pragma unroll
@@ -347,6 +428,13 @@ __global__ __launch_bounds__(256) void k_fitch_down(
   for (int i = 0; i < V; ++i)
 #pragma unroll
     for (int k = 0; k < 8; ++k) site[8 * i + k] += (cnt[i] >> (4 * k)) & 15u;
+  // one vector of atomics for 64 nodes of the block instead of one atomic a
+  // wave and node (64 taxa x 10^6 sites with node costs: 120 us so, now 50)
+  if (NODE_COST && nc_off >= 0) {
+    __syncthreads();
+    for (int k = tid; k < n_ops; k += bd)
+      if (ncl[k]) atomicAdd(&node_cost[prog[k].x - N], ncl[k]);
+  }
   if (MODE == MODE_PART) {
     if (act) {
       if (narrow) {  // 4 counts per word, 8V bytes per lane
@@ -652,43 +740,93 @@ int phy_fitch_select(phy_ctx* ctx, const uint64_t* d_states, int64_t n_sites,
 
 namespace {
 
-// Split passes (parts side by side, then the top) unless disabled; the
-// whole-tree program otherwise.
-bool use_split(const phy_topo* t) {
+// How a pass runs: the split (nullptr: the whole-tree program), the words per
+// lane it would like, and its block size.
+struct PassShape {
+  const FitchSplit* split;
+  int words, block;
+};
+
+// A pass with few waves is bound by its longest chain of nodes (0.3-0.9 us a
+// node at one wave per SIMD: instruction latency, at any ring depth), so it
+// takes the fine split, narrow lanes and one-wave blocks; a pass that fills
+// the chip takes the coarse split, whose larger parts write less scratch, with
+// wide lanes.  Down / up in us, coarse and fine: 32 taxa x 2,000 sites
+// 13.2 / 17.8 and 11.5 / 8.9; 301 x 50,021 41 / 77 and 24 / 30; 1,024 x 100,000
+// 70 / 106 and 51 / 66; 301 x 600,000 60 / 134 and 64 / 96; 1,024 x 300,000
+// 98 / 190 and 102 / 168; 64 x 10^6 40 / 41 and 41 / 31; 33 x 10^6 24 / 23 and
+// 33 / 21.  So the lines lie at 1,024 waves of the coarse pass down (16-byte
+// lanes; 256 where the coarse pass is the whole tree, whose chain is short),
+// and at 8,192 up (8-byte lanes); the up-pass narrows to
+// 4-byte lanes below 4,096 waves (1,024 x 100,000: 66 against 72 us; 301 x
+// 600,000: 102 against 96).  Trees below 24 leaves run whole (16 x 2,000 down:
+// 8.5 whole, 10.8 split).
+PassShape pass_shape(const phy_topo* t, int64_t W32, bool up) {
   const char* e = getenv("PHY_FITCH_SPLIT");
-  return t->parts.size() >= 2 && t->split_down.d_prog && !(e && e[0] == '0');
+  const bool may_split = !(e && e[0] == '0');
+  const FitchSplit* coarse = may_split && t->split.parts.size() >= 2 && t->split.down.d_prog ? &t->split : nullptr;
+  const FitchSplit* fine = may_split && t->fine.down.d_prog ? &t->fine : nullptr;
+  auto waves = [&](int words, const FitchSplit* f) {
+    return (W32 / words + 63) / 64 * (f ? (int64_t)f->parts.size() : 1);
+  };
+  if (up) {
+    if (waves(2, coarse) >= 8192) return {coarse, 2, 256};
+    const FitchSplit* f = fine ? fine : coarse;
+    return {f, waves(2, f) < 4096 ? 1 : 2, 64};
+  }
+  if (waves(4, coarse) >= (coarse ? 1024 : 256)) return {coarse, 4, 256};
+  return {fine ? fine : coarse, 2, 64};
 }
 
-template <int BATCH, int V, bool NT>
-int downpass_launch(phy_ctx* ctx, const phy_topo* topo, uint32_t* s32, int64_t stride32,
+// Scratch rows of the split down-pass (the part counts of every lane), grown on
+// demand.  During a graph capture nothing can be allocated, so a pass whose
+// fine split needs more than is there takes the coarse one (or runs whole).
+size_t scratch_need(const FitchSplit* f, int64_t W32) {
+  return f ? f->parts.size() * (size_t)W32 * 8 * sizeof(uint32_t) : 0;  // 8 counts per 32-bit word
+}
+bool capturing(phy_ctx* ctx) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(ctx->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
+template <int BATCH, int V, bool NT, bool PACED>
+int downpass_run(phy_ctx* ctx, const phy_topo* topo, uint32_t* s32, int64_t stride32,
                     int64_t W32, int64_t n_sites, const uint32_t* wt, uint32_t* site_cost,
-                    unsigned long long* node_cost, unsigned long long* total, int bs) {
+                    unsigned long long* node_cost, unsigned long long* total, int bs, const FitchSplit* split) {
   const int N = topo->n_leaves;
-  const bool split = use_split(topo);
-  const int depth = split ? topo->split_down.depth : topo->down_depth;
+  const int depth = split ? split->down.depth : topo->down_depth;
   // LDS per thread: the operand ring (2 BATCH entries) and the stack, V words
   // each; the block shrinks (down to one wave) until they fit
   auto lds_of = [&](int b) { return (size_t)(2 * BATCH + depth) * b * 4 * V; };
   while (bs > 64 && lds_of(bs) > 64 * 1024) bs /= 2;
-  const size_t lds = lds_of(bs);
+  size_t lds = lds_of(bs);
   if (lds > 64 * 1024) return set_err(ctx, PHY_ERANGE, "downpass: LDS stack too deep for this tree");
+  // the block's node costs after them, where they fit
+  int nc_off = -1;
+  if (node_cost) {
+    const int ops = split ? *std::max_element(split->down.n_ops.begin(), split->down.n_ops.end()) : N - 1;
+    if (lds + (size_t)ops * 8 <= 64 * 1024) {  // lds is a multiple of 16
+      nc_off = (int)lds;
+      lds += (size_t)ops * 8;
+    }
+  }
   const unsigned grid = (unsigned)((W32 / V + bs - 1) / bs);
   if (!split) {
     KernelSpan span(ctx, "fitch_down");
     if (node_cost)
-      hipLaunchKernelGGL((k_fitch_down<BATCH, true, MODE_WHOLE, V, NT>), dim3(grid), dim3(bs), lds, ctx->stream,
+      hipLaunchKernelGGL((k_fitch_down<BATCH, true, MODE_WHOLE, V, NT, PACED>), dim3(grid), dim3(bs), lds, ctx->stream,
                          topo->d_down_prog, N - 1, topo->d_down_fifo, nullptr, 0, nullptr, 0, s32, stride32, W32,
-                         n_sites, N, wt, site_cost, node_cost, total);
+                         n_sites, N, wt, site_cost, node_cost, total, nc_off);
     else
-      hipLaunchKernelGGL((k_fitch_down<BATCH, false, MODE_WHOLE, V, NT>), dim3(grid), dim3(bs), lds, ctx->stream,
+      hipLaunchKernelGGL((k_fitch_down<BATCH, false, MODE_WHOLE, V, NT, PACED>), dim3(grid), dim3(bs), lds, ctx->stream,
                          topo->d_down_prog, N - 1, topo->d_down_fifo, nullptr, 0, nullptr, 0, s32, stride32, W32,
-                         n_sites, N, wt, site_cost, node_cost, total);
+                         n_sites, N, wt, site_cost, node_cost, total, nc_off);
     PHY_LAUNCHED(ctx);
     return PHY_OK;
   }
-  const SplitProg& sp = topo->split_down;
-  const int P = (int)topo->parts.size();
-  const size_t need = (size_t)P * W32 * 8 * sizeof(uint32_t);  // 8 counts per 32-bit word
+  const SplitProg& sp = split->down;
+  const int P = (int)split->parts.size();
+  const size_t need = scratch_need(split, W32);
   if (topo->scratch_bytes < need) {
     if (topo->d_scratch) PHY_HIP(ctx, hipFree(topo->d_scratch));
     topo->d_scratch = nullptr;
@@ -707,32 +845,44 @@ int downpass_launch(phy_ctx* ctx, const phy_topo* topo, uint32_t* s32, int64_t s
   const int narrow = max_ops <= 255 && !(ne && ne[0] == '0');
   KernelSpan span(ctx, "fitch_down");
   if (node_cost) {
-    hipLaunchKernelGGL((k_fitch_down<BATCH, true, MODE_PART, V, NT>), dim3(grid, (unsigned)P), dim3(bs), lds,
+    hipLaunchKernelGGL((k_fitch_down<BATCH, true, MODE_PART, V, NT, PACED>), dim3(grid, (unsigned)P), dim3(bs), lds,
                        ctx->stream, sp.d_prog, 0, sp.d_fifo, sp.d_meta, P, scr, narrow, s32, stride32, W32, n_sites,
-                       N, wt, site_cost, node_cost, total);
+                       N, wt, site_cost, node_cost, total, nc_off);
     PHY_LAUNCHED(ctx);
-    hipLaunchKernelGGL((k_fitch_down<BATCH, true, MODE_TOP, V, NT>), dim3(grid), dim3(bs), lds, ctx->stream,
+    hipLaunchKernelGGL((k_fitch_down<BATCH, true, MODE_TOP, V, NT, PACED>), dim3(grid), dim3(bs), lds, ctx->stream,
                        sp.d_prog, 0, sp.d_fifo, sp.d_meta, P, scr, narrow, s32, stride32, W32, n_sites, N, wt,
-                       site_cost, node_cost, total);
+                       site_cost, node_cost, total, nc_off);
   } else {
-    hipLaunchKernelGGL((k_fitch_down<BATCH, false, MODE_PART, V, NT>), dim3(grid, (unsigned)P), dim3(bs), lds,
+    hipLaunchKernelGGL((k_fitch_down<BATCH, false, MODE_PART, V, NT, PACED>), dim3(grid, (unsigned)P), dim3(bs), lds,
                        ctx->stream, sp.d_prog, 0, sp.d_fifo, sp.d_meta, P, scr, narrow, s32, stride32, W32, n_sites,
-                       N, wt, site_cost, node_cost, total);
+                       N, wt, site_cost, node_cost, total, nc_off);
     PHY_LAUNCHED(ctx);
-    hipLaunchKernelGGL((k_fitch_down<BATCH, false, MODE_TOP, V, NT>), dim3(grid), dim3(bs), lds, ctx->stream,
+    hipLaunchKernelGGL((k_fitch_down<BATCH, false, MODE_TOP, V, NT, PACED>), dim3(grid), dim3(bs), lds, ctx->stream,
                        sp.d_prog, 0, sp.d_fifo, sp.d_meta, P, scr, narrow, s32, stride32, W32, n_sites, N, wt,
-                       site_cost, node_cost, total);
+                       site_cost, node_cost, total, nc_off);
   }
   PHY_LAUNCHED(ctx);
   return PHY_OK;
 }
 
+// paced: see stream.hpp; only the widest lanes ever fill the chip
+template <int BATCH, int V, bool NT>
+int downpass_launch(phy_ctx* ctx, const phy_topo* topo, uint32_t* s32, int64_t stride32, int64_t W32,
+                    int64_t n_sites, const uint32_t* wt, uint32_t* site_cost, unsigned long long* node_cost,
+                    unsigned long long* total, int bs, const FitchSplit* split) {
+  const int64_t waves = (W32 / V + 63) / 64 * (split ? (int64_t)split->parts.size() : 1);
+  if (V == 4 && waves >= 4096)
+    return downpass_run<BATCH, V, NT, V == 4>(ctx, topo, s32, stride32, W32, n_sites, wt, site_cost, node_cost,
+                                              total, bs, split);
+  return downpass_run<BATCH, V, NT, false>(ctx, topo, s32, stride32, W32, n_sites, wt, site_cost, node_cost, total,
+                                           bs, split);
+}
+
 template <int BATCH, int V, bool NT>
 int uppass_launch(phy_ctx* ctx, const phy_topo* topo, const uint32_t* s32, uint32_t* f32,
-                  int64_t stride32, int64_t W32, int bs) {
+                  int64_t stride32, int64_t W32, int bs, const FitchSplit* split) {
   const int N = topo->n_leaves;
-  const bool split = use_split(topo);
-  const int depth = split ? topo->split_up.depth : topo->up_depth;
+  const int depth = split ? split->up.depth : topo->up_depth;
   auto lds_of = [&](int b) { return (size_t)(2 * BATCH + 2 * depth) * b * 4 * V; };
   while (bs > 64 && lds_of(bs) > 64 * 1024) bs /= 2;
   const size_t lds = lds_of(bs);
@@ -746,13 +896,13 @@ int uppass_launch(phy_ctx* ctx, const phy_topo* topo, const uint32_t* s32, uint3
     PHY_LAUNCHED(ctx);
     return PHY_OK;
   }
-  const SplitProg& sp = topo->split_up;
-  const int P = (int)topo->parts.size();
+  const SplitProg& sp = split->up;
+  const int P = (int)split->parts.size();
   hipLaunchKernelGGL((k_fitch_up<BATCH, MODE_TOP, V, NT>), dim3(grid), dim3(bs), lds, ctx->stream, sp.d_prog,
-                     0, sp.d_fifo, sp.d_meta, P, topo->d_part_parent, s32, f32, stride32, W32, N);
+                     0, sp.d_fifo, sp.d_meta, P, split->d_part_parent, s32, f32, stride32, W32, N);
   PHY_LAUNCHED(ctx);
   hipLaunchKernelGGL((k_fitch_up<BATCH, MODE_PART, V, NT>), dim3(grid, (unsigned)P), dim3(bs), lds,
-                     ctx->stream, sp.d_prog, 0, sp.d_fifo, sp.d_meta, P, topo->d_part_parent, s32, f32,
+                     ctx->stream, sp.d_prog, 0, sp.d_fifo, sp.d_meta, P, split->d_part_parent, s32, f32,
                      stride32, W32, N);
   PHY_LAUNCHED(ctx);
   return PHY_OK;
@@ -807,18 +957,22 @@ int phy_fitch_downpass(phy_ctx* ctx, const phy_topo* topo, uint64_t* sets, int64
   if ((rc = phy_zero_u64(ctx, total, 1))) return rc;
   if (node_cost && (rc = phy_zero_u64(ctx, node_cost, N - 1))) return rc;
   if (W == 0) return PHY_OK;
-  const int bs = block_size_env("PHY_FITCH_BLOCK", 256);
   const int64_t W32 = 2 * W;  // 32-bit lanes
+  PassShape sh = pass_shape(topo, W32, false);
+  if (sh.split == &topo->fine && topo->scratch_bytes < scratch_need(sh.split, W32) && capturing(ctx))
+    sh.split = topo->split.parts.size() >= 2 ? &topo->split : nullptr;
+  const FitchSplit* split = sh.split;
+  const int bs = block_size_env("PHY_FITCH_BLOCK", sh.block);
   uint32_t* s32 = reinterpret_cast<uint32_t*>(sets);
   auto* nc = reinterpret_cast<unsigned long long*>(node_cost);
   auto* tt = reinterpret_cast<unsigned long long*>(total);
-  // 16-byte non-temporal lanes and a 4-deep ring: at 1,024 taxa x 10^6
-  // sites 0.243 ms against 0.266 ms for 8-byte cached lanes and an 8-deep
-  // ring (sweep over words 1 / 2 / 4, ring 4 / 8 / 16, non-temporal or not,
+  // full passes take 16-byte non-temporal lanes and a 4-deep ring: at 1,024
+  // taxa x 10^6 sites 0.243 ms against 0.266 ms for 8-byte cached lanes and an
+  // 8-deep ring (sweep over words 1 / 2 / 4, ring 4 / 8 / 16, non-temporal or not,
   // blocks of 128 / 256, 8 / 16 / 32 parts)
-  const int v = lane_words(words_env(4), s32, 2 * stride, W32);
-#define PHY_DOWN(B, VV) (nt_env(true) ? downpass_launch<B, VV, true>(ctx, topo, s32, 2 * stride, W32, n_sites, wt, site_cost, nc, tt, bs) \
-                              : downpass_launch<B, VV, false>(ctx, topo, s32, 2 * stride, W32, n_sites, wt, site_cost, nc, tt, bs))
+  const int v = lane_words(words_env(sh.words), s32, 2 * stride, W32);
+#define PHY_DOWN(B, VV) (nt_env(true) ? downpass_launch<B, VV, true>(ctx, topo, s32, 2 * stride, W32, n_sites, wt, site_cost, nc, tt, bs, split) \
+                              : downpass_launch<B, VV, false>(ctx, topo, s32, 2 * stride, W32, n_sites, wt, site_cost, nc, tt, bs, split))
   switch (batch_env(4)) {
     case 4: return v == 4 ? PHY_DOWN(4, 4) : v == 2 ? PHY_DOWN(4, 2) : PHY_DOWN(4, 1);
     case 8: return v == 4 ? PHY_DOWN(8, 4) : v == 2 ? PHY_DOWN(8, 2) : PHY_DOWN(8, 1);
@@ -836,16 +990,17 @@ int phy_fitch_uppass(phy_ctx* ctx, const phy_topo* topo, const uint64_t* sets, u
   if (n_sites < 0 || stride < W) return set_err(ctx, PHY_EINVAL, "uppass: stride < words");
   if (!sets || !fin) return set_err(ctx, PHY_EINVAL, "uppass: null buffer");
   if (W == 0) return PHY_OK;
-  const int bs = block_size_env("PHY_FITCH_BLOCK", 256);
   const int64_t W32 = 2 * W;
+  const PassShape sh = pass_shape(topo, W32, true);
+  const int bs = block_size_env("PHY_FITCH_BLOCK", sh.block);
   const uint32_t* s32 = reinterpret_cast<const uint32_t*>(sets);
   uint32_t* f32 = reinterpret_cast<uint32_t*>(fin);
-  // 8-byte cached lanes, 4-deep ring: 0.485 ms at 1,024 x 10^6 (16-byte
-  // non-temporal lanes 0.491 ms)
-  const int v = std::min(lane_words(words_env(2), s32, 2 * stride, W32),
-                         lane_words(words_env(2), f32, 2 * stride, W32));
-#define PHY_UP(B, VV) (nt_env(false) ? uppass_launch<B, VV, true>(ctx, topo, s32, f32, 2 * stride, W32, bs) \
-                            : uppass_launch<B, VV, false>(ctx, topo, s32, f32, 2 * stride, W32, bs))
+  // full passes take 8-byte cached lanes and a 4-deep ring: 0.485 ms at
+  // 1,024 x 10^6 (16-byte non-temporal lanes 0.491 ms)
+  const int v = std::min(lane_words(words_env(sh.words), s32, 2 * stride, W32),
+                         lane_words(words_env(sh.words), f32, 2 * stride, W32));
+#define PHY_UP(B, VV) (nt_env(false) ? uppass_launch<B, VV, true>(ctx, topo, s32, f32, 2 * stride, W32, bs, sh.split) \
+                            : uppass_launch<B, VV, false>(ctx, topo, s32, f32, 2 * stride, W32, bs, sh.split))
   switch (batch_env(4)) {
     case 4: return v == 4 ? PHY_UP(4, 4) : v == 2 ? PHY_UP(4, 2) : PHY_UP(4, 1);
     case 8: return v == 4 ? PHY_UP(8, 4) : v == 2 ? PHY_UP(8, 2) : PHY_UP(8, 1);

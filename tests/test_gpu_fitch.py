@@ -193,3 +193,20 @@ def test_empty_and_bad_arguments(ctx):
     host_topo = D.Topology(3, np.array([0, 1, 2, 3], np.int32), 4)
     assert lib.phy_fitch_uppass(ctx.handle, host_topo.handle, D.dptr(buf), D.dptr(buf), 1,
                                 1) == 1
+
+
+@pytest.mark.parametrize("N,S", [(23, 700), (24, 700), (40, 1), (40, 513), (301, 20_011),
+                                 (24, 530_001), (130, 400_003)])
+@pytest.mark.parametrize("weights", ["unit", "small", "heavy"])
+def test_pass_shapes_and_node_costs(ctx, rng, N, S, weights):
+    # both sides of the dispatch lines (whole tree below 24 leaves, fine split
+    # with narrow lanes, whole tree and wide lanes at many sites) with node
+    # costs counted, weighed by bit planes (up to 8 bits) or walked (one site
+    # of 2^20 makes its wave do so)
+    _say(f"fitch shapes N={N} S={S} weights={weights}")
+    ch, root = random_tree(rng, N)
+    leaves = rng.integers(1, 16, (N, S)).astype(np.uint8)
+    w = None if weights == "unit" else rng.integers(0, 256, S).astype(np.uint32)
+    if weights == "heavy":
+        w[S // 2] = 1 << 20
+    _tree_case(ctx, N, ch, root, leaves, w)
