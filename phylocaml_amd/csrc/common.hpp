@@ -94,6 +94,22 @@ struct FitchSplit {
   int32_t* d_part_parent = nullptr;
 };
 
+// Programs of the fused pruning pass with its cherries (nodes of two leaves)
+// as operands read from a table: one per part of the split form, or one for the
+// whole tree.  Entry {slot of A | slot of B << 16, node of A, node of B, flags}
+// with SRC_EXT for a table operand (its node field names some valid node) and,
+// from bit 8 of the flags, the row of the entry's first leaf or table operand
+// among the program's operands.  The fifo holds a pair of leaves per operand, in
+// row order: a cherry's two, or a leaf and -1.
+struct TabProg {
+  SplitProg sp;                 // prog, fifo, offsets; depth
+  std::vector<int32_t> n_rows;  // operands per program
+  std::vector<int32_t> cherry;  // {node, leaf a, leaf b, 0} per slot
+  int32_t n_progs = 0, max_rows = 0;
+  int4* d_cherry = nullptr;
+  int32_t* d_rows = nullptr;
+};
+
 struct phy_topo {
   phy_ctx* ctx = nullptr;
   int32_t n_leaves = 0;
@@ -128,6 +144,7 @@ struct phy_topo {
   SplitProg psplit;
   std::vector<int32_t> ptop_prog, ptop_fifo;
   int32_t ptop_depth = 0;
+  TabProg tab;
   int4* d_ptop_prog = nullptr;
   int32_t* d_ptop_fifo = nullptr;
   // per-part partial site costs of the split down-pass, grown on demand

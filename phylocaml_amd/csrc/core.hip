@@ -359,6 +359,63 @@ std::vector<int32_t> choose_cuts(int32_t N, const std::vector<int32_t>& ch,
   return cuts;
 }
 
+// Table programs of the subtrees under `tops` (see TabProg); none when a top is
+// itself a cherry or there are too many slots for 16 bits.
+int compile_tab(const phy_topo* t, const std::vector<int32_t>& tops, TabProg* out) {
+  const int32_t N = t->n_leaves;
+  const std::vector<int32_t>& ch = t->children;
+  *out = TabProg();
+  auto cherry = [&](int32_t v) { return v >= N && ch[2 * (v - N)] < N && ch[2 * (v - N) + 1] < N; };
+  const Stop stop = [N, &cherry](int32_t v) { return v < N || cherry(v); };
+  TabProg tp;
+  std::vector<int32_t> pg, ff;
+  int32_t d = 0;
+  for (int32_t top : tops) {
+    if (stop(top)) return 0;
+    if (!compile_down(N, ch, top, stop, &pg, &ff, &d)) return 11;
+    std::vector<int32_t> rows, prog;  // rows: leaf pairs
+    int32_t leaves = 0;
+    auto operand = [&](int32_t v, int src, int32_t* slot) {
+      if (src != SRC_LEAF) return src;
+      if (v < N) {
+        rows.insert(rows.end(), {v, -1});
+        ++leaves;
+        return src;
+      }
+      const int32_t a = ch[2 * (v - N)], b = ch[2 * (v - N) + 1];
+      rows.insert(rows.end(), {a, b});
+      leaves += 2;
+      *slot = (int32_t)tp.cherry.size() / 4;
+      tp.cherry.insert(tp.cherry.end(), {v, a, b, 0});
+      return (int)SRC_EXT;
+    };
+    int32_t subtree_ops = 0;
+    for (size_t i = 0; i < pg.size(); i += 4) {
+      const int32_t A = pg[i + 1], B = pg[i + 2], fl = pg[i + 3];
+      int32_t ka = 0, kb = 0;
+      const int32_t row = (int32_t)rows.size() / 2;
+      const int sa = operand(A, fl & 3, &ka), sb = operand(B, (fl >> 2) & 3, &kb);
+      const bool ta = sa == SRC_EXT, tb = sb == SRC_EXT;
+      if (ka > 0xffff || kb > 0xffff) return 0;
+      prog.insert(prog.end(), {ka | (int32_t)((uint32_t)kb << 16), ta ? (tb ? 0 : B) : A, tb ? (ta ? 0 : A) : B,
+                               (fl & ~15) | sa | (sb << 2) | (row << 8)});
+      subtree_ops += 1 + (ta ? 1 : 0) + (tb ? 1 : 0);
+    }
+    if (subtree_ops != t->subtree[top] - 1 || leaves != t->subtree[top]) return 12;
+    tp.sp.prog_off.push_back((int32_t)tp.sp.prog.size() / 4);
+    tp.sp.n_ops.push_back((int32_t)prog.size() / 4);
+    tp.sp.fifo_off.push_back((int32_t)tp.sp.fifo.size());
+    tp.sp.prog.insert(tp.sp.prog.end(), prog.begin(), prog.end());
+    tp.sp.fifo.insert(tp.sp.fifo.end(), rows.begin(), rows.end());
+    tp.sp.depth = std::max(tp.sp.depth, d);
+    tp.n_rows.push_back((int32_t)rows.size() / 2);
+    tp.max_rows = std::max(tp.max_rows, tp.n_rows.back());
+    ++tp.n_progs;
+  }
+  *out = tp;
+  return 0;
+}
+
 // Programs of the Fitch passes split under at most `want` cut nodes of at
 // least `min_leaves` leaves (no parts when fewer than two are found).
 int compile_fitch_split(const phy_topo* t, int want, int32_t min_leaves, FitchSplit* out) {
@@ -614,6 +671,14 @@ int phy_topo_create(phy_ctx* ctx, int32_t N, const int32_t* children, int32_t ro
       return set_err(ctx, PHY_EINVAL, "topology: program compilation failed");
     }
   }
+  // the table form pays where the patterns are many: see use_tables (prune.hip)
+  if (N >= 16) {
+    const std::vector<int32_t> whole = {t->root};
+    if (compile_tab(t, t->pparts.empty() ? whole : t->pparts, &t->tab)) {
+      delete t;
+      return set_err(ctx, PHY_EINVAL, "topology: program compilation failed");
+    }
+  }
   std::vector<int32_t> dfifo(phy_fifo_padded(t->down_fifo.size()), t->down_fifo[0]);
   std::vector<int32_t> ufifo(phy_fifo_padded(t->up_fifo.size()), t->up_fifo[0]);
   std::copy(t->down_fifo.begin(), t->down_fifo.end(), dfifo.begin());
@@ -629,6 +694,11 @@ int phy_topo_create(phy_ctx* ctx, int32_t N, const int32_t* children, int32_t ro
     up.put(&t->psplit);
     up.put(t->ptop_prog, &t->d_ptop_prog);
     up.put(t->ptop_fifo, &t->d_ptop_fifo);
+  }
+  if (t->tab.n_progs) {
+    up.put(&t->tab.sp);
+    up.put(t->tab.cherry, &t->tab.d_cherry);
+    up.put(t->tab.n_rows, &t->tab.d_rows);
   }
   const hipError_t e = up.run(&t->d_programs);
   if (e != hipSuccess) {

@@ -698,6 +698,170 @@ __global__ __launch_bounds__(512) void k_prune_part(
   if (!STORE) st.ext_store(y);
 }
 
+// ---------------------------------------------------------------------------
+// Table form of the fused pass.  A third of a tree's internal nodes are cherries
+// (both children leaves): their partial, carried along the branch above them,
+//   y = P_c ((P_a x(code_a)) (*) (P_b x(code_b))),
+// depends on the two 4-bit codes alone.  k_cherry_tab forms y for the 256 code
+// pairs of every cherry and class (the same operations in the same order as the
+// walk, so the results are the same bits), and the walk reads it as an operand:
+// one 16-byte (FP32) gather instead of a program entry and a product, ~8 VALU
+// instructions instead of ~90.  Entry [slot][class][code_a | code_b << 4]; an
+// entry that was rescaled carries its sign bit on y[0] (the values themselves
+// are never negative) and its exponent in etab.
+//
+// The walk stages the codes of its tile in LDS first, one byte per operand (a
+// leaf's code, or a cherry's pair) and pattern, shared by the R waves (each wave
+// of the plain walk loads its own), so that an operand's code is one LDS read
+// and the gathers are the only vector loads.  512 taxa x 200,000 patterns, R = 4,
+// whole evaluation: FP32 674 -> 465 us, FP64 904 -> 597 us; 411M -> 237M VALU wave
+// instructions a pass, still VALU-issue bound (97% of the issue cycles).  The
+// leaves' own products from a 16-entry table as well measured slower (510 us:
+// twice the gathers, each ~36 L1 accesses, against 20 VALU instructions saved).
+// ---------------------------------------------------------------------------
+constexpr int kTabCodes = 256;
+
+template <typename real, int R>
+__global__ __launch_bounds__(kTabCodes) void k_cherry_tab(const int4* __restrict__ cherry,
+                                                          const real* __restrict__ Pm, real* __restrict__ tab,
+                                                          int32_t* __restrict__ etab) {
+  const int k = blockIdx.x / R, r = blockIdx.x % R, code = threadIdx.x;
+  const int4 c = cherry[k];
+  real x[4], ya[4], yb[4], v[4], y[4];
+  int e = 0;
+  tipvec((uint32_t)code & 15u, x);
+  matvec4(Pm + ((size_t)c.y * R + r) * 16, x, ya);
+  tipvec((uint32_t)code >> 4, x);
+  matvec4(Pm + ((size_t)c.z * R + r) * 16, x, yb);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = ya[i] * yb[i];
+  rescale4(v, &e);
+  matvec4(Pm + ((size_t)c.x * R + r) * 16, v, y);
+  y[0] = e != 0 ? -y[0] : y[0];
+  real* d = tab + ((size_t)blockIdx.x * kTabCodes + code) * 4;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) d[i] = y[i];
+  etab[(size_t)blockIdx.x * kTabCodes + code] = e;
+}
+
+__device__ __forceinline__ bool sign_set(float x) { return (int32_t)__float_as_uint(x) < 0; }
+__device__ __forceinline__ bool sign_set(double x) { return __double2hiint(x) < 0; }
+
+// MODE 0: whole tree, ending with the root sum; MODE 1: parts side by side, each
+// storing its root partial in its slot of the part rows (as k_prune_part)
+template <typename real, int R, int LV, int MODE>
+__global__ __launch_bounds__(64 * R) void k_prune_tab(
+    const int4* __restrict__ prog, const int32_t* __restrict__ meta, const int32_t* __restrict__ n_rows,
+    int n_progs, const int32_t* __restrict__ fifo, const uint64_t* __restrict__ tips, int64_t stride,
+    int64_t n_pat, int64_t pitch, const real* __restrict__ Pm, const real* __restrict__ tab,
+    const int32_t* __restrict__ etab, const double* __restrict__ pi, const double* __restrict__ probs,
+    const uint32_t* __restrict__ weights, double* __restrict__ site_lnl, double* __restrict__ wave_sums,
+    real* __restrict__ xt, int32_t* __restrict__ xte, int N, int stack_depth, int tip_off) {
+  extern __shared__ unsigned char lds_raw[];
+  const int64_t nb = pitch / 64;
+  const int64_t t = xcd_tile(blockIdx.x);
+  if (t >= nb * n_progs) return;  // padding of the grid (whole block)
+  const int y = (int)(t / nb);
+  const int64_t tile = t - (int64_t)y * nb;
+  const int n_ops = meta[n_progs + y], nr = n_rows[y];
+  const int2* ids = reinterpret_cast<const int2*>(fifo + meta[2 * n_progs + y]);  // pairs: 8-byte aligned
+  unsigned char* codes = lds_raw + tip_off;  // [nr + 2][64]
+  {
+    const uint32_t* t32 = reinterpret_cast<const uint32_t*>(tips);
+    const int64_t last = 2 * ((n_pat + 15) / 16) - 1;  // patterns past the row read any code
+    auto bytes = [](uint32_t x) {                       // 4 nibbles -> 4 bytes
+      x = (x | (x << 8)) & 0x00ff00ffu;
+      return (x | (x << 4)) & 0x0f0f0f0fu;
+    };
+    for (int i = threadIdx.x; i < nr * 8; i += 64 * R) {  // 8 patterns each
+      const int2 id = ids[i >> 3];
+      const int64_t c0 = tile * 8 + (i & 7), col = c0 < last ? c0 : last;
+      const uint32_t a = t32[(int64_t)id.x * (2 * stride) + col];
+      const uint32_t b = id.y >= 0 ? t32[(int64_t)id.y * (2 * stride) + col] : 0u;
+      reinterpret_cast<uint2*>(codes)[i] =
+          make_uint2(bytes(a & 0xffffu) | (bytes(b & 0xffffu) << 4), bytes(a >> 16) | (bytes(b >> 16) << 4));
+    }
+  }
+  __syncthreads();
+  // registers, stack and root sum of the plain walk; its tip stream is unused
+  DownState<real, R, 1, true, LV, MODE> st;
+  st.tid = threadIdx.x;
+  st.r0 = __builtin_amdgcn_readfirstlane(st.tid >> 6);
+  st.tile = tile;
+  st.p = tile * 64 + (st.tid & 63);
+  st.act = st.p < n_pat;
+  st.pc = st.act ? st.p : 0;
+  st.pitch = pitch;
+  st.N = N;
+  st.xt = xt;
+  st.xte = xte;
+  st.stk = reinterpret_cast<real*>(lds_raw);
+  st.stke = reinterpret_cast<int32_t*>(st.stk + (size_t)max(stack_depth - LV, 0) * 4 * st.BD);
+  const int r = st.r0, lane = st.tid & 63;
+  const unsigned char* cl = codes + lane;
+  const real* tabr = tab + (size_t)r * kTabCodes * 4;
+  const int32_t* etabr = etab + (size_t)r * kTabCodes;
+
+  // y = the table's product for the code pair c, its exponent into e
+  auto table = [&](int slot, uint32_t c, real* yv, int* e) {
+    typedef real real4 __attribute__((ext_vector_type(4)));
+    const real4 v = *reinterpret_cast<const real4*>(tabr + (size_t)slot * (R * kTabCodes * 4) + c * 4);
+    *e = 0;
+    if (sign_set(v[0])) *e = etabr[(size_t)slot * (R * kTabCodes) + c];
+    yv[0] = fabs(v[0]);
+    yv[1] = v[1];
+    yv[2] = v[2];
+    yv[3] = v[3];
+  };
+  // codes of an entry's operands, read an entry ahead (an operand that is no leaf
+  // or table entry reads some row: one past the last is padding)
+  auto read = [&](int w, uint32_t* c) {
+    const int row = w >> 8;
+    const int sa = w & 3;
+    c[0] = cl[row * 64];
+    c[1] = cl[(row + (sa == SRC_LEAF || sa == SRC_EXT ? 1 : 0)) * 64];
+  };
+  uint32_t cn[2];
+  read(prog[meta[y]].w, cn);
+  for_each_entry_ahead(prog + meta[y], n_ops, [&](int, const int4 op, const int4 on) {
+    const int fl = op.w, sa = fl & 3, sb = (fl >> 2) & 3;
+    const uint32_t ca = cn[0], cb = cn[1];
+    read(on.w, cn);
+    real PA[16], PB[16];
+    load_mat<real, R>(Pm + ((size_t)op.y * R + r) * 16, PA);
+    load_mat<real, R>(Pm + ((size_t)op.z * R + r) * 16, PB);
+    st.spill_if(fl);
+    real xa[4], xb[4];
+    int ea, eb;
+    if (sa == SRC_EXT) {
+      table(op.x & 0xffff, ca, xa, &ea);
+    } else if (sa == SRC_LEAF) {
+      real x[4];
+      tipvec(ca, x);
+      matvec4(PA, x, xa);
+      ea = 0;
+    } else {
+      st.product_a(sa, 0, 0, reinterpret_cast<const real(*)[16]>(&PA), reinterpret_cast<real(*)[4]>(&xa), &ea);
+    }
+    if (sb == SRC_EXT) {
+      table((uint32_t)op.x >> 16, cb, xb, &eb);
+    } else if (sb == SRC_LEAF) {
+      real x[4];
+      tipvec(cb, x);
+      matvec4(PB, x, xb);
+      eb = 0;
+    } else {
+      matvec4(PB, st.acc[0], xb);
+      eb = st.acc_e[0];
+    }
+    st.combine(0, reinterpret_cast<const real(*)[4]>(&xa), reinterpret_cast<const real(*)[4]>(&xb), &ea, &eb);
+  });
+  if constexpr (MODE == 1)
+    st.ext_store(y);
+  else
+    down_root(st, lds_raw, pi, probs, weights, site_lnl, wave_sums);
+}
+
 // Many candidate topologies over the same tips and weights (fused form):
 // blockIdx.y selects candidate c, whose program, leaf order, P matrices and
 // per-wave sums sit at fixed strides.
@@ -2370,6 +2534,9 @@ struct Plan {
   bool split = false;
   int n_parts = 0;
   size_t off_xt = 0, off_xte = 0;
+  // fused pass with the cherries' products from a table
+  bool tab = false;
+  size_t off_tab_y = 0, off_tab_e = 0;
 };
 
 constexpr size_t kLdsMax = 64 * 1024;
@@ -2402,6 +2569,25 @@ int fit_block(int want, F lds_of, int min_bs = 64) {
 bool split_env() {
   const char* s = getenv("PHY_PRUNE_SPLIT");
   return !(s && s[0] == '0' && s[1] == 0);
+}
+
+// LDS of the table form: the stack (and the root exchange), then the codes of a
+// tile (64 bytes an operand)
+size_t tab_tip_off(int R, size_t esz, int depth, int lv) { return (down_lds(R, esz, true, depth, lv) + 15) / 16 * 16; }
+size_t tab_lds(int R, size_t esz, const TabProg& tp, int lv) {
+  return tab_tip_off(R, esz, tp.sp.depth, lv) + (size_t)(tp.max_rows + 2) * 64;
+}
+
+// The table form pays for its table kernel (one launch, ~4 us) where the walk is
+// long or wide: plain and table form in us, FP32 at R = 4, 32 taxa x 5,000
+// patterns 23.2 / 24.3, 64 x 20,000 39.3 / 39.2, 32 x 50,000 28.8 / 25.6, 200 x
+// 2,000 106 / 97, 512 x 4,000 102 / 99, 200 x 100,000 191 / 142.
+// PHY_PRUNE_TAB=0|1 overrides the size rule.
+bool use_tables(const phy_topo* t, int R, size_t esz, int64_t n_pat) {
+  if (!t->tab.n_progs || !t->tab.d_cherry || t->tab.cherry.empty() || tab_lds(R, esz, t->tab, 0) > kLdsMax) return false;
+  const char* s = getenv("PHY_PRUNE_TAB");
+  if (s && (s[0] == '0' || s[0] == '1') && s[1] == 0) return s[0] == '1';
+  return t->n_leaves >= 128 || n_pat >= 32768;
 }
 
 Plan make_plan(const phy_topo* t, const phy_model* m, int64_t n_pat, int32_t form, int32_t derivs,
@@ -2454,6 +2640,13 @@ Plan make_plan(const phy_topo* t, const phy_model* m, int64_t n_pat, int32_t for
     pl.off_xt = o; o = align256(o + (size_t)pl.n_parts * R * K * pl.pitch * pl.esz);
     pl.off_xte = o; o = align256(o + (size_t)pl.n_parts * R * pl.pitch * 4);
   }
+  // the split decision stands; without parts the table form runs whole
+  pl.tab = allow_split && pl.fused && pl.rpw == 1 && (pl.split || t->pparts.empty()) && use_tables(t, R, esz, n_pat);
+  if (pl.tab) {
+    const size_t ent = t->tab.cherry.size() / 4 * R * kTabCodes;
+    pl.off_tab_y = o; o = align256(o + ent * 4 * esz);
+    pl.off_tab_e = o; o = align256(o + ent * 4);
+  }
   pl.off_bsum = o; o = align256(o + (size_t)pl.n_waves * 8);
   if (derivs) {
     pl.off_wsum = o; o = align256(o + (size_t)pl.n_dwaves * M * 2 * 8);
@@ -2498,6 +2691,26 @@ int register_levels(int depth, int bs) {
   return best;
 }
 
+// Register levels of the table form's stack, chosen as register_levels does.
+template <typename real, int R, int MODE>
+int tab_register_levels(const TabProg& tp) {
+  const int depth = tp.sp.depth;
+  const char* s = getenv("PHY_PRUNE_REG");
+  if (s && s[0] >= '0' && s[0] <= '2' && s[1] == 0) return std::min(s[0] - '0', depth);
+  const void* kern[3] = {reinterpret_cast<const void*>(&k_prune_tab<real, R, 0, MODE>),
+                         reinterpret_cast<const void*>(&k_prune_tab<real, R, 1, MODE>),
+                         reinterpret_cast<const void*>(&k_prune_tab<real, R, 2, MODE>)};
+  int best = 0, best_nb = -1;
+  for (int lv = 0; lv <= std::min(2, depth); ++lv) {
+    int nb = 0;
+    const size_t lds = tab_lds(R, sizeof(real), tp, lv);
+    if (lds > kLdsMax || hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kern[lv], 64 * R, lds) != hipSuccess)
+      continue;
+    if (nb > best_nb) best = lv, best_nb = nb;
+  }
+  return best;
+}
+
 template <typename real, int R>
 int launch_tree(phy_ctx* ctx, const phy_topo* t, const phy_model* m, bool fused, bool derivs,
                 int64_t n_pat, const uint64_t* tips, int64_t stride, const uint32_t* weights,
@@ -2527,9 +2740,29 @@ int launch_tree(phy_ctx* ctx, const phy_topo* t, const phy_model* m, bool fused,
   };
   constexpr int G2 = (R % 2 == 0 && sizeof(real) == 4) ? 2 : 1;
   const int lv = ((fused || pl.lds_stack) && pl.rpw != 2) ? register_levels<real, R>(t->down_depth, pl.bs) : 0;
+  if (pl.tab) {
+    hipLaunchKernelGGL((k_cherry_tab<real, R>), dim3((unsigned)(t->tab.cherry.size() / 4 * R)), dim3(kTabCodes), 0,
+                       ctx->stream, t->tab.d_cherry, P, reinterpret_cast<real*>(work + pl.off_tab_y),
+                       reinterpret_cast<int32_t*>(work + pl.off_tab_e));
+    PHY_LAUNCHED(ctx);
+  }
+  auto tables = [&](auto kern, int lv, real* xt, int32_t* xte) {
+    const TabProg& tp = t->tab;
+    const size_t lds = tab_lds(R, sizeof(real), tp, lv);
+    hipLaunchKernelGGL(kern, dim3((unsigned)((pl.n_blocks * tp.n_progs + 31) / 32 * 32)), dim3(64 * R), lds,
+                       ctx->stream, tp.sp.d_prog, tp.sp.d_meta, tp.d_rows, tp.n_progs, tp.sp.d_fifo, tips, stride,
+                       n_pat, pl.pitch, P, reinterpret_cast<const real*>(work + pl.off_tab_y),
+                       reinterpret_cast<const int32_t*>(work + pl.off_tab_e), d_pi, d_probs, weights, site_lnl, bsum,
+                       xt, xte, N, tp.sp.depth, (int)tab_tip_off(R, sizeof(real), tp.sp.depth, lv));
+  };
   {
     KernelSpan span(ctx, "prune_down");
-    if (pl.split) {
+    if (pl.tab && !pl.split) {
+      const int lvt = tab_register_levels<real, R, 0>(t->tab);
+      if (lvt == 2) tables(k_prune_tab<real, R, 2, 0>, 2, nullptr, nullptr);
+      else if (lvt == 1) tables(k_prune_tab<real, R, 1, 0>, 1, nullptr, nullptr);
+      else tables(k_prune_tab<real, R, 0, 0>, 0, nullptr, nullptr);
+    } else if (pl.split) {
       const SplitProg& sd = t->psplit;
       const int np = pl.n_parts;
       real* xt = fused ? reinterpret_cast<real*>(work + pl.off_xt) : nullptr;
@@ -2542,7 +2775,12 @@ int launch_tree(phy_ctx* ctx, const phy_topo* t, const phy_model* m, bool fused,
                            sd.d_prog, sd.d_meta, np, sd.d_fifo, tips, stride, n_pat, pl.pitch, P, xt, xte,
                            part, ex, N, sd.depth);
       };
-      if (fused) {
+      if (pl.tab) {
+        const int lvt = tab_register_levels<real, R, 1>(t->tab);
+        if (lvt == 2) tables(k_prune_tab<real, R, 2, 1>, 2, xt, xte);
+        else if (lvt == 1) tables(k_prune_tab<real, R, 1, 1>, 1, xt, xte);
+        else tables(k_prune_tab<real, R, 0, 1>, 0, xt, xte);
+      } else if (fused) {
         if (lvp == 2)
           parts(k_prune_part<real, R, 2>);
         else if (lvp == 1)

@@ -404,3 +404,32 @@ def test_stored_form_stack_in_lds_matches_hbm_stack(ctx, rng, monkeypatch, R, sp
             pb, eb = b["ev"].partial(v)
             assert torch.equal(pa[:, :P].cpu(), pb[:, :P].cpu())
             assert torch.equal(ea[:, :P].cpu(), eb[:, :P].cpu())
+
+
+@pytest.mark.parametrize("R", [1, 2, 4, 8])
+@pytest.mark.parametrize("N,P", [(16, 1), (17, 65), (100, 300), (255, 8192), (600, 777), (1100, 63)])
+def test_cherry_tables_are_bit_identical(ctx, rng, monkeypatch, R, N, P):
+    # the fused pass with its cherries' products from a table, whole and split,
+    # against the plain walk: the same operations in the same order, ambiguous
+    # and missing tips, branches short enough that cherries are rescaled, and
+    # identity branches (below 1e-10) that leave all-zero vectors
+    _say(f"prune tables R={R} N={N} P={P}")
+    ch, root = random_tree(rng, N)
+    bl = rng.exponential(0.1, 2 * N - 1) + 1e-3
+    bl[rng.random(2 * N - 1) < 0.3] = 1e-9
+    bl[:N][rng.random(N) < 0.1] = 1e-12
+    bl[root] = 0.0
+    model = _model(rng, R)
+    tips = _tips(rng, N, P)
+    w = rng.integers(1, 6, P).astype(np.uint32)
+    for form in (F32 | FUSED, F64 | FUSED):
+        got = {}
+        for reg in ("0", "1", "2"):
+            monkeypatch.setenv("PHY_PRUNE_REG", reg)
+            for tab in ("0", "1"):
+                monkeypatch.setenv("PHY_PRUNE_TAB", tab)
+                got[reg, tab] = _run(ctx, N, ch, root, bl, model, tips, w, form, False)
+        a = got["0", "0"]
+        for b in got.values():
+            assert np.array_equal(np.float64(a["lnl"]), np.float64(b["lnl"]), equal_nan=True), form
+            assert np.array_equal(a["site"], b["site"], equal_nan=True)
