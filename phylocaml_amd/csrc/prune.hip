@@ -1648,7 +1648,12 @@ __global__ __launch_bounds__(256) void k_spr_insert(
 // entry in LDS -- exponents aligned over the non-zero terms, the FP64 rate
 // sum -- where wave 0 finishes target a and wave 1 target b (wave 0 both
 // when R = 1); double-buffered by entry parity, one barrier per entry.
-// wsum[(k * M + c) * n_blk + block]: per target and block of 64 patterns.
+// wsum[(k * M + c) * n_blk + block]: per target and block of 64 patterns.  Bound
+// by VALU issue: leaving the messages unscaled and exchanging the terms in the
+// working precision took 96 taxa x 10,007 patterns FP32 from 8.1 to 7.0 ms a round.
+// (Reading the full-branch matrices again after the barrier instead of keeping
+// them frees FP64's spilled SGPRs but costs more: 13.9 against 12.8 ms, FP32 7.8
+// against 7.0.)
 template <typename real, int R>
 __global__ __launch_bounds__(64 * R) void k_spr_insert_w(
     const int4* __restrict__ prog, int64_t prog_stride, const int32_t* __restrict__ meta,
@@ -1670,7 +1675,7 @@ __global__ __launch_bounds__(64 * R) void k_spr_insert_w(
   const int64_t pc = act ? p : 0;
   real* stk = reinterpret_cast<real*>(lds_raw);                                  // [depth][4][BD]
   int32_t* stke = reinterpret_cast<int32_t*>(stk + (size_t)up_depth * 4 * BD);  // [depth][BD]
-  double* xv = reinterpret_cast<double*>(stke + (size_t)up_depth * BD);         // [2][2][R][64]
+  real* xv = reinterpret_cast<real*>(stke + (size_t)up_depth * BD);              // [2][2][R][64]
   int32_t* xe = reinterpret_cast<int32_t*>(xv + 2 * 2 * R * 64);                // [2][2][R][64]
   const int32_t* rf = ref + (size_t)k * M;
   const int x = mk[2], s = mk[3];
@@ -1781,29 +1786,29 @@ __global__ __launch_bounds__(64 * R) void k_spr_insert_w(
     // exchange; wave 0 finishes target a, wave 1 (wave 0 when R = 1) b
     {
       const int buf = i & 1;
-      double* xb0 = xv + (size_t)buf * 2 * R * 64;
+      real* xb0 = xv + (size_t)buf * 2 * R * 64;
       int32_t* eb0 = xe + (size_t)buf * 2 * R * 64;
-      xb0[r * 64 + lane] = (double)sa;
+      xb0[r * 64 + lane] = sa;
       eb0[r * 64 + lane] = eAa + Xc[0] + eX;
-      xb0[(R + r) * 64 + lane] = (double)sb;
+      xb0[(R + r) * 64 + lane] = sb;
       eb0[(R + r) * 64 + lane] = eAb + Xc[1] + eX;
       __syncthreads();
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
         if (r != (R == 1 ? 0 : q)) continue;
-        const double* sq = xb0 + (size_t)q * R * 64;
+        const real* sq = xb0 + (size_t)q * R * 64;
         const int32_t* eq = eb0 + (size_t)q * R * 64;
         int m = kNoExp;
 #pragma unroll
         for (int rr = 0; rr < R; ++rr)
-          if (sq[rr * 64 + lane] != 0.0) m = max(m, eq[rr * 64 + lane]);
+          if (sq[rr * 64 + lane] != (real)0) m = max(m, eq[rr * 64 + lane]);
         // the class sum and its log in the working precision (single: the
         // per-pattern term to ~1e-7, far inside the path's 1e-6 on lnL);
         // the exponent offset and the weighted sums in FP64
         real L = (real)0;
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) {
-          const real v = (real)sq[rr * 64 + lane];
+          const real v = sq[rr * 64 + lane];
           if (v != (real)0) L += (real)probs[rr] * ldexp(v, eq[rr * 64 + lane] - m);
         }
         const double v = act ? (double)weights[p] * ((double)log(L) + (double)m * 0.6931471805599453) : 0.0;
@@ -1811,16 +1816,15 @@ __global__ __launch_bounds__(64 * R) void k_spr_insert_w(
         if (lane == 0) ws[(size_t)(q ? b : a) * n_blk + blockIdx.x] = S;
       }
     }
-    // messages to internal children: M_c = P_c^T A_c
+    // messages to internal children: M_c = P_c^T A_c, not rescaled (the rows of
+    // P sum to 1, so max M_c >= max A_c / 4; the next A is rescaled)
     real Ma[4], Mb[4];
     int eMa = eAa, eMb = eAb;
     if (!(fl & (UP_A_LEAF | UP_A_CUT))) {
       vecmat4(PA, Aa, Ma);
-      rescale4(Ma, &eMa);
     }
     if (!(fl & (UP_B_LEAF | UP_B_CUT))) {
       vecmat4(PB, Ab, Mb);
-      rescale4(Mb, &eMb);
     }
     if (fl & UP_PUSH) {
       const bool cb = fl & UP_CONT_B;
@@ -2055,7 +2059,7 @@ __global__ __launch_bounds__(64 * R) void k_tbr_insert_w(
   const int64_t pc = act ? p : 0;
   real* stk = reinterpret_cast<real*>(lds_raw);                                  // [depth][4][BD]
   int32_t* stke = reinterpret_cast<int32_t*>(stk + (size_t)up_depth * 4 * BD);  // [depth][BD]
-  double* xvl = reinterpret_cast<double*>(stke + (size_t)up_depth * BD);        // [2][chunk][R][64]
+  real* xvl = reinterpret_cast<real*>(stke + (size_t)up_depth * BD);            // [2][chunk][R][64]
   int32_t* xel = reinterpret_cast<int32_t*>(xvl + 2 * kTbrChunk * R * 64);      // [2][chunk][R][64]
   const int32_t* rf = ref + (size_t)k * M;
   const uint32_t* tm = tmask + (size_t)k * (M + 1);
@@ -2086,23 +2090,23 @@ __global__ __launch_bounds__(64 * R) void k_tbr_insert_w(
 #pragma unroll
           for (int i = 0; i < 4; ++i) sv = fma(q[i], xs[(size_t)i * pitch], sv);
           const int slot = ((buf * kTbrChunk + j) * R + r) * 64 + lane;
-          xvl[slot] = (double)sv;
+          xvl[slot] = sv;
           xel[slot] = eq + xe[((size_t)xr * R + r) * pitch + pc];
           ++n;
         }
       }
       __syncthreads();
       for (int j = r; j < n; j += R) {
-        const double* sq = xvl + (buf * kTbrChunk + j) * R * 64;
+        const real* sq = xvl + (buf * kTbrChunk + j) * R * 64;
         const int32_t* eqq = xel + (buf * kTbrChunk + j) * R * 64;
         int m = kNoExp;
 #pragma unroll
         for (int rr = 0; rr < R; ++rr)
-          if (sq[rr * 64 + lane] != 0.0) m = max(m, eqq[rr * 64 + lane]);
+          if (sq[rr * 64 + lane] != (real)0) m = max(m, eqq[rr * 64 + lane]);
         real L = (real)0;
 #pragma unroll
         for (int rr = 0; rr < R; ++rr) {
-          const real v = (real)sq[rr * 64 + lane];
+          const real v = sq[rr * 64 + lane];
           if (v != (real)0) L += (real)probs[rr] * ldexp(v, eqq[rr * 64 + lane] - m);
         }
         const double v = act ? (double)weights[p] * ((double)log(L) + (double)m * 0.6931471805599453) : 0.0;
@@ -2235,16 +2239,15 @@ __global__ __launch_bounds__(64 * R) void k_tbr_insert_w(
         pairs(tm[M], rb[M], q, eq);
       }
     }
-    // messages to internal children: M_c = P_c^T A_c
+    // messages to internal children: M_c = P_c^T A_c, not rescaled (as in
+    // k_spr_insert_w)
     real Ma[4], Mb[4];
     int eMa = eAa, eMb = eAb;
     if (!(fl & (UP_A_LEAF | UP_A_CUT))) {
       vecmat4(PA, Aa, Ma);
-      rescale4(Ma, &eMa);
     }
     if (!(fl & (UP_B_LEAF | UP_B_CUT))) {
       vecmat4(PB, Ab, Mb);
-      rescale4(Mb, &eMb);
     }
     if (fl & UP_PUSH) {
       const bool cb = fl & UP_CONT_B;
@@ -2272,7 +2275,7 @@ __global__ __launch_bounds__(64 * R) void k_tbr_insert_w(
 
 // LDS of k_tbr_insert_w: the message stack and the double-buffered exchange
 size_t tbr_insert_lds(int R, size_t esz, int depth) {
-  return (size_t)std::max(depth, 1) * 64 * R * (4 * esz + 4) + (size_t)2 * kTbrChunk * R * 64 * 12;
+  return (size_t)std::max(depth, 1) * 64 * R * (4 * esz + 4) + (size_t)2 * kTbrChunk * R * 64 * (esz + 4);
 }
 // LDS of k_tbr_reroot: the outside-vector stack
 size_t tbr_reroot_lds(int R, size_t esz, int depth) {
@@ -2281,7 +2284,7 @@ size_t tbr_reroot_lds(int R, size_t esz, int depth) {
 
 // LDS of k_spr_insert_w: the message stack and the double-buffered exchange
 size_t insert_w_lds(int R, size_t esz, int depth) {
-  return (size_t)std::max(depth, 1) * 64 * R * (4 * esz + 4) + (size_t)2 * 2 * R * 64 * 12;
+  return (size_t)std::max(depth, 1) * 64 * R * (4 * esz + 4) + (size_t)2 * 2 * R * 64 * (esz + 4);
 }
 
 // out[idx[j]] = compensated sum of row rows[j] of x (n values per row); one
@@ -3358,6 +3361,21 @@ IncrPlan incr_plan(const IncrTree& t, int R, int64_t n_pat, int32_t form, int32_
   return pl;
 }
 
+// Pruned subtrees per launch: the caller's s_batch, or more where few patterns
+// would leave the chip idle between the launches of a round (about 8,192 blocks,
+// eight rounds of resident ones, while the rows of a batch stay within 2 GiB).
+// s_batch = 16, whole rounds: 96 taxa x 10,007 patterns FP32 9.12 ms so and 8.13
+// with 53 subtrees a launch; x 1,000 patterns 3.3 and 1.6; TBR 64 x 5,003 FP64
+// 2.81 and 2.38.
+int incr_batch(const IncrTree& t, int R, int64_t n_pat, int32_t form, int32_t s_batch) {
+  const int64_t blocks = (n_pat + 63) / 64, pitch = ((n_pat + 255) / 256) * 256;
+  const int64_t esz = (form & PHY_F32) ? 4 : 8;
+  const int64_t slot = (int64_t)(std::max(t.lmax, 1) + 12) * R * (4 * esz + 4) * pitch +  // pool and reroot rows
+                       (int64_t)t.M * blocks * R * 8;                                       // sums
+  const int64_t want = std::min({(int64_t)t.M, (8192 + blocks - 1) / blocks, ((int64_t)2 << 30) / slot});
+  return (int)std::max<int64_t>(s_batch, want);
+}
+
 // Per pruned subtree: the pre-order program of the pruned tree on the
 // original node ids, pool rows, repair ops, and x and p (the merged branch
 // t_x + t_p; x = -1 when p is the root).
@@ -3912,11 +3930,12 @@ int tbr_group(const IncrTree& t, int64_t n_moves, const int32_t* moves, int S, T
 
 int tbr_plan_create(phy_ctx* ctx, const phy_model* m, int32_t form, int64_t n_pat, int32_t N,
                     const int32_t* children, int32_t root, int64_t n_moves, const int32_t* moves, int32_t s_batch,
-                    phy_spr_plan** out) {
+                    phy_spr_plan** out, bool grow = true) {
   std::unique_ptr<phy_spr_plan> sp(new phy_spr_plan());
   if (!sp->t.load(N, children, root)) return set_err(ctx, PHY_EINVAL, "tbr incremental: not a rooted binary tree");
   const IncrTree& t = sp->t;
-  const int M = t.M, S = s_batch, R = m->R;
+  const int M = t.M, R = m->R;
+  int S = grow ? incr_batch(t, R, n_pat, form, s_batch) : s_batch;
   sp->tbr = true;
   sp->form = form;
   sp->R = R;
@@ -3924,7 +3943,8 @@ int tbr_plan_create(phy_ctx* ctx, const phy_model* m, int32_t form, int64_t n_pa
   sp->n_moves = n_moves;
   TbrGroups grp;
   int64_t bad = -1;
-  const int gr = tbr_group(t, n_moves, moves, S, &grp, &bad);
+  int gr = tbr_group(t, n_moves, moves, S, &grp, &bad);
+  if (gr == 2 && S != s_batch) gr = tbr_group(t, n_moves, moves, S = s_batch, &grp, &bad);
   if (gr == 1) return set_err(ctx, PHY_EINVAL, "tbr incremental: invalid move " + std::to_string(bad));
   if (gr == 2) return set_err(ctx, PHY_ERANGE, "tbr incremental: too many pairs in a batch");
   const int n_sub = sp->n_sub = grp.n_sub;
@@ -4080,7 +4100,7 @@ int phy_lk_spr_incr_work_size(int32_t N, const int32_t* children, int32_t root, 
   try {
     IncrTree t;
     if (!t.load(N, children, root)) return PHY_EINVAL;
-    *bytes = incr_plan(t, m->R, n_pat, form, s_batch).total;
+    *bytes = incr_plan(t, m->R, n_pat, form, incr_batch(t, m->R, n_pat, form, s_batch)).total;
     return PHY_OK;
   } catch (...) {
     return PHY_ENOMEM;
@@ -4097,7 +4117,10 @@ int phy_spr_plan_create(phy_ctx* ctx, const phy_model* m, int32_t form, int64_t 
   int rc = check_plan_model(ctx, m);
   if (rc) return rc;
   try {
-    return plan_create(ctx, m, form, n_pat, N, children, root, n_moves, moves, s_batch, out);
+    IncrTree t;
+    if (!t.load(N, children, root)) return set_err(ctx, PHY_EINVAL, "spr incremental: not a rooted binary tree");
+    return plan_create(ctx, m, form, n_pat, N, children, root, n_moves, moves,
+                       incr_batch(t, m->R, n_pat, form, s_batch), out);
   } catch (...) {
     return set_err(ctx, PHY_ENOMEM, "spr plan: host allocation or thread start failed");
   }
@@ -4136,10 +4159,13 @@ int phy_lk_spr_scores_incr(phy_ctx* ctx, const phy_model* m, int32_t form, int64
   try {
     IncrTree t;
     if (!t.load(N, children, root)) return set_err(ctx, PHY_EINVAL, "spr incremental: not a rooted binary tree");
-    const IncrPlan lay = incr_plan(t, m->R, n_pat, form, s_batch);
+    // a workspace sized for s_batch itself is enough
+    int32_t S = incr_batch(t, m->R, n_pat, form, s_batch);
+    if (work_bytes < incr_plan(t, m->R, n_pat, form, S).total) S = s_batch;
+    const IncrPlan lay = incr_plan(t, m->R, n_pat, form, S);
     if (work_bytes < lay.total) return set_err(ctx, PHY_EINVAL, "spr incremental: workspace too small");
     phy_spr_plan* sp = nullptr;
-    rc = plan_create(ctx, m, form, n_pat, N, children, root, n_moves, moves, s_batch, &sp);
+    rc = plan_create(ctx, m, form, n_pat, N, children, root, n_moves, moves, S, &sp);
     if (rc) return rc;
     std::unique_ptr<phy_spr_plan> hold(sp);
     char* work = static_cast<char*>(d_work);
@@ -4166,9 +4192,11 @@ int phy_lk_tbr_incr_work_size(int32_t N, const int32_t* children, int32_t root, 
     if (!t.load(N, children, root)) return PHY_EINVAL;
     TbrGroups g;
     int64_t bad = -1;
-    const int gr = tbr_group(t, n_moves, moves, s_batch, &g, &bad);
+    int32_t S = incr_batch(t, m->R, n_pat, form, s_batch);
+    int gr = tbr_group(t, n_moves, moves, S, &g, &bad);
+    if (gr == 2 && S != s_batch) gr = tbr_group(t, n_moves, moves, S = s_batch, &g, &bad);
     if (gr) return gr == 1 ? PHY_EINVAL : PHY_ERANGE;
-    *bytes = incr_plan(t, m->R, n_pat, form, s_batch, g.n_sub, g.max_xrows, g.max_pairs).total;
+    *bytes = incr_plan(t, m->R, n_pat, form, S, g.n_sub, g.max_xrows, g.max_pairs).total;
     return PHY_OK;
   } catch (...) {
     return PHY_ENOMEM;
@@ -4206,6 +4234,11 @@ int phy_lk_tbr_scores_incr(phy_ctx* ctx, const phy_model* m, int32_t form, int64
     rc = tbr_plan_create(ctx, m, form, n_pat, N, children, root, n_moves, moves, s_batch, &sp);
     if (rc) return rc;
     std::unique_ptr<phy_spr_plan> hold(sp);
+    if (work_bytes < sp->pl.total) {  // a workspace sized for s_batch itself is enough
+      rc = tbr_plan_create(ctx, m, form, n_pat, N, children, root, n_moves, moves, s_batch, &sp, false);
+      if (rc) return rc;
+      hold.reset(sp);
+    }
     if (work_bytes < sp->pl.total) return set_err(ctx, PHY_EINVAL, "tbr incremental: workspace too small");
     char* work = static_cast<char*>(d_work);
     double* dbl = reinterpret_cast<double*>(work + sp->pl.off_blh);

@@ -269,3 +269,52 @@ def test_plan_runs_equal_the_one_shot_scores_and_replay_from_a_graph():
                       flush=True)
                 assert np.array_equal(got, want), (form, rep)
             plan.close()
+
+
+@pytest.mark.parametrize("form", [F32, F64])
+@pytest.mark.parametrize("kind", ["spr", "tbr"])
+def test_batch_size_does_not_change_a_score(ctx, form, kind):
+    # a launch takes more pruned subtrees than s_batch where the patterns are
+    # few; a workspace that only holds s_batch at a time is enough, and every
+    # score is the same bits either way
+    import ctypes as C
+
+    from phylocaml_amd import device as D, neighborhood as NB, spr, synth
+    from phylocaml_amd._lib import PhyError, lib, ptr
+
+    N, P = 30, 300
+    tree = synth.yule(N, 9, 0.1)
+    model = _model(9)
+    st, w = _data(tree, model, P, 9)
+    _, _, dm = _scorers(ctx, model, st, w, N, form)
+    tips, wd = D.to_device(synth.pack_dna(st)), D.to_device(w)
+    mv = spr.moves(N, tree.children, tree.root) if kind == "spr" else \
+        NB.tbr_moves(N, tree.children, tree.root, 3, 3)
+    ch = np.ascontiguousarray(tree.children, np.int32)
+    bl = np.ascontiguousarray(tree.blen, np.float64)
+    mv = np.ascontiguousarray(mv, np.int32)
+    nb = C.c_size_t()
+    if kind == "spr":
+        rc = lib.phy_lk_spr_incr_work_size(N, ptr(ch, C.c_int32), tree.root, dm.handle, P, form, 1,
+                                           C.byref(nb))
+    else:
+        rc = lib.phy_lk_tbr_incr_work_size(N, ptr(ch, C.c_int32), tree.root, dm.handle, P, form,
+                                           len(mv), ptr(mv, C.c_int32), 1, C.byref(nb))
+    assert rc == 0
+    fn = lib.phy_lk_spr_scores_incr if kind == "spr" else lib.phy_lk_tbr_scores_incr
+    work = torch.empty((nb.value,), dtype=torch.uint8, device="cuda")
+    got, refused = [], 0
+    for s_batch, size in ((1, nb.value), (1, nb.value // 2), (7, nb.value), (1, 4096)):
+        _say(f"{kind} batch {s_batch} form {form} workspace {size}")
+        out = torch.zeros((len(mv),), dtype=torch.float64, device="cuda")
+        try:
+            ctx.check(fn(ctx.handle, dm.handle, form, P, D.dptr(tips), D.words(P), D.dptr(wd), N,
+                         ptr(ch, C.c_int32), tree.root, ptr(bl, C.c_double), len(mv),
+                         ptr(mv, C.c_int32), s_batch, D.dptr(out), None, D.dptr(work), size), kind)
+        except PhyError as e:
+            assert e.code == 1
+            refused += 1
+            continue
+        got.append(out.cpu().numpy())
+    assert refused == 1 and len(got) == 3
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
