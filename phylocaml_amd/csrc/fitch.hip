@@ -578,37 +578,66 @@ __global__ __launch_bounds__(256) void k_fitch_up(const int4* __restrict__ prog,
   });
 }
 
-// Insertion costs of many (c, a, b) queries: block q sums, over the words of
-// the sites, w_s [P_c & med(F_a, F_b) = 0] with med the Fitch median.
+// Insertion costs of many (c, a, b) queries: sum over the sites of
+// w_s [P_c & med(F_a, F_b) = 0] with med the Fitch median.  A block takes a
+// chunk of words (one 16-site word a thread, whose weights it holds as bit
+// planes) through a run of queries, so that the weights are read once a run and
+// a word of P_c once for the neighbouring queries of one c; the waves' sums meet
+// in LDS.  Bound by the L2 reads of the F rows: 128 taxa, 20,011 weighted sites,
+// 61,976 queries take 190 us; one block per query over all words, with a
+// dependent weight load for each flagged site, took 522.
+constexpr int kMaxRun = 64;
+
 __global__ __launch_bounds__(256) void k_fitch_insert(const uint64_t* __restrict__ pre,
                                                       const uint64_t* __restrict__ fin,
                                                       int64_t stride, int64_t W, int64_t n_sites,
                                                       const uint32_t* __restrict__ wt,
-                                                      const int32_t* __restrict__ qs,
+                                                      const int32_t* __restrict__ qs, int64_t n_q, int run,
                                                       unsigned long long* __restrict__ cost) {
-  const int64_t q = blockIdx.x;
-  const int32_t c = qs[3 * q], a = qs[3 * q + 1], b = qs[3 * q + 2];
-  const uint64_t* pc = pre + (int64_t)c * stride;
-  const uint64_t* fa = fin + (int64_t)a * stride;
-  const uint64_t* fb = fin + (int64_t)b * stride;
-  uint64_t acc = 0;
-  for (int64_t w = threadIdx.x; w < W; w += blockDim.x) {
-    uint32_t t0, t1, elo, ehi;
-    const uint64_t m = fitch64(fa[w], fb[w], &t0, &t1);
-    (void)fitch64(m, pc[w], &elo, &ehi);
-    const uint64_t vm = valid_nibbles(w, n_sites);
-    elo &= (uint32_t)vm;
-    ehi &= (uint32_t)(vm >> 32);
-    acc += wt ? weigh(elo, ehi, wt, w) : (uint64_t)(__popc(elo) + __popc(ehi));
-  }
-  acc = wave_sum(acc);
-  __shared__ unsigned long long sh[4];
-  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
+  __shared__ unsigned long long sum[kMaxRun];
+  const int64_t q0 = (int64_t)blockIdx.x * run;
+  const int n = (int)(n_q - q0 < run ? n_q - q0 : run);
+  for (int k = threadIdx.x; k < n; k += blockDim.x) sum[k] = 0;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned long long t = 0;
-    for (int k = 0; k < (int)(blockDim.x >> 6); ++k) t += sh[k];
-    cost[q] = t;
+  const int32_t* qp = qs + 3 * q0;
+  for (int64_t w0 = (int64_t)blockIdx.y * blockDim.x; w0 < W; w0 += (int64_t)gridDim.y * blockDim.x) {
+    const int64_t w = w0 + threadIdx.x;
+    const bool act = w < W;
+    const int64_t wc = act ? w : 0;
+    WeightPlanes<2> planes;
+    if (wt) planes.load(wt, 2 * wc, n_sites, act);
+    const uint64_t vm = act ? valid_nibbles(w, n_sites) : 0ull;
+    int32_t last = -1;
+    uint64_t pc = 0;
+    uint64_t an = fin[(int64_t)qp[1] * stride + wc], bn = fin[(int64_t)qp[2] * stride + wc];
+    for (int k = 0; k < n; ++k) {
+      const int32_t c = qp[3 * k];  // the query is uniform
+      if (c != last) {
+        pc = pre[(int64_t)c * stride + wc];
+        last = c;
+      }
+      const uint64_t fa = an, fb = bn;
+      const int kn = k + 1 < n ? k + 1 : k;  // the next query's rows, a query ahead
+      an = fin[(int64_t)qp[3 * kn + 1] * stride + wc];
+      bn = fin[(int64_t)qp[3 * kn + 2] * stride + wc];
+      uint32_t t0, t1, e[2];
+      const uint64_t m = fitch64(fa, fb, &t0, &t1);
+      (void)fitch64(m, pc, &e[0], &e[1]);
+      e[0] &= (uint32_t)vm;
+      e[1] &= (uint32_t)(vm >> 32);
+      uint64_t v;
+      if (wt && planes.n > kPlanes) {  // wave-uniform
+        v = wave_sum(weigh(e[0], e[1], wt, w));
+      } else {
+        v = wave_sum32(wt ? planes.weigh(e) : (uint32_t)(__popc(e[0]) + __popc(e[1])));
+      }
+      if ((threadIdx.x & 63) == 0) atomicAdd(&sum[k], (unsigned long long)v);
+    }
+  }
+  __syncthreads();
+  for (int k = threadIdx.x; k < n; k += blockDim.x) {
+    if (gridDim.y == 1) cost[q0 + k] = sum[k];
+    else if (sum[k]) atomicAdd(&cost[q0 + k], sum[k]);
   }
 }
 
@@ -1019,8 +1048,17 @@ int phy_fitch_insertion_costs(phy_ctx* ctx, const uint64_t* pre, const uint64_t*
     return set_err(ctx, PHY_EINVAL, "insertion costs: bad argument");
   if (n_q == 0) return PHY_OK;
   if (n_q > 0x7fffffff) return set_err(ctx, PHY_ERANGE, "insertion costs: too many queries");
-  hipLaunchKernelGGL(k_fitch_insert, dim3((unsigned)n_q), dim3(256), 0, ctx->stream, pre, fin, stride, W,
-                     n_sites, wt, d_q, (unsigned long long*)d_costs);
+  if (W == 0) return phy_zero_u64(ctx, d_costs, n_q);
+  // one wave for each 64 words up to 4; runs of up to 64 queries, shorter where
+  // that would leave fewer than 2,048 blocks (8 a CU): a longer run reads its
+  // weights for more queries, but a CU without a block reads nothing
+  const int bs = (int)std::min<int64_t>(256, (W + 63) / 64 * 64);
+  const int64_t chunks = std::min<int64_t>((W + bs - 1) / bs, 0xffff);  // a block takes several beyond that
+  const int run = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxRun, n_q * chunks / 2048));
+  int rc;
+  if (chunks > 1 && (rc = phy_zero_u64(ctx, d_costs, n_q))) return rc;
+  hipLaunchKernelGGL(k_fitch_insert, dim3((unsigned)((n_q + run - 1) / run), (unsigned)chunks), dim3(bs), 0,
+                     ctx->stream, pre, fin, stride, W, n_sites, wt, d_q, n_q, run, (unsigned long long*)d_costs);
   PHY_LAUNCHED(ctx);
   return PHY_OK;
 }

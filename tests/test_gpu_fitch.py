@@ -210,3 +210,35 @@ def test_pass_shapes_and_node_costs(ctx, rng, N, S, weights):
     if weights == "heavy":
         w[S // 2] = 1 << 20
     _tree_case(ctx, N, ch, root, leaves, w)
+
+
+@pytest.mark.parametrize("S", [1, 1025, 4111, 70_003])
+@pytest.mark.parametrize("weights", ["unit", "small", "heavy"])
+def test_insertion_costs_match_oracle(ctx, rng, S, weights):
+    # one wave to several chunks of words a query, runs that share or change
+    # the inserted node, one query and more than a run, weights by bit planes
+    # or walked
+    from phylocaml_amd import device as D
+    from phylocaml_amd._lib import lib
+
+    rows = 9
+    sets = rng.integers(1, 16, (2, rows, S)).astype(np.uint8)
+    pre, fin = (D.to_device(D.pack_nibbles(x), ctx.device) for x in sets)
+    w = None if weights == "unit" else rng.integers(0, 256, S).astype(np.uint32)
+    if weights == "heavy":
+        w[S // 2] = 1 << 20
+    wd = None if w is None else D.to_device(w, ctx.device)
+    allq = np.stack([np.repeat(np.arange(rows), 81), np.tile(np.repeat(np.arange(rows), 9), rows),
+                     np.tile(np.arange(rows), 81)], 1).astype(np.int32)
+    pairs = {(a, b): O.fitch_median2(sets[1][a], sets[1][b])[0] for a in range(rows)
+             for b in range(rows)}
+    for n in (1, 65, len(allq)):
+        q = allq[:n]
+        _say(f"insertion costs S={S} {weights} n={n}")
+        dq = D.to_device(np.ascontiguousarray(q), ctx.device)
+        out = torch.full((n,), 7, dtype=torch.int64, device="cuda")
+        ctx.check(lib.phy_fitch_insertion_costs(ctx.handle, D.dptr(pre), D.dptr(fin), D.words(S), S,
+                                                D.dptr(wd), n, D.dptr(dq), D.dptr(out)), "insertion")
+        ww = np.ones(S, np.int64) if w is None else w.astype(np.int64)
+        want = [int(ww[(sets[0][c] & pairs[a, b]) == 0].sum()) for c, a, b in q.tolist()]
+        assert out.cpu().tolist() == want
