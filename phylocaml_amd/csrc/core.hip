@@ -417,8 +417,10 @@ int compile_tab(const phy_topo* t, const std::vector<int32_t>& tops, TabProg* ou
 }
 
 // Programs of the Fitch passes split under at most `want` cut nodes of at
-// least `min_leaves` leaves (no parts when fewer than two are found).
-int compile_fitch_split(const phy_topo* t, int want, int32_t min_leaves, FitchSplit* out) {
+// least `min_leaves` leaves (no parts when fewer than two are found).  With
+// `slots`, the top's down entries hold 1 + the part of A in bits 8-15 of the
+// flags and 1 + that of B in bits 16-23 where these are cut nodes.
+int compile_fitch_split(const phy_topo* t, int want, int32_t min_leaves, FitchSplit* out, bool slots = false) {
   const int32_t N = t->n_leaves, M = 2 * N - 1;
   const std::vector<int32_t>& ch = t->children;
   const Stop is_leaf = [N](int32_t v) { return v < N; };
@@ -450,6 +452,11 @@ int compile_fitch_split(const phy_topo* t, int want, int32_t min_leaves, FitchSp
     add(sd);
   }
   if (!compile_down(N, ch, t->root, stop_top, &pg, &ff, &d)) return 4;
+  if (slots) {
+    std::vector<int32_t> slot(M, 0);
+    for (size_t k = 0; k < cuts.size(); ++k) slot[cuts[k]] = (int32_t)k + 1;
+    for (size_t i = 0; i < pg.size(); i += 4) pg[i + 3] |= (slot[pg[i + 1]] << 8) | (slot[pg[i + 2]] << 16);
+  }
   add(sd);
   if (n_ops != N - 1) return 5;
   // up: the top first, then the parts (entered from the parent's final)
@@ -666,7 +673,7 @@ int phy_topo_create(phy_ctx* ctx, int32_t N, const int32_t* children, int32_t ro
   // shortest chain of two launches (PHY_FITCH_PARTS keeps to its one split)
   if (N >= 24 && !getenv("PHY_FITCH_PARTS")) {
     const int want = std::min(kMaxParts, (int)std::lround(std::sqrt((double)N)));
-    if (compile_fitch_split(t, want, std::max(3, N / want / 2), &t->fine)) {
+    if (compile_fitch_split(t, want, std::max(3, N / want / 2), &t->fine, true)) {
       delete t;
       return set_err(ctx, PHY_EINVAL, "topology: program compilation failed");
     }
