@@ -342,7 +342,7 @@ def bench_aa(torch, ctx, clock, n_trees, steps, cpu_baseline):
                         "frac": useful_tf / BF16_PEAK_TF, "executed_tflops": executed_tf,
                         "note": "6,400 useful BF16 MFMA flop per internal pattern.node "
                                 "(2 children x 4 rates x 20x20 MAC); 16,384 executed "
-                                "(states padded 20 -> 32 on both sides)"}}
+                                "(a child's 80 x 80 block matrix in 8 tiles of 16 x 32)"}}
     log(f"  aa: step {ms:.1f} ms, kernel {k_ms:.1f} ms ({tb.launches} launch(es)) for "
         f"{pn:.3e} pattern.nodes = {pn / (ms / 1e3):.3e}/s")
     if cpu_baseline:
@@ -786,10 +786,10 @@ def main():
     # then the top program; both grids are padded for the XCD-aware tile
     # order, and the traffic file keeps each kernel's largest launches
     grid = ((pr["P"] + 255) // 256) * 256 * 4
-    # (the fused pass's kernels: STORE = false; the stored form's end in true)
-    t_parts = measured_traffic("k_prune_part<float, 4,", suffix="false>")
-    t_top = measured_traffic("k_prune_down<float, 4, 1, true, 0, 2, false>")
-    traffic = None if t_parts is None or t_top is None else t_parts + t_top
+    # (the fused pass's top: STORE = false; the stored form's ends in true)
+    t_pass = [measured_traffic("k_cherry_tab<float, 4>"), measured_traffic("k_prune_tab<float, 4,"),
+              measured_traffic("k_prune_down<float, 4, 1, true, 0, 2, false>")]
+    traffic = None if None in t_pass else sum(t_pass)
     line = {
         "metric": "FP32-scaled vs FP64 pruning updates/s at rel ΔlnL≤1e-6; "
                   "Fitch site-node/s",
@@ -818,12 +818,14 @@ def main():
                      else traffic / (k_main / 1e3) / 1e9 / HBM_PEAK_GBS,
                      "note": "achieved = 272 flop per internal pattern.node x 511 nodes x "
                              "200,000 patterns / mean duration of the fused pass (HIP events "
-                             "around its two launches: k_prune_part, the tree's 4 parts "
-                             "side by side, then the top program k_prune_down<float, 4, 1, "
-                             "true, 0, 2>); packed FP32 is kept out of the build, so "
+                             "around its three launches: k_cherry_tab, the cherries' "
+                             "products, k_prune_tab, the tree's 4 parts side by side, then "
+                             "the top program k_prune_down<float, 4, 1, true, 0, 2>); the "
+                             "cherries' products come from a table per call, so fewer are "
+                             "executed; packed FP32 is kept out of the build, so "
                              "78.6 TFLOP/s is the reachable vector peak; traffic = HBM bytes "
                              "per pass from rocprofv3 FETCH_SIZE + WRITE_SIZE "
-                             "(copy-calibrated) of both kernels: interior partials stay "
+                             "(copy-calibrated) of the three kernels: interior partials stay "
                              "on chip, the parts' root partials go through HBM"},
         "cpu_baseline": cpu,
         "prune": {
