@@ -340,7 +340,7 @@ __global__ __launch_bounds__(64 * W) void k_mlp_fused(MlpArgs a) {
 #pragma unroll
       for (int k = 0; k < W; ++k) s += ys[k][16 * g + c];
       const float d = row < a.B ? (s + b3) - a.T[row] : 0.0f;
-      const float dy = d / (float)a.B;
+      const float dy = d / (float)a.B, dyb = (float)(__bf16)dy;
       if (w == 0 && q == 0) {
         loss += 0.5 * (double)d * (double)d / (double)a.B;
         gb3 += dy;
@@ -348,7 +348,7 @@ __global__ __launch_bounds__(64 * W) void k_mlp_fused(MlpArgs a) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const float zv = z2[g][v];
-        gw3[v] += gelu(zv) * dy;
+        gw3[v] += (float)(__bf16)gelu(zv) * dyb;  // BF16 operands, as the GEMM path's
         const float dz = dy * w3[v] * gelu_grad(zv);
         gb2[v] += dz;
         const __bf16 h = (__bf16)dz;

@@ -35,7 +35,7 @@ def _rounded(p, X, t, n_in, H):
     dy = d / len(t)
     dZ2 = np.outer(dy, w3) * MO.gelu_grad(Z2)
     dZ1 = (_bf(dZ2) @ W2.T) * MO.gelu_grad(Z1)
-    g = [X.T @ _bf(dZ1), dZ1.sum(0), H1.T @ _bf(dZ2), dZ2.sum(0), H2.T @ dy, dy.sum()]
+    g = [X.T @ _bf(dZ1), dZ1.sum(0), H1.T @ _bf(dZ2), dZ2.sum(0), _bf(H2).T @ _bf(dy), dy.sum()]
     return y, 0.5 * np.mean(d * d), g
 
 
@@ -59,9 +59,9 @@ def test_fused_pass_matches_rounded_oracle(ctx, n_in, H, B):
     t = rng.standard_normal(B).astype(np.float32)
     y, loss, g = _rounded(p, X, t, n_in, H)
     # FP32 sums put ~1e-3 of the BF16 roundings on the other side (2^-8 each):
-    # ~1.2e-4 of the norm a stage, four stages deep; the GEMM path also rounds
-    # H2 and dy (2^-9 each)
-    tol = 1e-3 if n_in <= 64 else 8e-3
+    # ~1.2e-4 of the norm a stage, four stages deep; the output layer's gradient
+    # is two stages deep, and unrounded H2 and dy (2^-9 each) would be ~1e-3 off
+    tol = 1e-3
     got = net.forward(D.to_device(X)).cpu().numpy()
     assert np.linalg.norm(got - y) <= tol * (np.linalg.norm(y) + 1e-3)
     for _ in range(2):  # the partial sums are rewritten by every call
@@ -70,5 +70,6 @@ def test_fused_pass_matches_rounded_oracle(ctx, n_in, H, B):
     o = 0
     for s, want in zip(sizes, g):
         want = np.ravel(want)
-        assert np.linalg.norm(gg[o:o + s] - want) <= tol * (np.linalg.norm(want) + 1e-6), s
+        rel = 4e-4 if o == n_in * H + H + H * H + H else tol
+        assert np.linalg.norm(gg[o:o + s] - want) <= rel * (np.linalg.norm(want) + 1e-6), (s, o)
         o += s
