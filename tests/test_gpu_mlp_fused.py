@@ -40,11 +40,12 @@ def _rounded(p, X, t, n_in, H):
 
 
 # a last row alone in its tile, a full tile, more tiles than blocks of the
-# backward (256) and of the forward (512); one and two feature chunks, rows
+# backward (256) and of the forward (768); one and two feature chunks, rows
 # readable 16 bytes at a time or not; a size that takes the GEMM path
 @pytest.mark.parametrize("n_in,H,B", [(32, 128, 1), (32, 128, 32), (5, 128, 33), (33, 128, 100),
                                       (64, 128, 257), (1, 64, 31), (32, 64, 4097), (63, 64, 65),
-                                      (32, 128, 8192 + 33), (32, 128, 16384 + 5), (65, 128, 40)])
+                                      (32, 128, 8192 + 33), (32, 128, 16384 + 5), (32, 128, 65536 + 5),
+                                      (32, 64, 65536 + 5), (65, 128, 40)])
 def test_fused_pass_matches_rounded_oracle(ctx, n_in, H, B):
     from phylocaml_amd import device as D, mlp
 
