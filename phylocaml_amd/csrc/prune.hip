@@ -729,9 +729,11 @@ __global__ __launch_bounds__(512) void k_prune_part(
 // pairs of every cherry and class (the same operations in the same order as the
 // walk, so the results are the same bits), and the walk reads it as an operand:
 // one 16-byte (FP32) gather instead of a program entry and a product, ~8 VALU
-// instructions instead of ~90.  Entry [slot][class][code_a | code_b << 4]; an
-// entry that was rescaled carries its sign bit on y[0] (the values themselves
-// are never negative) and its exponent in etab.
+// instructions instead of ~90.  Entry [slot][class][code_a | code_b << 4], its
+// exponent in etab; rescaled[slot][class] says whether any entry there has one
+// (only cherries of branches below ~1e-6 in FP32): the walk marks its entries
+// with that, 64 at a time, and reads etab under a uniform test.  (The values' own bits have no room for that mark: an
+// entry of P below ~1e-16 comes out of the eigen sums with either sign.)
 //
 // The walk stages the codes of its tile in LDS first, one byte per operand (a
 // leaf's code, or a cherry's pair) and pattern, shared by the R waves (each wave
@@ -743,11 +745,13 @@ __global__ __launch_bounds__(512) void k_prune_part(
 // twice the gathers, each ~36 L1 accesses, against 20 VALU instructions saved).
 // ---------------------------------------------------------------------------
 constexpr int kTabCodes = 256;
+constexpr int kTabResA = 32, kTabResB = 64;  // marks in an entry's flags: read the exponent of A, of B
 
 template <typename real, int R>
 __global__ __launch_bounds__(kTabCodes) void k_cherry_tab(const int4* __restrict__ cherry,
                                                           const real* __restrict__ Pm, real* __restrict__ tab,
-                                                          int32_t* __restrict__ etab) {
+                                                          int32_t* __restrict__ etab,
+                                                          int32_t* __restrict__ rescaled) {
   const int k = blockIdx.x / R, r = blockIdx.x % R, code = threadIdx.x;
   const int4 c = cherry[k];
   real x[4], ya[4], yb[4], v[4], y[4];
@@ -760,15 +764,13 @@ __global__ __launch_bounds__(kTabCodes) void k_cherry_tab(const int4* __restrict
   for (int i = 0; i < 4; ++i) v[i] = ya[i] * yb[i];
   rescale4(v, &e);
   matvec4(Pm + ((size_t)c.x * R + r) * 16, v, y);
-  y[0] = e != 0 ? -y[0] : y[0];
   real* d = tab + ((size_t)blockIdx.x * kTabCodes + code) * 4;
 #pragma unroll
   for (int i = 0; i < 4; ++i) d[i] = y[i];
   etab[(size_t)blockIdx.x * kTabCodes + code] = e;
+  const int any = __syncthreads_or(e != 0);
+  if (code == 0) rescaled[blockIdx.x] = any;
 }
-
-__device__ __forceinline__ bool sign_set(float x) { return (int32_t)__float_as_uint(x) < 0; }
-__device__ __forceinline__ bool sign_set(double x) { return __double2hiint(x) < 0; }
 
 // MODE 0: whole tree, ending with the root sum; MODE 1: parts side by side, each
 // storing its root partial in its slot of the part rows (as k_prune_part)
@@ -777,9 +779,10 @@ __global__ __launch_bounds__(64 * R) void k_prune_tab(
     const int4* __restrict__ prog, const int32_t* __restrict__ meta, const int32_t* __restrict__ n_rows,
     int n_progs, const int32_t* __restrict__ fifo, const uint64_t* __restrict__ tips, int64_t stride,
     int64_t n_pat, int64_t pitch, const real* __restrict__ Pm, const real* __restrict__ tab,
-    const int32_t* __restrict__ etab, const double* __restrict__ pi, const double* __restrict__ probs,
-    const uint32_t* __restrict__ weights, double* __restrict__ site_lnl, double* __restrict__ wave_sums,
-    real* __restrict__ xt, int32_t* __restrict__ xte, int N, int stack_depth, int tip_off) {
+    const int32_t* __restrict__ etab, const int32_t* __restrict__ rescaled, const double* __restrict__ pi,
+    const double* __restrict__ probs, const uint32_t* __restrict__ weights, double* __restrict__ site_lnl,
+    double* __restrict__ wave_sums, real* __restrict__ xt, int32_t* __restrict__ xte, int N, int stack_depth,
+    int tip_off) {
   extern __shared__ unsigned char lds_raw[];
   const int64_t nb = pitch / 64;
   const int64_t t = xcd_tile(blockIdx.x);
@@ -826,15 +829,13 @@ __global__ __launch_bounds__(64 * R) void k_prune_tab(
   const int32_t* etabr = etab + (size_t)r * kTabCodes;
 
   // y = the table's product for the code pair c, its exponent into e
-  auto table = [&](int slot, uint32_t c, real* yv, int* e) {
+  auto table = [&](int slot, int res, uint32_t c, real* yv, int* e) {
     typedef real real4 __attribute__((ext_vector_type(4)));
     const real4 v = *reinterpret_cast<const real4*>(tabr + (size_t)slot * (R * kTabCodes * 4) + c * 4);
     *e = 0;
-    if (sign_set(v[0])) *e = etabr[(size_t)slot * (R * kTabCodes) + c];
-    yv[0] = fabs(v[0]);
-    yv[1] = v[1];
-    yv[2] = v[2];
-    yv[3] = v[3];
+    if (res) *e = etabr[(size_t)slot * (R * kTabCodes) + c];  // uniform
+#pragma unroll
+    for (int k = 0; k < 4; ++k) yv[k] = v[k];
   };
   // codes of an entry's operands, read an entry ahead (an operand that is no leaf
   // or table entry reads some row: one past the last is padding)
@@ -857,7 +858,7 @@ __global__ __launch_bounds__(64 * R) void k_prune_tab(
     real xa[4], xb[4];
     int ea, eb;
     if (sa == SRC_EXT) {
-      table(op.x & 0xffff, ca, xa, &ea);
+      table(op.x & 0xffff, fl & kTabResA, ca, xa, &ea);
     } else if (sa == SRC_LEAF) {
       real x[4];
       tipvec(ca, x);
@@ -867,7 +868,7 @@ __global__ __launch_bounds__(64 * R) void k_prune_tab(
       st.product_a(sa, 0, 0, reinterpret_cast<const real(*)[16]>(&PA), reinterpret_cast<real(*)[4]>(&xa), &ea);
     }
     if (sb == SRC_EXT) {
-      table((uint32_t)op.x >> 16, cb, xb, &eb);
+      table((int)((uint32_t)op.x >> 16), fl & kTabResB, cb, xb, &eb);
     } else if (sb == SRC_LEAF) {
       real x[4];
       tipvec(cb, x);
@@ -878,6 +879,9 @@ __global__ __launch_bounds__(64 * R) void k_prune_tab(
       eb = st.acc_e[0];
     }
     st.combine(0, reinterpret_cast<const real(*)[4]>(&xa), reinterpret_cast<const real(*)[4]>(&xb), &ea, &eb);
+  }, [&](int4& e) {  // the lane's entry (an operand of another kind names slot 0, its mark is not looked at)
+    e.w |= rescaled[(e.x & 0xffff) * R + r] ? kTabResA : 0;
+    e.w |= rescaled[(int)((uint32_t)e.x >> 16) * R + r] ? kTabResB : 0;
   });
   if constexpr (MODE == 1)
     st.ext_store(y);
@@ -2562,7 +2566,7 @@ struct Plan {
   size_t off_xt = 0, off_xte = 0;
   // fused pass with the cherries' products from a table
   bool tab = false;
-  size_t off_tab_y = 0, off_tab_e = 0;
+  size_t off_tab_y = 0, off_tab_e = 0, off_tab_r = 0;
 };
 
 constexpr size_t kLdsMax = 64 * 1024;
@@ -2672,6 +2676,7 @@ Plan make_plan(const phy_topo* t, const phy_model* m, int64_t n_pat, int32_t for
     const size_t ent = t->tab.cherry.size() / 4 * R * kTabCodes;
     pl.off_tab_y = o; o = align256(o + ent * 4 * esz);
     pl.off_tab_e = o; o = align256(o + ent * 4);
+    pl.off_tab_r = o; o = align256(o + ent / kTabCodes * 4);
   }
   pl.off_bsum = o; o = align256(o + (size_t)pl.n_waves * 8);
   if (derivs) {
@@ -2769,7 +2774,8 @@ int launch_tree(phy_ctx* ctx, const phy_topo* t, const phy_model* m, bool fused,
   if (pl.tab) {
     hipLaunchKernelGGL((k_cherry_tab<real, R>), dim3((unsigned)(t->tab.cherry.size() / 4 * R)), dim3(kTabCodes), 0,
                        ctx->stream, t->tab.d_cherry, P, reinterpret_cast<real*>(work + pl.off_tab_y),
-                       reinterpret_cast<int32_t*>(work + pl.off_tab_e));
+                       reinterpret_cast<int32_t*>(work + pl.off_tab_e),
+                       reinterpret_cast<int32_t*>(work + pl.off_tab_r));
     PHY_LAUNCHED(ctx);
   }
   auto tables = [&](auto kern, int lv, real* xt, int32_t* xte) {
@@ -2778,7 +2784,8 @@ int launch_tree(phy_ctx* ctx, const phy_topo* t, const phy_model* m, bool fused,
     hipLaunchKernelGGL(kern, dim3((unsigned)((pl.n_blocks * tp.n_progs + 31) / 32 * 32)), dim3(64 * R), lds,
                        ctx->stream, tp.sp.d_prog, tp.sp.d_meta, tp.d_rows, tp.n_progs, tp.sp.d_fifo, tips, stride,
                        n_pat, pl.pitch, P, reinterpret_cast<const real*>(work + pl.off_tab_y),
-                       reinterpret_cast<const int32_t*>(work + pl.off_tab_e), d_pi, d_probs, weights, site_lnl, bsum,
+                       reinterpret_cast<const int32_t*>(work + pl.off_tab_e),
+                       reinterpret_cast<const int32_t*>(work + pl.off_tab_r), d_pi, d_probs, weights, site_lnl, bsum,
                        xt, xte, N, tp.sp.depth, (int)tab_tip_off(R, sizeof(real), tp.sp.depth, lv));
   };
   {

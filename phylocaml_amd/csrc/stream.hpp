@@ -65,9 +65,14 @@ __device__ __forceinline__ void for_each_entry(const int4* __restrict__ prog, in
 }
 
 // Same, passing the following entry too (equal to the last entry at the end),
-// for passes that prefetch operands one node ahead.
-template <class F>
-__device__ __forceinline__ void for_each_entry_ahead(const int4* __restrict__ prog, int n_ops, F&& f) {
+// for passes that prefetch operands one node ahead.  `mark` may add to a lane's
+// entry as its chunk of 64 is taken up (the following entry of a chunk's last
+// one is not marked yet).
+struct NoMark {
+  __device__ __forceinline__ void operator()(int4&) const {}
+};
+template <class F, class M = NoMark>
+__device__ __forceinline__ void for_each_entry_ahead(const int4* __restrict__ prog, int n_ops, F&& f, M&& mark = M()) {
   if (n_ops <= 0) return;
   const int lane = threadIdx.x & 63;
   int4 cur = prog[min(lane, n_ops - 1)];
@@ -75,6 +80,7 @@ __device__ __forceinline__ void for_each_entry_ahead(const int4* __restrict__ pr
   for (int base = 0; base < n_ops; base += 64) {
     const int cnt = __builtin_amdgcn_readfirstlane(min(64, n_ops - base));  // wave-uniform
     landed(cur);
+    mark(cur);
     for (int j = 0; j < cnt; ++j) {
       int4 op, on;
       op.x = __builtin_amdgcn_readlane(cur.x, j);

@@ -433,3 +433,33 @@ def test_cherry_tables_are_bit_identical(ctx, rng, monkeypatch, R, N, P):
         for b in got.values():
             assert np.array_equal(np.float64(a["lnl"]), np.float64(b["lnl"]), equal_nan=True), form
             assert np.array_equal(a["site"], b["site"], equal_nan=True)
+
+
+@pytest.mark.parametrize("co", [(0, 1, 1, 1, 1), (1, 0, 1, 1, 1), (1e-8, 2, 0.5, 1, 1),
+                                (1e-7, 1, 3, 1e-7, 1), (1e-6, 1, 1e-6, 1e-6, 1)])
+def test_cherry_tables_with_negative_entries_of_p(ctx, rng, monkeypatch, co):
+    # near-zero exchangeabilities and short branches: entries of P below the
+    # eigen sums' rounding come out negative, in cherries that are rescaled
+    _say(f"prune tables co={co}")
+    from phylocaml_amd import mlmodel as MM
+
+    N, P = 150, 2000
+    model = MM.create(MM.Spec(4, ("GTR", np.array(co, float)), ("DiscreteGamma", 4, 0.5),
+                              ("Empirical", rng.dirichlet(np.full(4, 5.0))), MM.PHY_GAMMA_MEAN))
+    ch, root = random_tree(rng, N)
+    bl = 10.0 ** rng.uniform(-9, -5, 2 * N - 1)
+    bl[root] = 0.0
+    rt = np.outer(bl, model.rates)
+    pm = np.einsum("ik,brk,kj->brij", model.u, np.exp(model.d * rt[..., None]), model.ui)
+    neg = (pm < 0) & (rt >= 1e-10)[..., None, None]
+    cherries = [ch[2 * k:2 * k + 2] for k in range(N - 1) if max(ch[2 * k:2 * k + 2]) < N]
+    assert sum(bool(neg[a].any() or neg[b].any()) for a, b in cherries) > 5
+    tips, w = _tips(rng, N, P), np.ones(P, np.uint32)
+    for form in (F32 | FUSED, F64 | FUSED):
+        got = {}
+        for tab in ("0", "1"):
+            monkeypatch.setenv("PHY_PRUNE_TAB", tab)
+            got[tab] = _run(ctx, N, ch, root, bl, model, tips, w, form, False)
+        assert np.isfinite(got["0"]["site"]).mean() > 0.5
+        assert np.array_equal(got["0"]["site"], got["1"]["site"], equal_nan=True), form
+        assert np.array_equal(np.float64(got["0"]["lnl"]), np.float64(got["1"]["lnl"]), equal_nan=True)
