@@ -222,12 +222,13 @@ int phy_fitch_insertion_costs(phy_ctx* ctx, const uint64_t* d_pre, const uint64_
  *   d_node_cost (nullable) N-1 uint64: weighted local cost of each internal
  *               node N+k (NonAdditive_c.t.cost of that node).
  *   d_total     1 uint64: sum_s w_s site_cost_s.
- * A tree of >= 24 leaves may run split (parts side by side, then the top);
- * the per-part site counts live in a device buffer owned by the topology,
- * allocated on the first call and grown with n_sites, so two down-passes of
- * one topology must not run at the same time on different streams.  Under
- * graph capture a pass that would have to grow it runs with fewer parts or
- * whole, where that needs less. */
+ * A tree of >= 24 leaves may run split (parts side by side, then the top).
+ * From 128 leaves on, passes over many sites keep the per-part site counts in a
+ * device buffer owned by the topology, allocated on the first such call and
+ * grown with n_sites, so two down-passes of one such topology must not run at
+ * the same time on different streams, and a pass over more sites than any before
+ * ends the use of graphs captured on that topology.  Under graph capture a pass
+ * that would have to grow the buffer runs without it. */
 int phy_fitch_downpass(phy_ctx* ctx, const phy_topo* topo, uint64_t* d_sets,
                        int64_t stride, int64_t n_sites, const uint32_t* d_weights,
                        uint32_t* d_site_cost, uint64_t* d_node_cost,

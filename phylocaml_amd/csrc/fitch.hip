@@ -308,7 +308,8 @@ struct SetLoad {
 
 // Pass modes: the whole tree in one program, or a tree split at cut nodes:
 // the parts side by side (grid.y = part; per-site counts of a part go to
-// scratch[part][lane][8V]) and then the top, which adds the parts' counts.
+// scratch[part][lane][8V], or without scratch are added up in site_cost) and then
+// the top, which adds the parts' counts.
 // A part's count at a site is at most its number of internal nodes, so when
 // every part has at most 255 of them (narrow) the counts are stored as bytes
 // (a quarter of the scratch traffic).
@@ -323,7 +324,86 @@ enum : int { MODE_WHOLE = 0, MODE_PART = 1, MODE_TOP = 2 };
     fifo_ids += meta[2 * (n_parts + 1) + (k)];          \
   } while (0)
 
-// W = number of 32-bit words per node row; lane w owns words V*w .. V*w+V-1
+// Parts' counts without scratch: the sites of a block keep their words of
+// site_cost for themselves until the block of the top has read them, so the
+// parts add their counts up in the first of those words, packed `per` = 4 (a
+// site's total is at most N - 1 <= 255) or 2 to a word, two words an atomic and
+// consecutive lanes on consecutive words.  A last block with too few sites for
+// that adds site by site, and so does every block (per = 1) where site_cost is
+// not 8-byte aligned.  64 taxa x 520,000 sites 26 us, 190 x 10^6 71.  (One
+// word and atomic a site: 33 and 88; packed but lane by lane, a 64-byte line
+// each: 44 and 123; rows of scratch a part, which passes of one tree would
+// share: 25 and 75.)
+template <int V, class F>
+__device__ __forceinline__ void part_counts(int64_t b0, int64_t n_sites, int bd, int per, F&& f) {
+  const int64_t left = n_sites - b0;  // sites of the block
+  if (per == 1 || left < 8 * V * bd / per) f(std::integral_constant<int, 1>());
+  else if (per == 4) f(std::integral_constant<int, 4>());
+  else f(std::integral_constant<int, 2>());
+}
+
+template <int V>
+__device__ __forceinline__ void add_counts(uint32_t* site_cost, int64_t b0, int64_t n_sites, int bd, int tid,
+                                           const uint32_t* site, int per) {
+  part_counts<V>(b0, n_sites, bd, per, [&](auto pc) {
+    constexpr int P = decltype(pc)::value, NW = 8 * V / P;  // counts a word, words a lane
+    if constexpr (P == 1) {
+#pragma unroll
+      for (int k = 0; k < 8 * V; ++k)
+        if (b0 + tid * (8 * V) + k < n_sites) atomicAdd(site_cost + b0 + tid * (8 * V) + k, site[k]);
+    } else {
+      auto* dst = reinterpret_cast<unsigned long long*>(site_cost + b0);
+#pragma unroll
+      for (int q = 0; q < NW / 2; ++q) {
+        unsigned long long x = 0;
+#pragma unroll
+        for (int b = 0; b < 2 * P; ++b) x |= (unsigned long long)site[2 * P * q + b] << (32 / P * b);
+        atomicAdd(dst + q * bd + tid, x);
+      }
+    }
+  });
+}
+
+template <int V>
+__device__ __forceinline__ void take_counts(const uint32_t* site_cost, int64_t b0, int64_t n_sites, int bd, int tid,
+                                            uint32_t* site, int per) {
+  part_counts<V>(b0, n_sites, bd, per, [&](auto pc) {
+    constexpr int P = decltype(pc)::value, NW = 8 * V / P;
+    if constexpr (P == 1) {
+#pragma unroll
+      for (int k = 0; k < 8 * V; ++k)
+        if (b0 + tid * (8 * V) + k < n_sites) site[k] += site_cost[b0 + tid * (8 * V) + k];
+    } else {
+      const auto* src = reinterpret_cast<const unsigned long long*>(site_cost + b0);
+      unsigned long long x[NW / 2];
+#pragma unroll
+      for (int q = 0; q < NW / 2; ++q) x[q] = src[q * bd + tid];
+#pragma unroll
+      for (int q = 0; q < NW / 2; ++q)
+#pragma unroll
+        for (int b = 0; b < 2 * P; ++b)
+          site[2 * P * q + b] += (uint32_t)(x[q] >> (32 / P * b)) & (P == 4 ? 255u : 65535u);
+    }
+  });
+}
+
+// What the down-pass adds to, cleared in one launch: the total, the node costs
+// and of every `run` site costs the first `head`.
+__global__ __launch_bounds__(256) void k_fitch_clear(unsigned long long* __restrict__ total,
+                                                     unsigned long long* __restrict__ node_cost, int n_nodes,
+                                                     uint32_t* __restrict__ site_cost, int64_t n_sites, int head,
+                                                     int run, int64_t n_words) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i == 0) *total = 0;
+  if (i < n_nodes) node_cost[i] = 0;
+  if (i < n_words) {
+    const int64_t k = i / head * run + i % head;
+    if (k < n_sites) site_cost[k] = 0;
+  }
+}
+
+// W = number of 32-bit words per node row; lane w owns words V*w .. V*w+V-1.
+// `narrow`: counts as bytes in the scratch rows, or part_counts' `per` without
 template <int BATCH, bool NODE_COST, int MODE, int V, bool NT, bool PACED>
 __global__ __launch_bounds__(256) void k_fitch_down(
     const int4* __restrict__ prog, int n_ops, const int32_t* __restrict__ fifo_ids,
@@ -435,6 +515,10 @@ __global__ __launch_bounds__(256) void k_fitch_down(
     for (int k = tid; k < n_ops; k += bd)
       if (ncl[k]) atomicAdd(&node_cost[prog[k].x - N], ncl[k]);
   }
+  if (MODE == MODE_PART && !scratch) {
+    if (act) add_counts<V>(site_cost, (int64_t)blockIdx.x * bd * (8 * V), n_sites, bd, tid, site, narrow);
+    return;
+  }
   if (MODE == MODE_PART) {
     if (act) {
       if (narrow) {  // 4 counts per word, 8V bytes per lane
@@ -451,7 +535,11 @@ __global__ __launch_bounds__(256) void k_fitch_down(
     }
     return;
   }
-  if (MODE == MODE_TOP && act) {
+  if (MODE == MODE_TOP && !scratch) {
+    if (act) take_counts<V>(site_cost, (int64_t)blockIdx.x * bd * (8 * V), n_sites, bd, tid, site, narrow);
+    __syncthreads();  // before the block's site costs go over them
+  }
+  if (MODE == MODE_TOP && act && scratch) {
     if (narrow) {
 #pragma unroll 4
       for (int pq = 0; pq < n_parts; ++pq) {
@@ -790,11 +878,14 @@ struct PassShape {
 // 4-byte lanes below 4,096 waves (1,024 x 100,000: 66 against 72 us; 301 x
 // 600,000: 102 against 96).  Trees below 24 leaves run whole (16 x 2,000 down:
 // 8.5 whole, 10.8 split).
+const FitchSplit* fine_split(const phy_topo* t) {  // (a site's total in 16 bits: add_counts)
+  return t->fine.down.d_prog && t->n_leaves <= 65536 ? &t->fine : nullptr;
+}
 PassShape pass_shape(const phy_topo* t, int64_t W32, bool up) {
   const char* e = getenv("PHY_FITCH_SPLIT");
   const bool may_split = !(e && e[0] == '0');
   const FitchSplit* coarse = may_split && t->split.parts.size() >= 2 && t->split.down.d_prog ? &t->split : nullptr;
-  const FitchSplit* fine = may_split && t->fine.down.d_prog ? &t->fine : nullptr;
+  const FitchSplit* fine = may_split ? fine_split(t) : nullptr;
   auto waves = [&](int words, const FitchSplit* f) {
     return (W32 / words + 63) / 64 * (f ? (int64_t)f->parts.size() : 1);
   };
@@ -807,15 +898,28 @@ PassShape pass_shape(const phy_topo* t, int64_t W32, bool up) {
   return {fine ? fine : coarse, 2, 64};
 }
 
-// Scratch rows of the split down-pass (the part counts of every lane), grown on
-// demand.  During a graph capture nothing can be allocated, so a pass whose
-// fine split needs more than is there takes the coarse one (or runs whole).
-size_t scratch_need(const FitchSplit* f, int64_t W32) {
-  return f ? f->parts.size() * (size_t)W32 * 8 * sizeof(uint32_t) : 0;  // 8 counts per 32-bit word
+// Scratch rows of the coarse down-pass (the part counts of every lane), grown on
+// demand.  The fine split's parts add their counts up in site_cost instead, so
+// that passes of a small tree share nothing.  During a graph capture nothing can
+// be allocated, so a coarse pass that needs more than is there takes the fine
+// split (or runs whole).
+size_t scratch_need(const phy_topo* t, int64_t W32) {
+  return t->split.parts.size() * (size_t)W32 * 8 * sizeof(uint32_t);  // 8 counts per 32-bit word
 }
 bool capturing(phy_ctx* ctx) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(ctx->stream, &st) == hipSuccess && st != hipStreamCaptureStatusNone;
+}
+
+int downpass_clear(phy_ctx* ctx, unsigned long long* total, unsigned long long* node_cost, int N,
+                   uint32_t* site_cost, int64_t n_sites, int head, int run) {
+  const int64_t n_words = (n_sites + run - 1) / run * head;
+  const int n_nodes = node_cost ? N - 1 : 0;
+  const int64_t n = std::max<int64_t>({1, n_nodes, n_words});
+  hipLaunchKernelGGL(k_fitch_clear, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, total, node_cost,
+                     n_nodes, site_cost, n_sites, head, run, n_words);
+  PHY_LAUNCHED(ctx);
+  return PHY_OK;
 }
 
 template <int BATCH, int V, bool NT, bool PACED>
@@ -840,6 +944,11 @@ int downpass_run(phy_ctx* ctx, const phy_topo* topo, uint32_t* s32, int64_t stri
     }
   }
   const unsigned grid = (unsigned)((W32 / V + bs - 1) / bs);
+  // of a fine pass also the words that part_counts names: a block's first ones
+  const bool fine = split && split == &topo->fine;
+  const int per = reinterpret_cast<uintptr_t>(site_cost) % 8 ? 1 : N <= 256 ? 4 : 2;
+  const int rc = downpass_clear(ctx, total, node_cost, N, site_cost, fine ? n_sites : 0, 8 * V * bs / per, 8 * V * bs);
+  if (rc) return rc;
   if (!split) {
     KernelSpan span(ctx, "fitch_down");
     if (node_cost)
@@ -855,7 +964,7 @@ int downpass_run(phy_ctx* ctx, const phy_topo* topo, uint32_t* s32, int64_t stri
   }
   const SplitProg& sp = split->down;
   const int P = (int)split->parts.size();
-  const size_t need = scratch_need(split, W32);
+  const size_t need = fine ? 0 : scratch_need(topo, W32);
   if (topo->scratch_bytes < need) {
     if (topo->d_scratch) PHY_HIP(ctx, hipFree(topo->d_scratch));
     topo->d_scratch = nullptr;
@@ -866,12 +975,12 @@ int downpass_run(phy_ctx* ctx, const phy_topo* topo, uint32_t* s32, int64_t stri
     }
     topo->scratch_bytes = need;
   }
-  uint4* scr = reinterpret_cast<uint4*>(topo->d_scratch);
+  uint4* scr = fine ? nullptr : reinterpret_cast<uint4*>(topo->d_scratch);
   int max_ops = 0;  // internal nodes of the largest part
   for (int k = 0; k < P; ++k) max_ops = std::max(max_ops, (int)sp.n_ops[k]);
   // PHY_FITCH_NARROW=0 keeps 32-bit counts
   const char* ne = getenv("PHY_FITCH_NARROW");
-  const int narrow = max_ops <= 255 && !(ne && ne[0] == '0');
+  const int narrow = fine ? per : max_ops <= 255 && !(ne && ne[0] == '0');
   KernelSpan span(ctx, "fitch_down");
   if (node_cost) {
     hipLaunchKernelGGL((k_fitch_down<BATCH, true, MODE_PART, V, NT, PACED>), dim3(grid, (unsigned)P), dim3(bs), lds,
@@ -982,19 +1091,16 @@ int phy_fitch_downpass(phy_ctx* ctx, const phy_topo* topo, uint64_t* sets, int64
   if (n_sites < 0 || stride < W) return set_err(ctx, PHY_EINVAL, "downpass: stride < words");
   if (!sets || !site_cost || !total) return set_err(ctx, PHY_EINVAL, "downpass: null output");
   const int N = topo->n_leaves;
-  int rc;
-  if ((rc = phy_zero_u64(ctx, total, 1))) return rc;
-  if (node_cost && (rc = phy_zero_u64(ctx, node_cost, N - 1))) return rc;
-  if (W == 0) return PHY_OK;
+  auto* nc = reinterpret_cast<unsigned long long*>(node_cost);
+  auto* tt = reinterpret_cast<unsigned long long*>(total);
+  if (W == 0) return downpass_clear(ctx, tt, nc, N, nullptr, 0, 1, 1);
   const int64_t W32 = 2 * W;  // 32-bit lanes
   PassShape sh = pass_shape(topo, W32, false);
-  if (sh.split == &topo->fine && topo->scratch_bytes < scratch_need(sh.split, W32) && capturing(ctx))
-    sh.split = topo->split.parts.size() >= 2 ? &topo->split : nullptr;
+  if (sh.split == &topo->split && topo->scratch_bytes < scratch_need(topo, W32) && capturing(ctx))
+    sh.split = fine_split(topo);
   const FitchSplit* split = sh.split;
   const int bs = block_size_env("PHY_FITCH_BLOCK", sh.block);
   uint32_t* s32 = reinterpret_cast<uint32_t*>(sets);
-  auto* nc = reinterpret_cast<unsigned long long*>(node_cost);
-  auto* tt = reinterpret_cast<unsigned long long*>(total);
   // full passes take 16-byte non-temporal lanes and a 4-deep ring: at 1,024
   // taxa x 10^6 sites 0.243 ms against 0.266 ms for 8-byte cached lanes and an
   // 8-deep ring (sweep over words 1 / 2 / 4, ring 4 / 8 / 16, non-temporal or not,

@@ -196,13 +196,14 @@ def test_empty_and_bad_arguments(ctx):
 
 
 @pytest.mark.parametrize("N,S", [(23, 700), (24, 700), (40, 1), (40, 513), (301, 20_011),
-                                 (24, 530_001), (130, 400_003)])
+                                 (24, 530_001), (130, 400_003), (256, 4099), (256, 5000), (257, 4103), (257, 4700)])
 @pytest.mark.parametrize("weights", ["unit", "small", "heavy"])
 def test_pass_shapes_and_node_costs(ctx, rng, N, S, weights):
     # both sides of the dispatch lines (whole tree below 24 leaves, fine split
-    # with narrow lanes, whole tree and wide lanes at many sites) with node
-    # costs counted, weighed by bit planes (up to 8 bits) or walked (one site
-    # of 2^20 makes its wave do so)
+    # with narrow lanes, its part counts in 8 bits up to 256 leaves and in 16
+    # beyond, or one a word in a last block of few sites, whole tree and wide
+    # lanes at many sites) with node costs counted, weighed by bit planes (up to
+    # 8 bits) or walked (one site of 2^20 makes its wave do so)
     _say(f"fitch shapes N={N} S={S} weights={weights}")
     ch, root = random_tree(rng, N)
     leaves = rng.integers(1, 16, (N, S)).astype(np.uint8)
@@ -242,3 +243,51 @@ def test_insertion_costs_match_oracle(ctx, rng, S, weights):
         ww = np.ones(S, np.int64) if w is None else w.astype(np.int64)
         want = [int(ww[(sets[0][c] & pairs[a, b]) == 0].sum()) for c, a, b in q.tolist()]
         assert out.cpu().tolist() == want
+
+
+@pytest.mark.parametrize("N", [24, 64, 127])
+def test_passes_of_one_small_topology_on_two_streams(rng, N):
+    # below 128 leaves a pass shares nothing with another one of its topology:
+    # two alignments of different lengths, passes in flight side by side
+    from phylocaml_amd import device as D, nonadditive as NA
+
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    _say(f"fitch two streams N={N}")
+    ch, root = random_tree(rng, N)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    ctxs = [D.Context(0, stream=s.cuda_stream) for s in streams]
+    topo = D.Topology(N, ch, root, ctxs[0])
+    leaves = [rng.integers(1, 16, (N, S)).astype(np.uint8) for S in (3001, 60_007)]
+    fts = [NA.alloc_tree(c, topo, lv.shape[1], D.pack_nibbles(lv), with_node_cost=True)
+           for c, lv in zip(ctxs, leaves)]
+    torch.cuda.synchronize()
+    for _ in range(30):
+        for c, ft in zip(ctxs, fts):
+            NA.downpass(c, topo, ft, None)
+    torch.cuda.synchronize()
+    for ft, lv in zip(fts, leaves):
+        osets, osc, onc, otot = O.fitch_downpass(N, ch, root, lv, None, threads=8)
+        assert np.array_equal(ft.sets.cpu().numpy()[N:], D.pack_nibbles(osets[N:]))
+        assert np.array_equal(ft.site_cost.cpu().numpy()[:lv.shape[1]], osc)
+        assert np.array_equal(ft.node_cost.cpu().numpy(), onc)
+        assert int(ft.total.cpu().numpy()[0]) == otot
+
+
+@pytest.mark.parametrize("N", [24, 200, 300])
+def test_site_costs_at_a_word_aligned_address(ctx, rng, N):
+    from phylocaml_amd import device as D, nonadditive as NA
+
+    S = 4099
+    _say(f"fitch unaligned site costs N={N}")
+    ch, root = random_tree(rng, N)
+    leaves = rng.integers(1, 16, (N, S)).astype(np.uint8)
+    topo = D.Topology(N, ch, root, ctx)
+    ft = NA.alloc_tree(ctx, topo, S, D.pack_nibbles(leaves), with_node_cost=True)
+    buf = torch.full((S + 3,), 7, dtype=torch.int32, device="cuda")
+    ft.site_cost = buf[1:S + 1].view(torch.uint32)
+    NA.downpass(ctx, topo, ft, None)
+    osets, osc, onc, otot = O.fitch_downpass(N, ch, root, leaves, None, threads=8)
+    assert np.array_equal(ft.site_cost.cpu().numpy(), osc)
+    assert int(ft.total.cpu().numpy()[0]) == otot
+    assert buf.cpu().tolist()[0] == 7 and buf.cpu().tolist()[S + 1:] == [7, 7]

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from conftest import random_tree
+from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -93,3 +94,43 @@ def test_fitch_graph_replays_match_eager(rng):
             assert np.array_equal(ft.final.cpu().numpy(), ref_fin), k
             NA.downpass(ctx, topo, ft)
             ctx.sync()
+
+
+@pytest.mark.parametrize("N", [60, 300])
+@pytest.mark.parametrize("warm", [0, 5000])
+def test_fitch_capture_without_a_warm_up(rng, N, warm):
+    # the first pass over these sites is the captured one (at 300 leaves an eager
+    # pass would allocate the parts' counts); then an eager pass of the same size,
+    # which may, between the replays
+    from phylocaml_amd import device as D, nonadditive as NA
+
+    _gpu()
+    s = torch.cuda.Stream()
+    ctx = D.Context(0, stream=s.cuda_stream)
+    S = 300_007
+    ch, root = random_tree(rng, N)
+    leaves = [rng.integers(1, 16, (N, n)).astype(np.uint8) for n in (S, max(warm, 1))]
+    with torch.cuda.stream(s):
+        topo = D.Topology(N, ch, root, ctx)
+        ft, small = (NA.alloc_tree(ctx, topo, lv.shape[1], D.pack_nibbles(lv), with_node_cost=True)
+                     for lv in leaves)
+        if warm:
+            NA.downpass(ctx, topo, small, None)
+        ctx.sync()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            NA.downpass(ctx, topo, ft, None)
+        osets, osc, onc, otot = O.fitch_downpass(N, ch, root, leaves[0], None, threads=8)
+        want = D.pack_nibbles(osets[N:])
+        for k in range(4):
+            for t in (ft.site_cost, ft.node_cost, ft.total):
+                t.view(torch.int32).fill_(7)
+            if k < 3:
+                g.replay()
+            else:
+                NA.downpass(ctx, topo, ft, None)
+            torch.cuda.synchronize()
+            assert np.array_equal(ft.sets.cpu().numpy()[N:], want), k
+            assert np.array_equal(ft.site_cost.cpu().numpy()[:S], osc), k
+            assert np.array_equal(ft.node_cost.cpu().numpy(), onc), k
+            assert int(ft.total.cpu().numpy()[0]) == otot, k
