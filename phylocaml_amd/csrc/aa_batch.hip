@@ -446,10 +446,9 @@ __global__ __launch_bounds__(64 * (TW / G)) void k_aa_prune(AADev a) {
           else acc_e[g] = ea[g] + x[g].e;
         }
       }
-      // Rescale, except at a node of two leaves: its values are products of two
-      // entries of P (>= ~1e-15 each: a branch below 1e-10 is the identity), far
-      // inside the range, and its parent tests again.
-      if ((fl & 15) != (SRC_LEAF | SRC_LEAF << 2))
+      // Every node is rescaled, one of two leaves too: two such sisters of ~1e-17
+      // each (short branches, states without direct exchange) leave FP32's range
+      // at their parent.
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         // per-pattern rescale: lanes l, l^16, l^32, l^48 share pattern pl

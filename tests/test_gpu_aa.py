@@ -189,3 +189,43 @@ def test_every_tile_gives_the_same_trees(ctx, R):
         for k, t in enumerate(trees):
             ov = _oracle(t)
             assert abs(got[4][k] - ov) <= 2e-3 * abs(ov), (k, got[4][k], ov)
+
+
+@pytest.mark.parametrize("t", [2e-10, 5e-10, 1e-8])
+def test_sister_cherries_of_short_branches(ctx, t):
+    # ((a, b), (c, d)) with no direct exchange between the four states: each
+    # cherry's values are ~1e-21, and without a rescale there their product at
+    # the parent (branches of length 0) leaves FP32's range.  The same tree with a missing leaf beside
+    # a and c on branches of length 0 (P = 1) has the same values at every node
+    # and no node of two leaves that needs a rescale.
+    from phylocaml_amd import aa
+
+    rng = np.random.default_rng(5)
+    pi = rng.dirichlet(np.full(20, 20.0))
+    ex = rng.uniform(0.5, 2.0, (20, 20))
+    ex[:4, :4] = 0.0
+    ex = np.triu(ex, 1)
+    q = (ex + ex.T) * pi[None, :]
+    np.fill_diagonal(q, -q.sum(1))
+    q /= -(pi * np.diag(q)).sum()
+    one, w = np.ones(1), np.ones(1, np.uint32)
+
+    def tree(n, children, blen, codes):
+        return aa.AATree(n, np.array(children, np.int32), 2 * n - 2, np.array(blen), pi, q, one, one,
+                         np.array(codes, np.uint8)[:, None], w)
+
+    plain, padded = [], []
+    for p in ([0, 1, 2, 3], [1, 3, 0, 2], [2, 0, 3, 1], [3, 2, 1, 0], [0, 1, 5, 3], [7, 8, 9, 10]):
+        plain.append(tree(4, [0, 1, 2, 3, 4, 5], [t] * 4 + [0.0] * 3, p))
+        # leaves a b c d ? ?: 6 = (a, ?), 7 = (6, b), 8 = (c, ?), 9 = (8, d), 10 = (7, 9)
+        padded.append(tree(6, [0, 4, 6, 1, 2, 5, 8, 3, 7, 9],
+                           [0.0, t, 0.0, t, 0.0, 0.0, t, 0.0, t, 0.0, 0.0], p + [255, 255]))
+    print(f"aa sister cherries t={t}", flush=True)
+    b = aa.AABatch(ctx, plain + padded, waves=4)
+    b.run()
+    ctx.sync()
+    got, want = np.split(b.lnl.cpu().numpy(), 2)
+    print(got, want, flush=True)
+    ok = np.isfinite(want)  # a negative entry of P (rounding of its eigen sum) may leave no value
+    assert ok.sum() >= 3
+    assert np.all(np.abs(got[ok] - want[ok]) <= 1e-6 * np.abs(want[ok]))
