@@ -538,14 +538,17 @@ int phy_lk_spr_scores(phy_ctx* ctx, const phy_model* model, int32_t form,
  * every branch (the lnL of every regraft of s is a sum over patterns of
  * log sum_r prob_r [P(t_v/2)^T A_v] . ([P(t_v/2) D_v] (*) P(t_s) D_s)).
  * About 2N node operations per pruned subtree instead of N per move; the
- * values equal phy_lk_spr_scores' up to rounding.  At least s_batch pruned
- * subtrees run per launch, more where few patterns would leave the chip idle
- * (within 2 GiB of rows); the workspace depends on the tree (its longest
- * repair path), the patterns and s_batch, and the call takes one sized for
- * s_batch subtrees a launch too.  d_base_lnl (nullable, device) receives the base
+ * values equal phy_lk_spr_scores' up to rounding.  s_batch pruned subtrees
+ * run per launch; the workspace depends on the tree (its longest repair
+ * path) and on s_batch.  phy_lk_incr_batch gives a batch worth the workspace:
+ * s_batch, or more where few patterns would leave the chip idle (about 2 GiB
+ * at most).  d_base_lnl (nullable, device) receives the base
  * tree's lnL.  Replaces the per-move evaluation of the candidates of
  * TreeNeighborhoods' SPR generator (lib/treeNeighborhoods.ml:27-75), whose
  * trees the reference scores one Tree.join at a time (lib/tree.ml:400-494). */
+int phy_lk_incr_batch(int32_t n_leaves, const int32_t* children, int32_t root,
+                      const phy_model* model, int64_t n_patterns, int32_t form,
+                      int32_t s_batch, int32_t* batch);
 int phy_lk_spr_incr_work_size(int32_t n_leaves, const int32_t* children, int32_t root,
                               const phy_model* model, int64_t n_patterns, int32_t form,
                               int32_t s_batch, size_t* bytes);

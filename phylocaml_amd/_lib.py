@@ -106,6 +106,7 @@ SIGNATURES = {
                                     P_i32, i32, vp, vp, sz]),
     "phy_lk_tbr_scores": (C.c_int, [vp, vp, i32, i64, vp, i64, vp, i32, P_i32, i32, P_f64, i64,
                                     P_i32, i32, vp, vp, sz]),
+    "phy_lk_incr_batch": (C.c_int, [i32, P_i32, i32, vp, i64, i32, i32, P_i32]),
     "phy_lk_spr_incr_work_size": (C.c_int, [i32, P_i32, i32, vp, i64, i32, i32, C.POINTER(sz)]),
     "phy_lk_spr_scores_incr": (C.c_int, [vp, vp, i32, i64, vp, i64, vp, i32, P_i32, i32, P_f64,
                                          i64, P_i32, i32, vp, vp, vp, sz]),

@@ -3391,9 +3391,10 @@ IncrPlan incr_plan(const IncrTree& t, int R, int64_t n_pat, int32_t form, int32_
   return pl;
 }
 
-// Pruned subtrees per launch: the caller's s_batch, or more where few patterns
-// would leave the chip idle between the launches of a round (about 8,192 blocks,
-// eight rounds of resident ones, while the rows of a batch stay within 2 GiB).
+// Pruned subtrees per launch worth asking for (phy_lk_incr_batch): s_batch, or
+// more where few patterns would leave the chip idle between the launches of a
+// round (about 8,192 blocks, eight rounds of resident ones, while the rows of a
+// batch stay within 2 GiB).
 // s_batch = 16, whole rounds: 96 taxa x 10,007 patterns FP32 9.12 ms so and 8.13
 // with 53 subtrees a launch; x 1,000 patterns 3.3 and 1.6; TBR 64 x 5,003 FP64
 // 2.81 and 2.38.
@@ -3960,12 +3961,11 @@ int tbr_group(const IncrTree& t, int64_t n_moves, const int32_t* moves, int S, T
 
 int tbr_plan_create(phy_ctx* ctx, const phy_model* m, int32_t form, int64_t n_pat, int32_t N,
                     const int32_t* children, int32_t root, int64_t n_moves, const int32_t* moves, int32_t s_batch,
-                    phy_spr_plan** out, bool grow = true) {
+                    phy_spr_plan** out) {
   std::unique_ptr<phy_spr_plan> sp(new phy_spr_plan());
   if (!sp->t.load(N, children, root)) return set_err(ctx, PHY_EINVAL, "tbr incremental: not a rooted binary tree");
   const IncrTree& t = sp->t;
-  const int M = t.M, R = m->R;
-  int S = grow ? incr_batch(t, R, n_pat, form, s_batch) : s_batch;
+  const int M = t.M, S = s_batch, R = m->R;
   sp->tbr = true;
   sp->form = form;
   sp->R = R;
@@ -3973,8 +3973,7 @@ int tbr_plan_create(phy_ctx* ctx, const phy_model* m, int32_t form, int64_t n_pa
   sp->n_moves = n_moves;
   TbrGroups grp;
   int64_t bad = -1;
-  int gr = tbr_group(t, n_moves, moves, S, &grp, &bad);
-  if (gr == 2 && S != s_batch) gr = tbr_group(t, n_moves, moves, S = s_batch, &grp, &bad);
+  const int gr = tbr_group(t, n_moves, moves, S, &grp, &bad);
   if (gr == 1) return set_err(ctx, PHY_EINVAL, "tbr incremental: invalid move " + std::to_string(bad));
   if (gr == 2) return set_err(ctx, PHY_ERANGE, "tbr incremental: too many pairs in a batch");
   const int n_sub = sp->n_sub = grp.n_sub;
@@ -4124,13 +4123,26 @@ int check_plan_model(phy_ctx* ctx, const phy_model* m) {
 
 extern "C" {
 
+int phy_lk_incr_batch(int32_t N, const int32_t* children, int32_t root, const phy_model* m, int64_t n_pat,
+                      int32_t form, int32_t s_batch, int32_t* batch) {
+  if (!m || !batch || !children || N < 3 || n_pat < 1 || s_batch < 1) return PHY_EINVAL;
+  try {
+    IncrTree t;
+    if (!t.load(N, children, root)) return PHY_EINVAL;
+    *batch = incr_batch(t, m->R, n_pat, form, s_batch);
+    return PHY_OK;
+  } catch (...) {
+    return PHY_ENOMEM;
+  }
+}
+
 int phy_lk_spr_incr_work_size(int32_t N, const int32_t* children, int32_t root, const phy_model* m,
                               int64_t n_pat, int32_t form, int32_t s_batch, size_t* bytes) {
   if (!m || !bytes || !children || N < 3 || n_pat < 1 || s_batch < 1) return PHY_EINVAL;
   try {
     IncrTree t;
     if (!t.load(N, children, root)) return PHY_EINVAL;
-    *bytes = incr_plan(t, m->R, n_pat, form, incr_batch(t, m->R, n_pat, form, s_batch)).total;
+    *bytes = incr_plan(t, m->R, n_pat, form, s_batch).total;
     return PHY_OK;
   } catch (...) {
     return PHY_ENOMEM;
@@ -4147,10 +4159,7 @@ int phy_spr_plan_create(phy_ctx* ctx, const phy_model* m, int32_t form, int64_t 
   int rc = check_plan_model(ctx, m);
   if (rc) return rc;
   try {
-    IncrTree t;
-    if (!t.load(N, children, root)) return set_err(ctx, PHY_EINVAL, "spr incremental: not a rooted binary tree");
-    return plan_create(ctx, m, form, n_pat, N, children, root, n_moves, moves,
-                       incr_batch(t, m->R, n_pat, form, s_batch), out);
+    return plan_create(ctx, m, form, n_pat, N, children, root, n_moves, moves, s_batch, out);
   } catch (...) {
     return set_err(ctx, PHY_ENOMEM, "spr plan: host allocation or thread start failed");
   }
@@ -4189,13 +4198,10 @@ int phy_lk_spr_scores_incr(phy_ctx* ctx, const phy_model* m, int32_t form, int64
   try {
     IncrTree t;
     if (!t.load(N, children, root)) return set_err(ctx, PHY_EINVAL, "spr incremental: not a rooted binary tree");
-    // a workspace sized for s_batch itself is enough
-    int32_t S = incr_batch(t, m->R, n_pat, form, s_batch);
-    if (work_bytes < incr_plan(t, m->R, n_pat, form, S).total) S = s_batch;
-    const IncrPlan lay = incr_plan(t, m->R, n_pat, form, S);
+    const IncrPlan lay = incr_plan(t, m->R, n_pat, form, s_batch);
     if (work_bytes < lay.total) return set_err(ctx, PHY_EINVAL, "spr incremental: workspace too small");
     phy_spr_plan* sp = nullptr;
-    rc = plan_create(ctx, m, form, n_pat, N, children, root, n_moves, moves, S, &sp);
+    rc = plan_create(ctx, m, form, n_pat, N, children, root, n_moves, moves, s_batch, &sp);
     if (rc) return rc;
     std::unique_ptr<phy_spr_plan> hold(sp);
     char* work = static_cast<char*>(d_work);
@@ -4222,11 +4228,9 @@ int phy_lk_tbr_incr_work_size(int32_t N, const int32_t* children, int32_t root, 
     if (!t.load(N, children, root)) return PHY_EINVAL;
     TbrGroups g;
     int64_t bad = -1;
-    int32_t S = incr_batch(t, m->R, n_pat, form, s_batch);
-    int gr = tbr_group(t, n_moves, moves, S, &g, &bad);
-    if (gr == 2 && S != s_batch) gr = tbr_group(t, n_moves, moves, S = s_batch, &g, &bad);
+    const int gr = tbr_group(t, n_moves, moves, s_batch, &g, &bad);
     if (gr) return gr == 1 ? PHY_EINVAL : PHY_ERANGE;
-    *bytes = incr_plan(t, m->R, n_pat, form, S, g.n_sub, g.max_xrows, g.max_pairs).total;
+    *bytes = incr_plan(t, m->R, n_pat, form, s_batch, g.n_sub, g.max_xrows, g.max_pairs).total;
     return PHY_OK;
   } catch (...) {
     return PHY_ENOMEM;
@@ -4264,11 +4268,6 @@ int phy_lk_tbr_scores_incr(phy_ctx* ctx, const phy_model* m, int32_t form, int64
     rc = tbr_plan_create(ctx, m, form, n_pat, N, children, root, n_moves, moves, s_batch, &sp);
     if (rc) return rc;
     std::unique_ptr<phy_spr_plan> hold(sp);
-    if (work_bytes < sp->pl.total) {  // a workspace sized for s_batch itself is enough
-      rc = tbr_plan_create(ctx, m, form, n_pat, N, children, root, n_moves, moves, s_batch, &sp, false);
-      if (rc) return rc;
-      hold.reset(sp);
-    }
     if (work_bytes < sp->pl.total) return set_err(ctx, PHY_EINVAL, "tbr incremental: workspace too small");
     char* work = static_cast<char*>(d_work);
     double* dbl = reinterpret_cast<double*>(work + sp->pl.off_blh);

@@ -24,7 +24,7 @@ from dataclasses import dataclass
 
 import numpy as np
 
-from . import device as D
+from . import device as D, spr
 from ._lib import PhyError, check, lib, ptr
 
 
@@ -178,7 +178,7 @@ class Scorer:
 
     def __init__(self, ctx: D.Context, dm, n_leaves: int, tips, stride: int, weights,
                  n_patterns: int, form: int = 0, chunk: int = 2048,
-                 incremental: bool | None = None, s_batch: int = 16):
+                 incremental: bool | None = None, s_batch: int = spr.DEFAULT_BATCH):
         torch = __import__("torch")
         self.ctx, self.dm, self.N = ctx, dm, int(n_leaves)
         self.tips, self.stride, self.weights = tips, int(stride), weights
@@ -229,24 +229,27 @@ class Scorer:
 
     def _score_incremental(self, ch, root, bl, mv, tbr, out):
         torch = __import__("torch")
-        nb = C.c_size_t()
-        if tbr:
-            check(lib.phy_lk_tbr_incr_work_size(
-                self.N, ptr(ch, C.c_int32), int(root), self.dm.handle, self.n_patterns,
-                self.form, len(mv), ptr(mv, C.c_int32), self.s_batch, C.byref(nb)),
-                None, "tbr incremental work size")
-        else:
-            check(lib.phy_lk_spr_incr_work_size(
-                self.N, ptr(ch, C.c_int32), int(root), self.dm.handle, self.n_patterns,
-                self.form, self.s_batch, C.byref(nb)), None, "spr incremental work size")
-        if self.iwork.numel() < nb.value:
-            self.iwork = torch.empty((nb.value,), dtype=torch.uint8,
-                                     device=f"cuda:{self.ctx.device}")
+        def size(b):
+            nb = C.c_size_t()
+            if tbr:
+                check(lib.phy_lk_tbr_incr_work_size(
+                    self.N, ptr(ch, C.c_int32), int(root), self.dm.handle, self.n_patterns,
+                    self.form, len(mv), ptr(mv, C.c_int32), b, C.byref(nb)),
+                    None, "tbr incremental work size")
+            else:
+                check(lib.phy_lk_spr_incr_work_size(
+                    self.N, ptr(ch, C.c_int32), int(root), self.dm.handle, self.n_patterns,
+                    self.form, b, C.byref(nb)), None, "spr incremental work size")
+            return nb.value
+
+        batches = spr.launch_batches(self.dm, self.N, ch, root, self.n_patterns, self.form,
+                                     self.s_batch)
+        self.iwork, batch = spr.batch_workspace(self.iwork, batches, size)
         fn = lib.phy_lk_tbr_scores_incr if tbr else lib.phy_lk_spr_scores_incr
         self.ctx.check(fn(self.ctx.handle, self.dm.handle, self.form, self.n_patterns,
                           D.dptr(self.tips), self.stride, D.dptr(self.weights), self.N,
                           ptr(ch, C.c_int32), int(root), ptr(bl, C.c_double), len(mv),
-                          ptr(mv, C.c_int32), self.s_batch, D.dptr(out),
+                          ptr(mv, C.c_int32), batch, D.dptr(out),
                           D.dptr(self.base_lnl), D.dptr(self.iwork), self.iwork.numel()),
                        "neighbour scores (incremental)")
         return out[: len(mv)]

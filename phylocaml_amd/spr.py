@@ -11,7 +11,9 @@ import ctypes as C
 import numpy as np
 
 from . import device as D
-from ._lib import check, lib, ptr
+from ._lib import PhyError, check, lib, ptr
+
+DEFAULT_BATCH = 16  # pruned subtrees per launch of the incremental scorers
 
 
 def moves(n_leaves: int, children, root: int) -> np.ndarray:
@@ -68,15 +70,44 @@ class Scorer:
         return out[: len(mv)]
 
 
+def launch_batches(dm, n_leaves: int, children, root: int, n_patterns: int, form: int,
+                   s_batch: int) -> list[int]:
+    """Batches for the incremental scorers, the first one preferred:
+    DEFAULT_BATCH is raised where few patterns would leave the chip idle
+    (phy_lk_incr_batch) if there is memory for that; another s_batch is taken
+    as it is."""
+    if s_batch != DEFAULT_BATCH:
+        return [s_batch]
+    b = C.c_int32()
+    check(lib.phy_lk_incr_batch(n_leaves, ptr(children, C.c_int32), int(root), dm.handle,
+                                n_patterns, form, s_batch, C.byref(b)), None, "launch batch")
+    return sorted({b.value, s_batch}, reverse=True)
+
+
+def batch_workspace(work, batches: list[int], size):
+    """(workspace, batch): the first batch whose workspace of size(batch) bytes
+    fits in `work` or can be allocated."""
+    torch = __import__("torch")
+    for b in batches:
+        try:
+            need = size(b)
+            if work.numel() < need:
+                work = torch.empty((need,), dtype=torch.uint8, device=work.device)
+            return work, b
+        except (PhyError, torch.OutOfMemoryError):
+            if b == batches[-1]:
+                raise
+
+
 class IncrementalScorer:
     """Exact lnL of SPR neighbours without a tree per move
     (phy_lk_spr_scores_incr): per pruned subtree, a repair of the base
     tree's partials and one pre-order pass score every regraft.  Same
     values as Scorer up to rounding; the workspace grows with the tree's
-    longest repair path."""
+    longest repair path and with s_batch (see launch_batches)."""
 
     def __init__(self, ctx: D.Context, dm, n_leaves: int, tips, stride: int, weights,
-                 n_patterns: int, form: int = 0, s_batch: int = 16):
+                 n_patterns: int, form: int = 0, s_batch: int = DEFAULT_BATCH):
         torch = __import__("torch")
         self.ctx, self.dm, self.N = ctx, dm, int(n_leaves)
         self.tips, self.stride, self.weights = tips, int(stride), weights
@@ -84,11 +115,12 @@ class IncrementalScorer:
         self.work = torch.empty((0,), dtype=torch.uint8, device=f"cuda:{ctx.device}")
         self.base_lnl = torch.zeros((1,), dtype=torch.float64, device=f"cuda:{ctx.device}")
 
-    def work_size(self, children, root: int) -> int:
+    def work_size(self, children, root: int, s_batch: int | None = None) -> int:
         ch = np.ascontiguousarray(children, np.int32)
         nb = C.c_size_t()
         check(lib.phy_lk_spr_incr_work_size(self.N, ptr(ch, C.c_int32), int(root), self.dm.handle,
-                                            self.n_patterns, self.form, self.s_batch, C.byref(nb)))
+                                            self.n_patterns, self.form, s_batch or self.s_batch,
+                                            C.byref(nb)))
         return nb.value
 
     def score(self, children, root: int, blen, mv: np.ndarray):
@@ -98,14 +130,13 @@ class IncrementalScorer:
         mv = np.ascontiguousarray(mv, np.int32)
         ch = np.ascontiguousarray(children, np.int32)
         bl = np.ascontiguousarray(blen, np.float64)
-        need = self.work_size(ch, root)
-        if self.work.numel() < need:
-            self.work = torch.empty((need,), dtype=torch.uint8, device=f"cuda:{self.ctx.device}")
+        batches = launch_batches(self.dm, self.N, ch, root, self.n_patterns, self.form, self.s_batch)
+        self.work, batch = batch_workspace(self.work, batches, lambda b: self.work_size(ch, root, b))
         out = torch.empty((max(len(mv), 1),), dtype=torch.float64, device=f"cuda:{self.ctx.device}")
         self.ctx.check(lib.phy_lk_spr_scores_incr(
             self.ctx.handle, self.dm.handle, self.form, self.n_patterns, D.dptr(self.tips),
             self.stride, D.dptr(self.weights), self.N, ptr(ch, C.c_int32), int(root),
-            ptr(bl, C.c_double), len(mv), ptr(mv, C.c_int32), self.s_batch, D.dptr(out),
+            ptr(bl, C.c_double), len(mv), ptr(mv, C.c_int32), batch, D.dptr(out),
             D.dptr(self.base_lnl), D.dptr(self.work), self.work.numel()), "spr_scores_incr")
         return out[: len(mv)]
 
@@ -121,7 +152,7 @@ class SprPlan:
 
     def __init__(self, ctx: D.Context, dm, n_leaves: int, tips, stride: int, weights,
                  n_patterns: int, children, root: int, mv: np.ndarray, form: int = 0,
-                 s_batch: int = 16):
+                 s_batch: int = DEFAULT_BATCH):
         torch = __import__("torch")
         self.ctx, self.dm, self.N = ctx, dm, int(n_leaves)
         self.tips, self.stride, self.weights = tips, int(stride), weights
@@ -129,17 +160,24 @@ class SprPlan:
         tbr = mv.ndim == 2 and mv.shape[1] == 3
         self.mv = mv if tbr else mv.reshape(-1, 2)
         ch = np.ascontiguousarray(children, np.int32)
-        h = C.c_void_p()
         create = lib.phy_tbr_plan_create if tbr else lib.phy_spr_plan_create
-        ctx.check(create(ctx.handle, dm.handle, int(form), int(n_patterns), self.N,
-                         ptr(ch, C.c_int32), int(root), len(self.mv), ptr(self.mv, C.c_int32),
-                         int(s_batch), C.byref(h)),
-                  "tbr_plan_create" if tbr else "spr_plan_create")
-        self.handle = h
-        nb = C.c_size_t()
-        check(lib.phy_spr_plan_work_size(h, C.byref(nb)))
         dev = f"cuda:{ctx.device}"
-        self.work = torch.empty((max(nb.value, 8),), dtype=torch.uint8, device=dev)
+        self.handle = None
+
+        def plan(b):  # the plan for b subtrees a launch, and its workspace's size
+            self.close()
+            h = C.c_void_p()
+            ctx.check(create(ctx.handle, dm.handle, int(form), int(n_patterns), self.N,
+                             ptr(ch, C.c_int32), int(root), len(self.mv),
+                             ptr(self.mv, C.c_int32), b, C.byref(h)),
+                      "tbr_plan_create" if tbr else "spr_plan_create")
+            self.handle = h
+            nb = C.c_size_t()
+            check(lib.phy_spr_plan_work_size(h, C.byref(nb)))
+            return max(nb.value, 8)
+
+        batches = launch_batches(dm, self.N, ch, root, int(n_patterns), int(form), int(s_batch))
+        self.work, _ = batch_workspace(torch.empty((0,), dtype=torch.uint8, device=dev), batches, plan)
         self.lnl = torch.zeros((max(len(self.mv), 1),), dtype=torch.float64, device=dev)
         self.base_lnl = torch.zeros((1,), dtype=torch.float64, device=dev)
 

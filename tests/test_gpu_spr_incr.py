@@ -274,13 +274,13 @@ def test_plan_runs_equal_the_one_shot_scores_and_replay_from_a_graph():
 @pytest.mark.parametrize("form", [F32, F64])
 @pytest.mark.parametrize("kind", ["spr", "tbr"])
 def test_batch_size_does_not_change_a_score(ctx, form, kind):
-    # a launch takes more pruned subtrees than s_batch where the patterns are
-    # few; a workspace that only holds s_batch at a time is enough, and every
-    # score is the same bits either way
+    # s_batch bounds the workspace of one-shot calls and of plans; the batch that
+    # phy_lk_incr_batch proposes (one launch here) takes more of it; every score
+    # is the same bits, and a workspace for a smaller batch is refused
     import ctypes as C
 
     from phylocaml_amd import device as D, neighborhood as NB, spr, synth
-    from phylocaml_amd._lib import PhyError, lib, ptr
+    from phylocaml_amd._lib import PhyError, check, lib, ptr
 
     N, P = 30, 300
     tree = synth.yule(N, 9, 0.1)
@@ -293,28 +293,75 @@ def test_batch_size_does_not_change_a_score(ctx, form, kind):
     ch = np.ascontiguousarray(tree.children, np.int32)
     bl = np.ascontiguousarray(tree.blen, np.float64)
     mv = np.ascontiguousarray(mv, np.int32)
-    nb = C.c_size_t()
-    if kind == "spr":
-        rc = lib.phy_lk_spr_incr_work_size(N, ptr(ch, C.c_int32), tree.root, dm.handle, P, form, 1,
-                                           C.byref(nb))
-    else:
-        rc = lib.phy_lk_tbr_incr_work_size(N, ptr(ch, C.c_int32), tree.root, dm.handle, P, form,
-                                           len(mv), ptr(mv, C.c_int32), 1, C.byref(nb))
-    assert rc == 0
-    fn = lib.phy_lk_spr_scores_incr if kind == "spr" else lib.phy_lk_tbr_scores_incr
-    work = torch.empty((nb.value,), dtype=torch.uint8, device="cuda")
-    got, refused = [], 0
-    for s_batch, size in ((1, nb.value), (1, nb.value // 2), (7, nb.value), (1, 4096)):
-        _say(f"{kind} batch {s_batch} form {form} workspace {size}")
+    auto = C.c_int32()
+    check(lib.phy_lk_incr_batch(N, ptr(ch, C.c_int32), tree.root, dm.handle, P, form, 1,
+                                C.byref(auto)))
+    assert auto.value == 2 * N - 1
+
+    def size(b):
+        nb = C.c_size_t()
+        if kind == "spr":
+            check(lib.phy_lk_spr_incr_work_size(N, ptr(ch, C.c_int32), tree.root, dm.handle, P, form,
+                                                b, C.byref(nb)))
+        else:
+            check(lib.phy_lk_tbr_incr_work_size(N, ptr(ch, C.c_int32), tree.root, dm.handle, P, form,
+                                                len(mv), ptr(mv, C.c_int32), b, C.byref(nb)))
+        return nb.value
+
+    sizes = [size(b) for b in (1, 7, auto.value)]
+    assert sizes[0] < sizes[1] < sizes[2]
+    one_shot = lib.phy_lk_spr_scores_incr if kind == "spr" else lib.phy_lk_tbr_scores_incr
+    create = lib.phy_spr_plan_create if kind == "spr" else lib.phy_tbr_plan_create
+    work = torch.empty((sizes[2],), dtype=torch.uint8, device="cuda")
+    bld, got = D.to_device(bl), []
+    for b, need in zip((1, 7, auto.value), sizes):
+        _say(f"{kind} batch {b} form {form} workspace {need}")
         out = torch.zeros((len(mv),), dtype=torch.float64, device="cuda")
-        try:
-            ctx.check(fn(ctx.handle, dm.handle, form, P, D.dptr(tips), D.words(P), D.dptr(wd), N,
-                         ptr(ch, C.c_int32), tree.root, ptr(bl, C.c_double), len(mv),
-                         ptr(mv, C.c_int32), s_batch, D.dptr(out), None, D.dptr(work), size), kind)
-        except PhyError as e:
-            assert e.code == 1
-            refused += 1
-            continue
-        got.append(out.cpu().numpy())
-    assert refused == 1 and len(got) == 3
-    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+        h, nb = C.c_void_p(), C.c_size_t()
+        ctx.check(create(ctx.handle, dm.handle, form, P, N, ptr(ch, C.c_int32), tree.root, len(mv),
+                         ptr(mv, C.c_int32), b, C.byref(h)), "plan")
+        check(lib.phy_spr_plan_work_size(h, C.byref(nb)))
+        assert nb.value <= need
+
+        def run(plan, nbytes):
+            if plan:
+                ctx.check(lib.phy_spr_plan_run(ctx.handle, h, dm.handle, D.dptr(tips), D.words(P),
+                                               D.dptr(wd), D.dptr(bld), D.dptr(out), None,
+                                               D.dptr(work), nbytes), "plan run")
+            else:
+                ctx.check(one_shot(ctx.handle, dm.handle, form, P, D.dptr(tips), D.words(P), D.dptr(wd),
+                                   N, ptr(ch, C.c_int32), tree.root, ptr(bl, C.c_double), len(mv),
+                                   ptr(mv, C.c_int32), b, D.dptr(out), None, D.dptr(work), nbytes), kind)
+
+        for plan in (True, False):
+            out.zero_()
+            run(plan, nb.value if plan else need)
+            got.append(out.cpu().numpy())
+            with pytest.raises(PhyError) as e:
+                run(plan, (nb.value if plan else need) - 1)
+            assert e.value.code == 1
+        lib.phy_spr_plan_destroy(h)
+    assert np.all(np.isfinite(got[0])) and all(np.array_equal(got[0], g) for g in got)
+
+
+def test_scorers_batches(ctx, monkeypatch):
+    # the scorers raise the default batch, take another one as given, and fall
+    # back to the default where there is no memory for the raised one
+    from phylocaml_amd import spr, synth
+
+    N, P = 30, 300
+    tree = synth.yule(N, 9, 0.1)
+    model = _model(9)
+    st, w = _data(tree, model, P, 9)
+    mv = spr.moves(N, tree.children, tree.root)
+    ref, sizes = None, {}
+    for s_batch in (16, 5, 0):
+        inc, _, _ = _scorers(ctx, model, st, w, N, F64, s_batch=s_batch or 16)
+        if s_batch == 0:
+            size = inc.work_size
+            monkeypatch.setattr(inc, "work_size", lambda c, r, b: size(c, r, b) if b == 16 else 1 << 60)
+        got = inc.score(tree.children, tree.root, tree.blen, mv).cpu().numpy()
+        ref = got if ref is None else ref
+        assert np.array_equal(got, ref)
+        sizes[s_batch] = inc.work.numel()
+    assert sizes[5] < sizes[0] < sizes[16]
