@@ -2621,7 +2621,7 @@ bool use_tables(const phy_topo* t, int R, size_t esz, int64_t n_pat) {
 }
 
 Plan make_plan(const phy_topo* t, const phy_model* m, int64_t n_pat, int32_t form, int32_t derivs,
-               bool allow_split = true) {
+               bool allow_split = true, bool allow_tab = true) {
   Plan pl;
   const int N = t->n_leaves, M = 2 * N - 1, R = m->R, K = m->K;
   pl.esz = (form & PHY_F32) ? 4 : 8;
@@ -2671,9 +2671,9 @@ Plan make_plan(const phy_topo* t, const phy_model* m, int64_t n_pat, int32_t for
     pl.off_xte = o; o = align256(o + (size_t)pl.n_parts * R * pl.pitch * 4);
   }
   // the split decision stands; without parts the table form runs whole
-  pl.tab = allow_split && pl.fused && pl.rpw == 1 && (pl.split || t->pparts.empty()) && use_tables(t, R, esz, n_pat);
-  if (pl.tab) {
-    const size_t ent = t->tab.cherry.size() / 4 * R * kTabCodes;
+  pl.tab = allow_split && allow_tab && pl.fused && pl.rpw == 1 && (pl.split || t->pparts.empty()) && use_tables(t, R, esz, n_pat);
+  if (pl.tab) {  // room for the most cherries of N leaves: trees of one size need one workspace
+    const size_t ent = (size_t)(N / 2) * R * kTabCodes;
     pl.off_tab_y = o; o = align256(o + ent * 4 * esz);
     pl.off_tab_e = o; o = align256(o + ent * 4);
     pl.off_tab_r = o; o = align256(o + ent / kTabCodes * 4);
@@ -3043,7 +3043,9 @@ int phy_lk_tree(phy_ctx* ctx, const phy_topo* t, const phy_model* m, int32_t for
   if (n_pat < 1) return set_err(ctx, PHY_EINVAL, "lk_tree: need at least one pattern");
   if (stride < phy_words(n_pat)) return set_err(ctx, PHY_EINVAL, "lk_tree: tip stride < words");
   if (!tips || !weights || !blen || !lnl || !work) return set_err(ctx, PHY_EINVAL, "lk_tree: null argument");
-  const Plan pl = make_plan(t, m, n_pat, form, derivs);
+  Plan pl = make_plan(t, m, n_pat, form, derivs);
+  // (a workspace that only holds the plain form, from a tree without tables, serves it)
+  if (work_bytes < pl.total && pl.tab) pl = make_plan(t, m, n_pat, form, derivs, true, false);
   if (work_bytes < pl.total) return set_err(ctx, PHY_EINVAL, "lk_tree: workspace too small");
   char* w = static_cast<char*>(work);
   if (form & PHY_F32)

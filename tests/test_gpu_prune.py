@@ -463,3 +463,45 @@ def test_cherry_tables_with_negative_entries_of_p(ctx, rng, monkeypatch, co):
         assert np.isfinite(got["0"]["site"]).mean() > 0.5
         assert np.array_equal(got["0"]["site"], got["1"]["site"], equal_nan=True), form
         assert np.array_equal(np.float64(got["0"]["lnl"]), np.float64(got["1"]["lnl"]), equal_nan=True)
+
+
+@pytest.mark.parametrize("form", [F32 | FUSED, F64 | FUSED])
+def test_one_workspace_serves_trees_of_one_size(ctx, rng, monkeypatch, form):
+    # a caterpillar (one node of two leaves) and a balanced tree (N / 2 of them)
+    # need the same workspace, and one that holds the plain form alone is enough
+    import ctypes as C
+
+    from phylocaml_amd import device as D, likelihood as LK
+    from phylocaml_amd._lib import PhyError, check, lib
+
+    N, P = 128, 700
+    model = _model(rng, 4)
+    dm = LK.DeviceModel(ctx, model)
+    tips, w = _tips(rng, N, P), np.ones(P, np.uint32)
+    bl = rng.exponential(0.1, 2 * N - 1) + 1e-3
+    bl[2 * N - 2] = 0.0
+    trees = {"balanced": np.arange(2 * N - 2, dtype=np.int32), "caterpillar": caterpillar(N)[0]}
+    td, wd, bd = D.to_device(D.pack_nibbles(tips)), D.to_device(w), D.to_device(bl)
+    sizes, got = {}, {}
+    for name, ch in trees.items():
+        topo = D.Topology(N, ch, 2 * N - 2, ctx)
+        for tab in ("0", "1"):
+            monkeypatch.setenv("PHY_PRUNE_TAB", tab)
+            nb = C.c_size_t()
+            check(lib.phy_lk_tree_work_size(topo.handle, dm.handle, P, form, 0, C.byref(nb)))
+            sizes[name, tab] = nb.value
+        for nbytes in (sizes[name, "1"], sizes[name, "1"] - 1, sizes[name, "0"], sizes[name, "0"] - 1):
+            _say(f"lk_tree {name} form {form} workspace {nbytes}")
+            work = torch.empty((nbytes,), dtype=torch.uint8, device="cuda")
+            lnl, site = (torch.zeros((n,), dtype=torch.float64, device="cuda") for n in (1, P))
+            args = (ctx.handle, topo.handle, dm.handle, form, P, D.dptr(td), D.words(P), D.dptr(wd),
+                    D.dptr(bd), D.dptr(lnl), D.dptr(site), None, None, D.dptr(work), nbytes)
+            if nbytes < sizes[name, "0"]:
+                with pytest.raises(PhyError):
+                    ctx.check(lib.phy_lk_tree(*args), "lk_tree")
+                continue
+            ctx.check(lib.phy_lk_tree(*args), "lk_tree")
+            got.setdefault(name, site.cpu().numpy())
+            assert np.array_equal(got[name], site.cpu().numpy())
+    assert sizes["balanced", "0"] == sizes["caterpillar", "0"]
+    assert sizes["balanced", "1"] == sizes["caterpillar", "1"] > sizes["balanced", "0"]
