@@ -577,14 +577,6 @@ int phy_compile_topo(phy_topo* t) {
   return 0;
 }
 
-static std::vector<int32_t> split_meta(const SplitProg& sp) {
-  std::vector<int32_t> meta;
-  meta.insert(meta.end(), sp.prog_off.begin(), sp.prog_off.end());
-  meta.insert(meta.end(), sp.n_ops.begin(), sp.n_ops.end());
-  meta.insert(meta.end(), sp.fifo_off.begin(), sp.fifo_off.end());
-  return meta;
-}
-
 // Device copies of every program of a topology, packed into one allocation and
 // one copy (a search makes a topology per accepted move): `put` queues an array
 // and the pointer that is to hold its device address.
