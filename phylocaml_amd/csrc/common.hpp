@@ -135,6 +135,7 @@ struct phy_topo {
   // (about sqrt(N) parts, device only) for passes whose sites leave the chip
   // idle, which are bound by the longest chain of nodes
   FitchSplit split, fine;
+  bool fitch_fine = true;
   // split form of the fused pruning pass (its own cuts, fewer than the Fitch
   // passes take: every part adds a stored root partial per pattern):
   // psplit holds the part programs; the top program reads the cut nodes as

@@ -662,8 +662,10 @@ int phy_topo_create(phy_ctx* ctx, int32_t N, const int32_t* children, int32_t ro
     return PHY_OK;
   }
   // about sqrt(N) parts of sqrt(N) leaves under a top of as many nodes: the
-  // shortest chain of two launches (PHY_FITCH_PARTS keeps to its one split)
-  if (N >= 24 && !getenv("PHY_FITCH_PARTS")) {
+  // shortest chain of two launches (with PHY_FITCH_PARTS the Fitch passes keep to
+  // its one split)
+  t->fitch_fine = !getenv("PHY_FITCH_PARTS");
+  if (N >= 24) {
     const int want = std::min(kMaxParts, (int)std::lround(std::sqrt((double)N)));
     if (compile_fitch_split(t, want, std::max(3, N / want / 2), &t->fine, true)) {
       delete t;

@@ -879,7 +879,7 @@ struct PassShape {
 // 600,000: 102 against 96).  Trees below 24 leaves run whole (16 x 2,000 down:
 // 8.5 whole, 10.8 split).
 const FitchSplit* fine_split(const phy_topo* t) {  // (a site's total in 16 bits: add_counts)
-  return t->fine.down.d_prog && t->n_leaves <= 65536 ? &t->fine : nullptr;
+  return t->fitch_fine && t->fine.down.d_prog && t->n_leaves <= 65536 ? &t->fine : nullptr;
 }
 PassShape pass_shape(const phy_topo* t, int64_t W32, bool up) {
   const char* e = getenv("PHY_FITCH_SPLIT");

@@ -28,6 +28,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <cstdlib>
 
 #include "common.hpp"
 #include "stream.hpp"
@@ -258,9 +259,10 @@ int sankoff_launch(phy_ctx* ctx, const phy_topo* topo, const int32_t* tcm, const
   // against 136; 128 taxa, K = 8, 100,003 sites 123 against 118, 50,000 sites 84
   // against 97.  Under three waves a block it does not pay at all.  Of the
   // numbers of waves the largest serves where every CU has at most one block, the
-  // one with the most waves on a CU elsewhere.
+  // one with the most waves on a CU elsewhere.  PHY_SANKOFF_SPLIT=0: the whole form.
   const FitchSplit& f = topo->fine;
-  const int P = (int)f.parts.size();
+  const char* env = getenv("PHY_SANKOFF_SPLIT");
+  const int P = env && env[0] == '0' ? 0 : (int)f.parts.size();
   int waves = 0, held = 0;
   size_t lds = 0;
   for (int w = std::min(kSplitWaves, P); w >= 3; --w) {

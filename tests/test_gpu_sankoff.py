@@ -100,15 +100,15 @@ def test_sankoff_argument_errors(ctx, rng):
 @pytest.mark.parametrize("N,S", [(24, 63), (97, 1000), (511, 4097), (64, 300_001)])
 def test_split_and_whole_walks_agree(ctx, rng, monkeypatch, K, N, S):
     # blocks of 64 sites whose waves share the tree's parts, against one wave for
-    # the tree (a topology made under PHY_FITCH_PARTS has no fine split)
+    # the tree (PHY_SANKOFF_SPLIT=0 runs the whole form)
     for kind in ("random", "caterpillar"):
         _say(f"sankoff split K={K} N={N} S={S} {kind}")
         ch, root = random_tree(rng, N) if kind == "random" else caterpillar(N)
         tcm = rng.integers(0, 50, (K, K)).astype(np.int32)
         leaves = rng.integers(0, 1 << K, (N, S)).astype(np.uint8)
         w = rng.integers(0, 7, S).astype(np.uint32)
-        monkeypatch.delenv("PHY_FITCH_PARTS", raising=False)
+        monkeypatch.delenv("PHY_SANKOFF_SPLIT", raising=False)
         split = _run(ctx, N, ch, root, tcm, leaves, w, stride=S + 5)
-        monkeypatch.setenv("PHY_FITCH_PARTS", "1")
+        monkeypatch.setenv("PHY_SANKOFF_SPLIT", "0")
         whole = _run(ctx, N, ch, root, tcm, leaves, w, stride=S + 5)
         assert np.array_equal(split[0], whole[0]) and split[1] == whole[1]
