@@ -1,6 +1,7 @@
 // Shared definitions of the gfx950 library: context, topology programs,
 // error reporting.
 #pragma once
+#include <atomic>
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -146,6 +147,9 @@ struct phy_topo {
   std::vector<int32_t> ptop_prog, ptop_fifo;
   int32_t ptop_depth = 0;
   TabProg tab;
+  // 1 + the register levels of the table form's stack, by precision, log2 of the
+  // rate classes and whether it runs in parts; 0: not chosen yet
+  mutable std::atomic<int> tab_levels[2][4][2] = {};
   int4* d_ptop_prog = nullptr;
   int32_t* d_ptop_fifo = nullptr;
   // per-part partial site costs of the split down-pass, grown on demand

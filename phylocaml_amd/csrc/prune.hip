@@ -21,7 +21,6 @@
 // FP64 dynamic range without rounding from the scaling itself.
 #include <algorithm>
 #include <climits>
-#include <atomic>
 #include <memory>
 #include <cmath>
 #include <mutex>
@@ -2722,12 +2721,16 @@ int register_levels(int depth, int bs) {
   return best;
 }
 
-// Register levels of the table form's stack, chosen as register_levels does.
+// Register levels of the table form's stack, chosen as register_levels does and
+// kept with the topology (the LDS depends on its programs).
 template <typename real, int R, int MODE>
-int tab_register_levels(const TabProg& tp) {
+int tab_register_levels(const phy_topo* t) {
+  const TabProg& tp = t->tab;
   const int depth = tp.sp.depth;
   const char* s = getenv("PHY_PRUNE_REG");
   if (s && s[0] >= '0' && s[0] <= '2' && s[1] == 0) return std::min(s[0] - '0', depth);
+  std::atomic<int>& chosen = t->tab_levels[sizeof(real) == 8][R == 8 ? 3 : R / 2][MODE];
+  if (const int c = chosen.load()) return c - 1;
   const void* kern[3] = {reinterpret_cast<const void*>(&k_prune_tab<real, R, 0, MODE>),
                          reinterpret_cast<const void*>(&k_prune_tab<real, R, 1, MODE>),
                          reinterpret_cast<const void*>(&k_prune_tab<real, R, 2, MODE>)};
@@ -2739,6 +2742,7 @@ int tab_register_levels(const TabProg& tp) {
       continue;
     if (nb > best_nb) best = lv, best_nb = nb;
   }
+  chosen.store(best + 1);
   return best;
 }
 
@@ -2791,7 +2795,7 @@ int launch_tree(phy_ctx* ctx, const phy_topo* t, const phy_model* m, bool fused,
   {
     KernelSpan span(ctx, "prune_down");
     if (pl.tab && !pl.split) {
-      const int lvt = tab_register_levels<real, R, 0>(t->tab);
+      const int lvt = tab_register_levels<real, R, 0>(t);
       if (lvt == 2) tables(k_prune_tab<real, R, 2, 0>, 2, nullptr, nullptr);
       else if (lvt == 1) tables(k_prune_tab<real, R, 1, 0>, 1, nullptr, nullptr);
       else tables(k_prune_tab<real, R, 0, 0>, 0, nullptr, nullptr);
@@ -2809,7 +2813,7 @@ int launch_tree(phy_ctx* ctx, const phy_topo* t, const phy_model* m, bool fused,
                            part, ex, N, sd.depth);
       };
       if (pl.tab) {
-        const int lvt = tab_register_levels<real, R, 1>(t->tab);
+        const int lvt = tab_register_levels<real, R, 1>(t);
         if (lvt == 2) tables(k_prune_tab<real, R, 2, 1>, 2, xt, xte);
         else if (lvt == 1) tables(k_prune_tab<real, R, 1, 1>, 1, xt, xte);
         else tables(k_prune_tab<real, R, 0, 1>, 0, xt, xte);
