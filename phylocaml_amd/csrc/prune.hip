@@ -2775,13 +2775,6 @@ int launch_tree(phy_ctx* ctx, const phy_topo* t, const phy_model* m, bool fused,
   };
   constexpr int G2 = (R % 2 == 0 && sizeof(real) == 4) ? 2 : 1;
   const int lv = ((fused || pl.lds_stack) && pl.rpw != 2) ? register_levels<real, R>(t->down_depth, pl.bs) : 0;
-  if (pl.tab) {
-    hipLaunchKernelGGL((k_cherry_tab<real, R>), dim3((unsigned)(t->tab.cherry.size() / 4 * R)), dim3(kTabCodes), 0,
-                       ctx->stream, t->tab.d_cherry, P, reinterpret_cast<real*>(work + pl.off_tab_y),
-                       reinterpret_cast<int32_t*>(work + pl.off_tab_e),
-                       reinterpret_cast<int32_t*>(work + pl.off_tab_r));
-    PHY_LAUNCHED(ctx);
-  }
   auto tables = [&](auto kern, int lv, real* xt, int32_t* xte) {
     const TabProg& tp = t->tab;
     const size_t lds = tab_lds(R, sizeof(real), tp, lv);
@@ -2794,6 +2787,13 @@ int launch_tree(phy_ctx* ctx, const phy_topo* t, const phy_model* m, bool fused,
   };
   {
     KernelSpan span(ctx, "prune_down");
+    if (pl.tab) {
+      hipLaunchKernelGGL((k_cherry_tab<real, R>), dim3((unsigned)(t->tab.cherry.size() / 4 * R)), dim3(kTabCodes), 0,
+                         ctx->stream, t->tab.d_cherry, P, reinterpret_cast<real*>(work + pl.off_tab_y),
+                         reinterpret_cast<int32_t*>(work + pl.off_tab_e),
+                         reinterpret_cast<int32_t*>(work + pl.off_tab_r));
+      PHY_LAUNCHED(ctx);
+    }
     if (pl.tab && !pl.split) {
       const int lvt = tab_register_levels<real, R, 0>(t);
       if (lvt == 2) tables(k_prune_tab<real, R, 2, 0>, 2, nullptr, nullptr);
