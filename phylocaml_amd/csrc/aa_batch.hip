@@ -22,11 +22,12 @@
 // The extra tile takes R products over the same operands (A holds the rows of
 // rate r only), so a child is 2R products of R operands.
 // (Padding each rate to 32 states gave 8R values a lane, 12 of every 32 of
-// them zero: 196 VGPRs and two waves per SIMD against 156 and three here.
-// With the rest of the node loop below, 256 trees of 16-256 taxa and
-// 1,000-20,000 patterns take 8.0 ms against 17.1 at 8 groups per tile and 8.3
-// against 16.2 at 4.  Bound: VALU issue ~60% and the node's LDS reads and
-// barrier; MFMA busy ~27%.)
+// them zero: 196 VGPRs and two waves per SIMD against 146 to 158 and three at 4
+// groups per tile here.  With the rest of the node loop below, 256 trees of 16-256
+// taxa and 1,000-20,000 patterns take 9.1 ms against 17.1 at 8 groups per tile and
+// 9.8 against 16.2 at 4.  Bound: the node's LDS reads and barrier, with the VALU
+// held 59% and the matrix cores 29% of the time.  The pairs of figures at the rules
+// below compare forms of one earlier state on one box, 8.0 and 8.3 ms there.)
 // Combining the two children, per-pattern power-of-two rescaling and the root
 // sum are FP32 / FP64 VALU work on 4R + 4 values per lane.  A wave may own G
 // groups of 16 patterns, which share each P operand it reads from LDS.

@@ -672,7 +672,7 @@ int phy_topo_create(phy_ctx* ctx, int32_t N, const int32_t* children, int32_t ro
       return set_err(ctx, PHY_EINVAL, "topology: program compilation failed");
     }
   }
-  // the table form pays where the patterns are many: see use_tables (prune.hip)
+  // the table form of the fused pass (use_tables in prune.hip has its rule)
   if (N >= 16) {
     const std::vector<int32_t> whole = {t->root};
     if (compile_tab(t, t->pparts.empty() ? whole : t->pparts, &t->tab)) {

@@ -671,7 +671,8 @@ __global__ __launch_bounds__(256) void k_fitch_up(const int4* __restrict__ prog,
 // chunk of words (one 16-site word a thread, whose weights it holds as bit
 // planes) through a run of queries, so that the weights are read once a run and
 // a word of P_c once for the neighbouring queries of one c; the waves' sums meet
-// in LDS.  Bound by the L2 reads of the F rows: 128 taxa, 20,011 weighted sites,
+// in LDS.  Bound by VALU issue (80%; 6 TB/s of rows from the L2, 97% of them
+// hits): 128 taxa, 20,011 weighted sites,
 // 61,976 queries take 190 us; one block per query over all words, with a
 // dependent weight load for each flagged site, took 522.
 constexpr int kMaxRun = 64;

@@ -731,17 +731,19 @@ __global__ __launch_bounds__(512) void k_prune_part(
 // instructions instead of ~90.  Entry [slot][class][code_a | code_b << 4], its
 // exponent in etab; rescaled[slot][class] says whether any entry there has one
 // (only cherries of branches below ~1e-6 in FP32): the walk marks its entries
-// with that, 64 at a time, and reads etab under a uniform test.  (The values' own bits have no room for that mark: an
-// entry of P below ~1e-16 comes out of the eigen sums with either sign.)
+// with that, 64 at a time, and reads etab under a uniform test.  (The values' own
+// bits have no room for that mark: an entry of P below ~1e-16 comes out of the
+// eigen sums with either sign.)
 //
 // The walk stages the codes of its tile in LDS first, one byte per operand (a
 // leaf's code, or a cherry's pair) and pattern, shared by the R waves (each wave
 // of the plain walk loads its own), so that an operand's code is one LDS read
 // and the gathers are the only vector loads.  512 taxa x 200,000 patterns, R = 4,
-// whole evaluation: FP32 674 -> 465 us, FP64 904 -> 597 us; 411M -> 237M VALU wave
-// instructions a pass, still VALU-issue bound (97% of the issue cycles).  The
-// leaves' own products from a 16-entry table as well measured slower (510 us:
-// twice the gathers, each ~36 L1 accesses, against 20 VALU instructions saved).
+// whole evaluation, plain and table form: FP32 641 / 460 us, FP64 834 / 590 us;
+// 233M VALU wave instructions in the parts, which hold the VALU 98% of their time
+// (FP32).  The leaves' own products from a 16-entry table as well measured slower
+// (510 us when the rest took 468: twice the gathers against 20 VALU instructions
+// saved).
 // ---------------------------------------------------------------------------
 constexpr int kTabCodes = 256;
 constexpr int kTabResA = 32, kTabResB = 64;  // marks in an entry's flags: read the exponent of A, of B
@@ -2607,16 +2609,19 @@ size_t tab_lds(int R, size_t esz, const TabProg& tp, int lv) {
   return tab_tip_off(R, esz, tp.sp.depth, lv) + (size_t)(tp.max_rows + 2) * 64;
 }
 
-// The table form pays for its table kernel (one launch, ~4 us) where the walk is
-// long or wide: plain and table form in us, FP32 at R = 4, 32 taxa x 5,000
-// patterns 23.2 / 24.3, 64 x 20,000 39.3 / 39.2, 32 x 50,000 28.8 / 25.6, 200 x
-// 2,000 106 / 97, 512 x 4,000 102 / 99, 200 x 100,000 191 / 142.
-// PHY_PRUNE_TAB=0|1 overrides the size rule.
+// The table form pays for its table kernel (one launch, ~5 us) where there are
+// blocks enough to hide latency, and in the parts of a split tree.  A whole tree in
+// up to 512 blocks is the plain walk's, which then touches its P matrices first
+// (kWarmBlocks).  Plain and table form in us at R = 4, FP32 and FP64: 32 taxa x 5,000
+// patterns 20.4 / 23.3 and 21.2 / 24.5; 200 x 8,000 84.9 / 92.8 and 92.0 / 96.2;
+// 128 x 32,000 63.7 / 65.1 and 73.2 / 67.4; 32 x 50,000 29.0 / 25.7 and 32.5 / 27.3;
+// 200 x 100,000 183 / 133 and 235 / 173; split: 300 x 500 127 / 114 and 133 / 115;
+// 512 x 4,000 101 / 95 and 109 / 100.  PHY_PRUNE_TAB=0|1 overrides the size rule.
 bool use_tables(const phy_topo* t, int R, size_t esz, int64_t n_pat) {
   if (!t->tab.n_progs || !t->tab.d_cherry || t->tab.cherry.empty() || tab_lds(R, esz, t->tab, 0) > kLdsMax) return false;
   const char* s = getenv("PHY_PRUNE_TAB");
   if (s && (s[0] == '0' || s[0] == '1') && s[1] == 0) return s[0] == '1';
-  return t->n_leaves >= 128 || n_pat >= 32768;
+  return t->pparts.size() >= 2 || n_pat >= 32768;
 }
 
 Plan make_plan(const phy_topo* t, const phy_model* m, int64_t n_pat, int32_t form, int32_t derivs,
