@@ -865,6 +865,12 @@ struct PassShape {
   int words, block;
 };
 
+// the fine split, if there is one that the pass can take (down, a site's total is
+// added up in 16 bits: add_counts)
+const FitchSplit* fine_split(const phy_topo* t, bool up) {
+  return t->fitch_fine && t->fine.down.d_prog && (up || t->n_leaves <= 65536) ? &t->fine : nullptr;
+}
+
 // A pass with few waves is bound by its longest chain of nodes (0.3-0.9 us a
 // node at one wave per SIMD: instruction latency, at any ring depth), so it
 // takes the fine split, narrow lanes and one-wave blocks; a pass that fills
@@ -878,15 +884,13 @@ struct PassShape {
 // and at 8,192 up (8-byte lanes); the up-pass narrows to
 // 4-byte lanes below 4,096 waves (1,024 x 100,000: 66 against 72 us; 301 x
 // 600,000: 102 against 96).  Trees below 24 leaves run whole (16 x 2,000 down:
-// 8.5 whole, 10.8 split).
-const FitchSplit* fine_split(const phy_topo* t) {  // (a site's total in 16 bits: add_counts)
-  return t->fitch_fine && t->fine.down.d_prog && t->n_leaves <= 65536 ? &t->fine : nullptr;
-}
+// 8.5 whole, 10.8 split).  (The down figures are with part counts in scratch rows;
+// added up in site_cost they are within 4% or lower.)
 PassShape pass_shape(const phy_topo* t, int64_t W32, bool up) {
   const char* e = getenv("PHY_FITCH_SPLIT");
   const bool may_split = !(e && e[0] == '0');
   const FitchSplit* coarse = may_split && t->split.parts.size() >= 2 && t->split.down.d_prog ? &t->split : nullptr;
-  const FitchSplit* fine = may_split ? fine_split(t) : nullptr;
+  const FitchSplit* fine = may_split ? fine_split(t, up) : nullptr;
   auto waves = [&](int words, const FitchSplit* f) {
     return (W32 / words + 63) / 64 * (f ? (int64_t)f->parts.size() : 1);
   };
@@ -1098,7 +1102,7 @@ int phy_fitch_downpass(phy_ctx* ctx, const phy_topo* topo, uint64_t* sets, int64
   const int64_t W32 = 2 * W;  // 32-bit lanes
   PassShape sh = pass_shape(topo, W32, false);
   if (sh.split == &topo->split && topo->scratch_bytes < scratch_need(topo, W32) && capturing(ctx))
-    sh.split = fine_split(topo);
+    sh.split = fine_split(topo, false);
   const FitchSplit* split = sh.split;
   const int bs = block_size_env("PHY_FITCH_BLOCK", sh.block);
   uint32_t* s32 = reinterpret_cast<uint32_t*>(sets);
