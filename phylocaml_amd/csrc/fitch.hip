@@ -666,15 +666,47 @@ __global__ __launch_bounds__(256) void k_fitch_up(const int4* __restrict__ prog,
   });
 }
 
+// Insertion costs with a block per query: each lane adds up its words, one wave
+// sum a query, a load per flagged site where there are weights.
+__global__ __launch_bounds__(256) void k_fitch_insert_each(const uint64_t* __restrict__ pre,
+                                                           const uint64_t* __restrict__ fin, int64_t stride,
+                                                           int64_t W, int64_t n_sites,
+                                                           const uint32_t* __restrict__ wt,
+                                                           const int32_t* __restrict__ qs,
+                                                           unsigned long long* __restrict__ cost) {
+  const int64_t q = blockIdx.x;
+  const uint64_t* pc = pre + (int64_t)qs[3 * q] * stride;
+  const uint64_t* fa = fin + (int64_t)qs[3 * q + 1] * stride;
+  const uint64_t* fb = fin + (int64_t)qs[3 * q + 2] * stride;
+  uint64_t acc = 0;
+  for (int64_t w = threadIdx.x; w < W; w += blockDim.x) {
+    uint32_t t0, t1, elo, ehi;
+    const uint64_t m = fitch64(fa[w], fb[w], &t0, &t1);
+    (void)fitch64(m, pc[w], &elo, &ehi);
+    const uint64_t vm = valid_nibbles(w, n_sites);
+    elo &= (uint32_t)vm;
+    ehi &= (uint32_t)(vm >> 32);
+    acc += wt ? weigh(elo, ehi, wt, w) : (uint64_t)(__popc(elo) + __popc(ehi));
+  }
+  acc = wave_sum(acc);
+  __shared__ unsigned long long sh[4];
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long t = 0;
+    for (int k = 0; k < (int)(blockDim.x >> 6); ++k) t += sh[k];
+    cost[q] = t;
+  }
+}
+
 // Insertion costs of many (c, a, b) queries: sum over the sites of
 // w_s [P_c & med(F_a, F_b) = 0] with med the Fitch median.  A block takes a
 // chunk of words (one 16-site word a thread, whose weights it holds as bit
 // planes) through a run of queries, so that the weights are read once a run and
 // a word of P_c once for the neighbouring queries of one c; the waves' sums meet
 // in LDS.  Bound by VALU issue (80%; 6 TB/s of rows from the L2, 97% of them
-// hits): 128 taxa, 20,011 weighted sites,
-// 61,976 queries take 190 us; one block per query over all words, with a
-// dependent weight load for each flagged site, took 522.
+// hits): 128 taxa, 20,011 weighted sites, 61,976 queries take 190 us, a block per
+// query (k_fitch_insert_each) 540.
 constexpr int kMaxRun = 64;
 
 __global__ __launch_bounds__(256) void k_fitch_insert(const uint64_t* __restrict__ pre,
@@ -1160,12 +1192,29 @@ int phy_fitch_insertion_costs(phy_ctx* ctx, const uint64_t* pre, const uint64_t*
   if (n_q == 0) return PHY_OK;
   if (n_q > 0x7fffffff) return set_err(ctx, PHY_ERANGE, "insertion costs: too many queries");
   if (W == 0) return phy_zero_u64(ctx, d_costs, n_q);
-  // one wave for each 64 words up to 4; runs of up to 64 queries, shorter where
+  // Runs: one wave for each 64 words up to 4; runs of up to 64 queries, shorter where
   // that would leave fewer than 2,048 blocks (8 a CU): a longer run reads its
   // weights for more queries, but a CU without a block reads nothing
   const int bs = (int)std::min<int64_t>(256, (W + 63) / 64 * 64);
   const int64_t chunks = std::min<int64_t>((W + bs - 1) / bs, 0xffff);  // a block takes several beyond that
   const int run = (int)std::max<int64_t>(1, std::min<int64_t>(kMaxRun, n_q * chunks / 2048));
+  // Without weights a run saves the reads of P_c and fills small blocks, but pays a
+  // wave sum per query and chunk: worth it for one chunk of words only.  With
+  // weights it has to be long enough to pay for its planes (~300 instructions a
+  // word).  A block per query and runs, us, unweighted: 64 taxa (14,714 queries) x
+  // 1,000 sites 10.5 / 6.3, x 5,000 15 / 22, 128 (61,976) x 4,000 49 / 39, x 20,011
+  // 135 / 153; weighted: 24 (1,812) x 5,000 6.5 / 26 (runs of 1), 50 (8,856) x 1,000
+  // 10.8 / 9.5 (of 4), x 2,500 14.5 / 20 (4), x 5,000 22 / 27 (8), 64 x 2,500 23 / 22
+  // (7), x 5,000 37 / 34 (14), 24 x 50,000 35 / 34 (11), 64 x 20,000 139 / 63 (35).
+  // PHY_FITCH_INSERT=0|1 takes the one or the other.
+  const char* e = getenv("PHY_FITCH_INSERT");
+  const bool runs = e ? e[0] != '0' : wt ? run >= (chunks > 1 ? 11 : 3 + bs / 64) : chunks == 1;
+  if (!runs) {
+    hipLaunchKernelGGL(k_fitch_insert_each, dim3((unsigned)n_q), dim3(256), 0, ctx->stream, pre, fin, stride, W, n_sites,
+                       wt, d_q, (unsigned long long*)d_costs);
+    PHY_LAUNCHED(ctx);
+    return PHY_OK;
+  }
   int rc;
   if (chunks > 1 && (rc = phy_zero_u64(ctx, d_costs, n_q))) return rc;
   hipLaunchKernelGGL(k_fitch_insert, dim3((unsigned)((n_q + run - 1) / run), (unsigned)chunks), dim3(bs), 0,

@@ -215,10 +215,11 @@ def test_pass_shapes_and_node_costs(ctx, rng, N, S, weights):
 
 @pytest.mark.parametrize("S", [1, 1025, 4111, 70_003])
 @pytest.mark.parametrize("weights", ["unit", "small", "heavy"])
-def test_insertion_costs_match_oracle(ctx, rng, S, weights):
+def test_insertion_costs_match_oracle(ctx, rng, monkeypatch, S, weights):
     # one wave to several chunks of words a query, runs that share or change
     # the inserted node, one query and more than a run, weights by bit planes
-    # or walked
+    # or walked; a block per query, runs, and the choice between them on both
+    # sides of its line (many queries)
     from phylocaml_amd import device as D
     from phylocaml_amd._lib import lib
 
@@ -233,16 +234,20 @@ def test_insertion_costs_match_oracle(ctx, rng, S, weights):
                      np.tile(np.arange(rows), 81)], 1).astype(np.int32)
     pairs = {(a, b): O.fitch_median2(sets[1][a], sets[1][b])[0] for a in range(rows)
              for b in range(rows)}
-    for n in (1, 65, len(allq)):
-        q = allq[:n]
-        _say(f"insertion costs S={S} {weights} n={n}")
-        dq = D.to_device(np.ascontiguousarray(q), ctx.device)
+    ww = np.ones(S, np.int64) if w is None else w.astype(np.int64)
+    want = [int(ww[(sets[0][c] & pairs[a, b]) == 0].sum()) for c, a, b in allq.tolist()]
+    many = np.tile(allq, (25, 1))
+    for n, form in ((1, "0"), (1, "1"), (65, "0"), (65, "1"), (729, "0"), (729, "1"), (729, None),
+                    (25 * 729, None), (25 * 729 - 3, "1")):
+        monkeypatch.delenv("PHY_FITCH_INSERT", raising=False)
+        if form:
+            monkeypatch.setenv("PHY_FITCH_INSERT", form)
+        _say(f"insertion costs S={S} {weights} n={n} form {form}")
+        dq = D.to_device(np.ascontiguousarray(many[:n]), ctx.device)
         out = torch.full((n,), 7, dtype=torch.int64, device="cuda")
         ctx.check(lib.phy_fitch_insertion_costs(ctx.handle, D.dptr(pre), D.dptr(fin), D.words(S), S,
                                                 D.dptr(wd), n, D.dptr(dq), D.dptr(out)), "insertion")
-        ww = np.ones(S, np.int64) if w is None else w.astype(np.int64)
-        want = [int(ww[(sets[0][c] & pairs[a, b]) == 0].sum()) for c, a, b in q.tolist()]
-        assert out.cpu().tolist() == want
+        assert out.cpu().tolist() == (want * 25)[:n]
 
 
 @pytest.mark.parametrize("N", [24, 64, 127])
