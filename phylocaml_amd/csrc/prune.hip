@@ -1068,7 +1068,7 @@ __global__ __launch_bounds__(256, sizeof(real) == 8 ? 3 : 1) void k_prune_deriv(
   real accM[4] = {(real)0, (real)0, (real)0, (real)0};
   int accE = 0;
   int sp = 0;
-  for_each_entry_ahead(prog, n_ops, [&](int i, const int4 op, const int4 on) {
+  for_each_entry_ahead<true>(prog, n_ops, [&](int i, const int4 op, const int4 on) {
     real Dn[8], En[8];
     int Xn[2] = {0, 0};
     const bool more = i + 1 < n_ops;

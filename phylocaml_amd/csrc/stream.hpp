@@ -37,7 +37,9 @@ __device__ __forceinline__ void static_for(F&& f) {
 // The Fitch down-pass over 301 taxa x 600,000 sites took 74.5 us so, 60.8 with
 // it (1,024 x 100,000: 58.9 and 51.0).  At 1,024 x 10^6, where the HBM is the
 // bound and 8 waves per SIMD wait for it, the held-back form keeps fewer rows
-// open at a time and is the faster one, 244 against 254 us: PACED.
+// open at a time and is the faster one, 244 against 254 us: PACED.  So it is in
+// the derivative pass, lnL + d1/d2, FP32 at 512 taxa x 30,000 patterns, R = 2 and 4:
+// 1,030 and 1,330 us against 1,115 and 1,418; FP64, R = 1: 1,300 against 1,382.
 __device__ __forceinline__ void landed(int4& e) {
   asm volatile("" : "+v"(e.x), "+v"(e.y), "+v"(e.z), "+v"(e.w));
 }
@@ -71,7 +73,7 @@ __device__ __forceinline__ void for_each_entry(const int4* __restrict__ prog, in
 struct NoMark {
   __device__ __forceinline__ void operator()(int4&) const {}
 };
-template <class F, class M = NoMark>
+template <bool PACED = false, class F, class M = NoMark>
 __device__ __forceinline__ void for_each_entry_ahead(const int4* __restrict__ prog, int n_ops, F&& f, M&& mark = M()) {
   if (n_ops <= 0) return;
   const int lane = threadIdx.x & 63;
@@ -79,7 +81,7 @@ __device__ __forceinline__ void for_each_entry_ahead(const int4* __restrict__ pr
   int4 nxt = prog[min(64 + lane, n_ops - 1)];
   for (int base = 0; base < n_ops; base += 64) {
     const int cnt = __builtin_amdgcn_readfirstlane(min(64, n_ops - base));  // wave-uniform
-    landed(cur);
+    if constexpr (!PACED) landed(cur);
     mark(cur);
     for (int j = 0; j < cnt; ++j) {
       int4 op, on;
