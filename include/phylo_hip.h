@@ -222,7 +222,7 @@ int phy_fitch_insertion_costs(phy_ctx* ctx, const uint64_t* d_pre, const uint64_
  *   d_node_cost (nullable) N-1 uint64: weighted local cost of each internal
  *               node N+k (NonAdditive_c.t.cost of that node).
  *   d_total     1 uint64: sum_s w_s site_cost_s.
- * A tree of >= 24 leaves may run split (parts side by side, then the top).
+ * A tree of >= 32 leaves may run split (parts side by side, then the top).
  * From 128 leaves on, passes over many sites keep the per-part site counts in a
  * device buffer owned by the topology, allocated on the first such call and
  * grown with n_sites, so two down-passes of one such topology must not run at

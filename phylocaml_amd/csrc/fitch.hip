@@ -897,10 +897,14 @@ struct PassShape {
   int words, block;
 };
 
-// the fine split, if there is one that the pass can take (down, a site's total is
-// added up in 16 bits: add_counts)
+// The fine split, if there is one that the pass can take: down, a site's total is
+// added up in 16 bits (add_counts), and trees below 32 leaves do not pay for the
+// second launch (28 x 2,000 to 400,000 sites, whole and split: 12.5 / 12.6 to 17.0 /
+// 17.9 us, 24: 11.1 / 11.8 to 16.0 / 17.5; 32: 13.1 / 11.9 to 18.4 / 19.1; 40: 15.6 /
+// 13.3 to 20.6 / 19.4).
 const FitchSplit* fine_split(const phy_topo* t, bool up) {
-  return t->fitch_fine && t->fine.down.d_prog && (up || t->n_leaves <= 65536) ? &t->fine : nullptr;
+  return t->fitch_fine && t->fine.down.d_prog && (up || (t->n_leaves >= 32 && t->n_leaves <= 65536)) ? &t->fine
+                                                                                                  : nullptr;
 }
 
 // A pass with few waves is bound by its longest chain of nodes (0.3-0.9 us a
