@@ -922,7 +922,7 @@ const FitchSplit* fine_split(const phy_topo* t, bool up) {
 // 600,000: 102 against 96).  Trees below 24 leaves run whole (16 x 2,000 down:
 // 8.5 whole, 10.8 split).  (The down figures are with part counts in scratch rows;
 // added up in site_cost they are within 4% or lower.)
-PassShape pass_shape(const phy_topo* t, int64_t W32, bool up) {
+PassShape pass_shape(const phy_topo* t, int64_t W32, bool up, bool node_costs = false) {
   const char* e = getenv("PHY_FITCH_SPLIT");
   const bool may_split = !(e && e[0] == '0');
   const FitchSplit* coarse = may_split && t->split.parts.size() >= 2 && t->split.down.d_prog ? &t->split : nullptr;
@@ -935,6 +935,10 @@ PassShape pass_shape(const phy_topo* t, int64_t W32, bool up) {
     const FitchSplit* f = fine ? fine : coarse;
     return {f, waves(2, f) < 4096 ? 1 : 2, 64};
   }
+  // each block adds its nodes' costs to memory, and the fine split's blocks are
+  // eight times as many: down with node costs, fine and coarse, 128 x 300,000 sites
+  // 60 / 55, 200 x 150,000 42 / 45, x 300,000 67 / 52, x 600,000 123 / 56
+  if (node_costs && coarse && W32 >= 32768) return {coarse, 4, 256};
   if (waves(4, coarse) >= (coarse ? 1024 : 256)) return {coarse, 4, 256};
   return {fine ? fine : coarse, 2, 64};
 }
@@ -1136,7 +1140,7 @@ int phy_fitch_downpass(phy_ctx* ctx, const phy_topo* topo, uint64_t* sets, int64
   auto* tt = reinterpret_cast<unsigned long long*>(total);
   if (W == 0) return downpass_clear(ctx, tt, nc, N, nullptr, 0, 1, 1);
   const int64_t W32 = 2 * W;  // 32-bit lanes
-  PassShape sh = pass_shape(topo, W32, false);
+  PassShape sh = pass_shape(topo, W32, false, node_cost != nullptr);
   if (sh.split == &topo->split && topo->scratch_bytes < scratch_need(topo, W32) && capturing(ctx))
     sh.split = fine_split(topo, false);
   const FitchSplit* split = sh.split;

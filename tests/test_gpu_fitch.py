@@ -195,16 +195,17 @@ def test_empty_and_bad_arguments(ctx):
                                 1) == 1
 
 
-@pytest.mark.parametrize("N,S", [(23, 700), (24, 700), (31, 2100), (32, 2100), (40, 1), (40, 513), (301, 20_011),
-                                 (24, 530_001), (130, 400_003), (256, 4099), (256, 5000), (257, 4103), (257, 4700)])
+@pytest.mark.parametrize("N,S", [(23, 700), (24, 700), (31, 2100), (32, 2100), (40, 1), (40, 513),
+                                 (301, 20_011), (24, 530_001), (130, 200_003), (130, 400_003),
+                                 (256, 4099), (256, 5000), (257, 4103), (257, 4700)])
 @pytest.mark.parametrize("weights", ["unit", "small", "heavy"])
 def test_pass_shapes_and_node_costs(ctx, rng, N, S, weights):
     # both sides of the dispatch lines (whole tree below 24 leaves up and 32
-    # down, fine split
-    # with narrow lanes, its part counts in 8 bits up to 256 leaves and in 16
-    # beyond, or one a word in a last block of few sites, whole tree and wide
-    # lanes at many sites) with node costs counted, weighed by bit planes (up to
-    # 8 bits) or walked (one site of 2^20 makes its wave do so)
+    # down, fine split with narrow lanes, its part counts in 8 bits up to 256
+    # leaves and in 16 beyond, or one a word in a last block of few sites, whole
+    # tree or coarse split and wide lanes at many sites) with node costs counted,
+    # weighed by bit planes (up to 8 bits) or walked (one site of 2^20 makes its
+    # wave do so)
     _say(f"fitch shapes N={N} S={S} weights={weights}")
     ch, root = random_tree(rng, N)
     leaves = rng.integers(1, 16, (N, S)).astype(np.uint8)
