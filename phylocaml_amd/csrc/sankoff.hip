@@ -257,7 +257,11 @@ int sankoff_launch(phy_ctx* ctx, const phy_topo* topo, const int32_t* tcm, const
   // its matrix no longer stays in SGPRs and it has to hold two and three times as
   // many: 301 taxa, K = 7, 100,003 sites 179 us against 175, 5,000 sites 61
   // against 136; 128 taxa, K = 8, 100,003 sites 123 against 118, 50,000 sites 84
-  // against 97.  Under three waves a block it does not pay at all.  Of the
+  // against 97.  At K = 6 half as many again: 300,000 sites, 64 taxa 104 against 110,
+  // 100 taxa 134 against 130, 150 taxa 158 against 147.  Below 48 taxa, whose parts
+  // are a few leaves, from K = 7 on twice that: 40 taxa, K = 7, 200,000 sites 90
+  // against 86, K = 8, 100,000 sites 74 against 72, 50,000 sites 55 against 60.
+  // Under three waves a block it does not pay at all.  Of the
   // numbers of waves the largest serves where every CU has at most one block, the
   // one with the most waves on a CU elsewhere.  PHY_SANKOFF_SPLIT=0: the whole form.
   const FitchSplit& f = topo->fine;
@@ -271,7 +275,8 @@ int sankoff_launch(phy_ctx* ctx, const phy_topo* topo, const int32_t* tcm, const
     if (need > kLdsMax || h <= held || (waves && groups <= 256)) continue;
     waves = w, held = h, lds = need;
   }
-  if ((int64_t)held * 256 > groups * std::max(1, K - 5)) {
+  const int twice = K <= 5 ? 2 : K == 6 ? 3 : 2 * (K - 5) * (topo->n_leaves < 48 ? 2 : 1);  // 2 x the factor
+  if ((int64_t)held * 512 > groups * twice) {
     hipLaunchKernelGGL((k_sankoff_down<K, true>), dim3((unsigned)groups), dim3(64 * waves), lds, ctx->stream,
                        f.down.d_prog, 0, f.down.d_fifo, f.down.d_meta, P, topo->n_leaves, f.down.depth, tcm, tips,
                        stride, n_sites, wt, site_cost, total);
