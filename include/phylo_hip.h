@@ -333,9 +333,9 @@ int phy_lk_tree_work_size(const phy_topo* topo, const phy_model* model,
 /* Whole-tree evaluation (Node.Make1D.median_2 in post-order + root_cost,
  * lib/node.ml:183-198,272), one launch for the partials (PHY_FUSED on a tree
  * of >= 256 leaves that splits into parts: two, the parts side by side and
- * then the top of the tree; in that form, or from 32,768 patterns on, where
- * d_work has room, one before these that forms the products of every node of
- * two leaves; the result is the same bit for bit):
+ * then the top of the tree; in that form, or over many patterns (32,768 and
+ * more), where d_work has room, one before these that forms the products of
+ * every node of two leaves; the result is the same bit for bit):
  *   d_tips     N rows x stride words: tip state sets (nibble blocks; a gap is
  *              all four bits = missing data).
  *   d_weights  n_patterns uint32 pattern weights.

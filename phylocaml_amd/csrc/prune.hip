@@ -2616,12 +2616,16 @@ size_t tab_lds(int R, size_t esz, const TabProg& tp, int lv) {
 // patterns 20.4 / 23.3 and 21.2 / 24.5; 200 x 8,000 84.9 / 92.8 and 92.0 / 96.2;
 // 128 x 32,000 63.7 / 65.1 and 73.2 / 67.4; 32 x 50,000 29.0 / 25.7 and 32.5 / 27.3;
 // 200 x 100,000 183 / 133 and 235 / 173; split: 300 x 500 127 / 114 and 133 / 115;
-// 512 x 4,000 101 / 95 and 109 / 100.  PHY_PRUNE_TAB=0|1 overrides the size rule.
+// 512 x 4,000 101 / 95 and 109 / 100.  Below 48 leaves there has to be work for it,
+// FP32: 16 x 60,000 patterns R = 1 16.8 / 19.9, R = 4 20.1 / 19.9, 16 x 100,000 R = 2
+// 20.8 / 20.6, 32 x 100,000 R = 1 25.8 / 26.8, R = 2 30.6 / 27.1, 48 x 33,000 R = 1 33.2 /
+// 31.2.  PHY_PRUNE_TAB=0|1 overrides the size rule.
 bool use_tables(const phy_topo* t, int R, size_t esz, int64_t n_pat) {
   if (!t->tab.n_progs || !t->tab.d_cherry || t->tab.cherry.empty() || tab_lds(R, esz, t->tab, 0) > kLdsMax) return false;
   const char* s = getenv("PHY_PRUNE_TAB");
   if (s && (s[0] == '0' || s[0] == '1') && s[1] == 0) return s[0] == '1';
-  return t->pparts.size() >= 2 || n_pat >= 32768;
+  return t->pparts.size() >= 2 ||
+         (n_pat >= 32768 && (t->n_leaves >= 48 || (double)t->n_leaves * R * (double)n_pat >= 3.5e6));
 }
 
 Plan make_plan(const phy_topo* t, const phy_model* m, int64_t n_pat, int32_t form, int32_t derivs,
