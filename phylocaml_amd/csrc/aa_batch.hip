@@ -623,18 +623,24 @@ size_t lds_bytes(int waves, int R, int depth, int lv) {
 // workgroup then share its operand copies less often but read each operand
 // from LDS once for 32 patterns: 8.0 against 12.1 ms for the 256 trees above),
 // else one (at 4 groups per tile two waves would copy the 16 KiB of a node:
-// 15.1 against 8.3 ms).
-constexpr int aa_groups(int waves) { return waves == 8 ? 2 : 1; }
+// 15.1 against 8.3 ms).  One too where every CU has at most one workgroup, whose
+// chain of nodes is then the bound (one tree of 200 taxa x 2,000 patterns, R = 4:
+// 258 against 285 us; 12 trees of 64 x 3,000, 259 tiles: 158 against 127), and with
+// two rate classes (64 trees of 200 x 9,000: 1,647 against 1,728; R = 1 1,237
+// against 1,007).
+int aa_groups(int waves, int R, int64_t n_items, int n_cu) {
+  return waves == 8 && R != 2 && n_items > n_cu ? 2 : 1;
+}
 
 // Stack levels kept in registers: none for stacks of 1 or 2 levels (fewer
 // VGPRs), else 3, or 4 with one group per wave for stacks of 5 or more (at 5
 // levels three workgroups of 4 waves then fit a CU's LDS instead of two, and
 // the registers still allow three waves per SIMD: 8.3 against 10.9 ms).
 // PHY_AA_REG=0|3 overrides.
-int aa_register_levels(int depth, int waves) {
+int aa_register_levels(int depth, int groups) {
   const char* s = getenv("PHY_AA_REG");
   if (s && (s[0] == '0' || s[0] == '3') && s[1] == 0) return s[0] - '0';
-  return depth >= 5 && aa_groups(waves) == 1 ? 4 : depth >= 3 ? 3 : 0;
+  return depth >= 5 && groups == 1 ? 4 : depth >= 3 ? 3 : 0;
 }
 
 template <int TW, int G, int R, int LV>
@@ -674,14 +680,22 @@ int launch(phy_ctx* ctx, phy_aa_batch* b) {
   return PHY_OK;
 }
 
-template <int TW, int R>
-int launch_l(phy_ctx* ctx, phy_aa_batch* b) {
-  constexpr int G = aa_groups(TW);
-  switch (aa_register_levels(std::max(1, b->depth), TW)) {
+template <int TW, int G, int R>
+int launch_g(phy_ctx* ctx, phy_aa_batch* b) {
+  switch (aa_register_levels(std::max(1, b->depth), G)) {
     case 0: return launch<TW, G, R, 0>(ctx, b);
     case 3: return launch<TW, G, R, 3>(ctx, b);
     default: return launch<TW, G, R, G == 1 ? 4 : 3>(ctx, b);
   }
+}
+
+template <int TW, int R>
+int launch_l(phy_ctx* ctx, phy_aa_batch* b) {
+  int n_cu = 256;
+  (void)hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, ctx->device);
+  if constexpr (TW == 8 && R != 2)
+    if (aa_groups(TW, R, b->n_items, n_cu) == 2) return launch_g<TW, 2, R>(ctx, b);
+  return launch_g<TW, 1, R>(ctx, b);
 }
 
 template <int R>
@@ -797,7 +811,7 @@ int phy_aa_batch_create(phy_ctx* ctx, int32_t T, const int32_t* n_leaves, const 
   int lds_max = 64 * 1024, dev = 0;
   (void)hipGetDevice(&dev);
   (void)hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
-  const int lv = aa_register_levels(std::max(1, b->depth), waves);
+  const int lv = aa_register_levels(std::max(1, b->depth), waves == 8 ? 2 : 1);  // the larger stack of the two forms
   if (lds_bytes(waves, R, std::max(1, b->depth), lv) + (size_t)2 * 2 * aa_blocks(R) * OPB * sizeof(uint4) > (size_t)lds_max) {
     delete b;
     return set_err(ctx, PHY_ERANGE, "aa_batch: LDS stack too deep for this many waves per workgroup");

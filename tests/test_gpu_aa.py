@@ -229,3 +229,35 @@ def test_sister_cherries_of_short_branches(ctx, t):
     ok = np.isfinite(want)  # a negative entry of P (rounding of its eigen sum) may leave no value
     assert ok.sum() >= 3
     assert np.all(np.abs(got[ok] - want[ok]) <= 1e-6 * np.abs(want[ok]))
+
+
+@pytest.mark.parametrize("R", [1, 2, 4])
+def test_groups_of_a_wave_give_the_same_bits(ctx, R):
+    # at 8 waves a wave takes two groups of 16 patterns where the tiles are more
+    # than the CUs, one otherwise (always at R = 2): the same trees alone and
+    # among many
+    from dataclasses import replace
+
+    from phylocaml_amd import aa
+
+    rng = np.random.default_rng(13)
+    trees = []
+    for k in range(5):
+        t = aa.synth_tree(3000 + k, int(rng.integers(4, 90)), int(rng.integers(200, 900)), n_sim=200)
+        if R != 4:
+            t = replace(t, rates=np.array([0.4, 1.6])[:R] if R > 1 else np.ones(1),
+                        probs=np.full(R, 1.0 / R))
+        trees.append(t)
+    print(f"aa groups R={R}", flush=True)
+    got = []
+    for copies in (1, 40):
+        b = aa.AABatch(ctx, trees * copies, waves=8)
+        assert (b.n_items > 512) == (copies > 1) and (copies > 1 or b.n_items <= 64)
+        b.run()
+        ctx.sync()
+        got.append(b.lnl.cpu().numpy().reshape(copies, -1))
+        b.close()
+    assert np.array_equal(got[1], np.repeat(got[0], 40, 0))
+    for k, t in enumerate(trees):
+        ov = _oracle(t)
+        assert abs(got[0][0, k] - ov) <= 2e-3 * abs(ov)
