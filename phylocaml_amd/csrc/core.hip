@@ -18,7 +18,6 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
-#include <functional>
 
 #include "common.hpp"
 
@@ -189,9 +188,10 @@ int phy_copy_d2h(phy_ctx* ctx, void* h_dst, const void* d_src, size_t bytes) {
 // ---------------------------------------------------------------------------
 namespace {
 
-using Stop = std::function<bool(int32_t)>;  // nodes compiled as leaves
+// `stop` below is a predicate on nodes: those compiled as leaves.
 
 // post-order of the subtree under `top`, stop nodes as leaves
+template <class Stop>
 void post_order(int32_t N, int32_t top, const std::vector<int32_t>& ch, const Stop& stop,
                 std::vector<int32_t>* post) {
   post->clear();
@@ -213,11 +213,15 @@ void post_order(int32_t N, int32_t top, const std::vector<int32_t>& ch, const St
 
 // Post-order program of the subtree under `top` with an accumulator and a
 // stack (Sethi-Ullman order); returns false on an internal inconsistency.
+// `need` is scratch of 2N - 1 entries, which the programs of one topology share
+// (clearing one for each of the ~60 made that the larger part at 10,000 leaves).
+template <class Stop>
 bool compile_down(int32_t N, const std::vector<int32_t>& ch, int32_t top, const Stop& stop,
-                  std::vector<int32_t>* prog, std::vector<int32_t>* fifo, int32_t* depth_out) {
+                  std::vector<int32_t>* prog, std::vector<int32_t>* fifo, int32_t* depth_out,
+                  std::vector<int32_t>& need) {
   std::vector<int32_t> post;
   post_order(N, top, ch, stop, &post);
-  std::vector<int32_t> need(2 * N - 1, 0);
+  need.resize(2 * N - 1);
   for (int32_t v : post) {
     if (stop(v)) continue;
     const int32_t a = ch[2 * (v - N)], b = ch[2 * (v - N) + 1];
@@ -281,6 +285,7 @@ bool compile_down(int32_t N, const std::vector<int32_t>& ch, int32_t top, const 
 // node (left to the program of its own part).  The first entry reads the
 // subtree root's set from the fifo with source `first_src` (SRC_LEAF at the
 // tree root: F = P; SRC_EXT at a cut node: the parent's final from memory).
+template <class Stop>
 bool compile_up(int32_t N, const std::vector<int32_t>& ch, const std::vector<int32_t>& size,
                 int32_t top, const Stop& stop, int first_src, std::vector<int32_t>* prog,
                 std::vector<int32_t>* fifo, int32_t* depth_out) {
@@ -366,13 +371,15 @@ int compile_tab(const phy_topo* t, const std::vector<int32_t>& tops, TabProg* ou
   const std::vector<int32_t>& ch = t->children;
   *out = TabProg();
   auto cherry = [&](int32_t v) { return v >= N && ch[2 * (v - N)] < N && ch[2 * (v - N) + 1] < N; };
-  const Stop stop = [N, &cherry](int32_t v) { return v < N || cherry(v); };
+  const auto stop = [N, &cherry](int32_t v) { return v < N || cherry(v); };
   TabProg tp;
-  std::vector<int32_t> pg, ff;
+  std::vector<int32_t> pg, ff, need;
+  tp.sp.prog.reserve(4 * (size_t)N);
+  tp.sp.fifo.reserve(2 * (size_t)N);
   int32_t d = 0;
   for (int32_t top : tops) {
     if (stop(top)) return 0;
-    if (!compile_down(N, ch, top, stop, &pg, &ff, &d)) return 11;
+    if (!compile_down(N, ch, top, stop, &pg, &ff, &d, need)) return 11;
     std::vector<int32_t> rows, prog;  // rows: leaf pairs
     int32_t leaves = 0;
     auto operand = [&](int32_t v, int src, int32_t* slot) {
@@ -412,7 +419,7 @@ int compile_tab(const phy_topo* t, const std::vector<int32_t>& tops, TabProg* ou
     tp.max_rows = std::max(tp.max_rows, tp.n_rows.back());
     ++tp.n_progs;
   }
-  *out = tp;
+  *out = std::move(tp);
   return 0;
 }
 
@@ -423,17 +430,21 @@ int compile_tab(const phy_topo* t, const std::vector<int32_t>& tops, TabProg* ou
 int compile_fitch_split(const phy_topo* t, int want, int32_t min_leaves, FitchSplit* out, bool slots = false) {
   const int32_t N = t->n_leaves, M = 2 * N - 1;
   const std::vector<int32_t>& ch = t->children;
-  const Stop is_leaf = [N](int32_t v) { return v < N; };
+  const auto is_leaf = [N](int32_t v) { return v < N; };
   *out = FitchSplit();
   if (want < 2) return 0;
   const std::vector<int32_t> cuts = choose_cuts(N, ch, t->subtree, t->root, want, min_leaves);
   if (cuts.size() < 2) return 0;
   std::vector<char> is_cut(M, 0);
   for (int32_t c : cuts) is_cut[c] = 1;
-  const Stop stop_top = [N, &is_cut](int32_t v) { return v < N || is_cut[v]; };
+  const auto stop_top = [N, &is_cut](int32_t v) { return v < N || is_cut[v]; };
   SplitProg& sd = out->down;
   SplitProg& su = out->up;
-  std::vector<int32_t> pg, ff;
+  std::vector<int32_t> pg, ff, need;
+  for (SplitProg* sp : {&sd, &su}) {
+    sp->prog.reserve(4 * (size_t)N);
+    sp->fifo.reserve(2 * (size_t)N + 256 * cuts.size());
+  }
   int32_t d = 0, n_ops = 0;
   auto add = [&](SplitProg& sp) {
     sp.prog_off.push_back((int32_t)sp.prog.size() / 4);
@@ -448,10 +459,10 @@ int compile_fitch_split(const phy_topo* t, int want, int32_t min_leaves, FitchSp
   };
   // down: parts first, then the top (cut nodes read as leaves)
   for (int32_t c : cuts) {
-    if (!compile_down(N, ch, c, is_leaf, &pg, &ff, &d)) return 4;
+    if (!compile_down(N, ch, c, is_leaf, &pg, &ff, &d, need)) return 4;
     add(sd);
   }
-  if (!compile_down(N, ch, t->root, stop_top, &pg, &ff, &d)) return 4;
+  if (!compile_down(N, ch, t->root, stop_top, &pg, &ff, &d, need)) return 4;
   if (slots) {
     std::vector<int32_t> slot(M, 0);
     for (size_t k = 0; k < cuts.size(); ++k) slot[cuts[k]] = (int32_t)k + 1;
@@ -479,10 +490,10 @@ void phy_compile_up_program(int32_t N, const std::vector<int32_t>& ch, const std
                             const std::vector<char>* enter) {
   std::vector<int32_t> fifo;
   if (enter) {
-    const Stop cut = [N, enter](int32_t v) { return v < N || !(*enter)[v]; };
+    const auto cut = [N, enter](int32_t v) { return v < N || !(*enter)[v]; };
     compile_up(N, ch, size, top, cut, SRC_LEAF, prog, &fifo, depth);
   } else {
-    const Stop is_leaf = [N](int32_t v) { return v < N; };
+    const auto is_leaf = [N](int32_t v) { return v < N; };
     compile_up(N, ch, size, top, is_leaf, SRC_LEAF, prog, &fifo, depth);
   }
 }
@@ -490,14 +501,15 @@ void phy_compile_up_program(int32_t N, const std::vector<int32_t>& ch, const std
 int phy_compile_topo(phy_topo* t) {
   const int32_t N = t->n_leaves, M = 2 * N - 1;
   const std::vector<int32_t>& ch = t->children;
-  const Stop is_leaf = [N](int32_t v) { return v < N; };
+  const auto is_leaf = [N](int32_t v) { return v < N; };
   std::vector<int32_t> post;
   post_order(N, t->root, ch, is_leaf, &post);
   if ((int32_t)post.size() != M) return 1;
   t->subtree.assign(M, 0);
   for (int32_t v : post)
     t->subtree[v] = v < N ? 1 : t->subtree[ch[2 * (v - N)]] + t->subtree[ch[2 * (v - N) + 1]];
-  if (!compile_down(N, ch, t->root, is_leaf, &t->down_prog, &t->down_fifo, &t->down_depth) ||
+  std::vector<int32_t> need;
+  if (!compile_down(N, ch, t->root, is_leaf, &t->down_prog, &t->down_fifo, &t->down_depth, need) ||
       (int32_t)t->down_prog.size() != 4 * (N - 1) || (int32_t)t->down_fifo.size() != N)
     return 2;
   compile_up(N, ch, t->subtree, t->root, is_leaf, SRC_LEAF, &t->up_prog, &t->up_fifo, &t->up_depth);
@@ -532,7 +544,7 @@ int phy_compile_topo(phy_topo* t) {
       std::vector<int32_t> pg, ff;
       int32_t d = 0, n_ops = 0;
       for (int32_t c : cuts) {
-        if (!compile_down(N, ch, c, is_leaf, &pg, &ff, &d)) return 8;
+        if (!compile_down(N, ch, c, is_leaf, &pg, &ff, &d, need)) return 8;
         ps.prog_off.push_back((int32_t)ps.prog.size() / 4);
         ps.n_ops.push_back((int32_t)pg.size() / 4);
         ps.fifo_off.push_back((int32_t)ps.fifo.size());
@@ -545,8 +557,8 @@ int phy_compile_topo(phy_topo* t) {
       }
       // the top: cut nodes stop the walk; their "leaf" operands become
       // stored operands and leave the leaf stream
-      const Stop stop_top = [N, &slot](int32_t v) { return v < N || slot[v] >= 0; };
-      if (!compile_down(N, ch, t->root, stop_top, &pg, &ff, &d)) return 8;
+      const auto stop_top = [N, &slot](int32_t v) { return v < N || slot[v] >= 0; };
+      if (!compile_down(N, ch, t->root, stop_top, &pg, &ff, &d, need)) return 8;
       t->ptop_depth = d;
       n_ops += (int32_t)pg.size() / 4;
       if (n_ops != N - 1) return 9;
@@ -685,6 +697,7 @@ int phy_topo_create(phy_ctx* ctx, int32_t N, const int32_t* children, int32_t ro
   std::copy(t->down_fifo.begin(), t->down_fifo.end(), dfifo.begin());
   std::copy(t->up_fifo.begin(), t->up_fifo.end(), ufifo.begin());
   TopoUpload up;
+  up.all.reserve((size_t)N * 64 + 65536);  // ~12 words a leaf and program set, four sets
   up.put(t->down_prog, &t->d_down_prog);
   up.put(dfifo, &t->d_down_fifo);
   up.put(t->up_prog, &t->d_up_prog);
