@@ -1213,10 +1213,11 @@ int phy_fitch_insertion_costs(phy_ctx* ctx, const uint64_t* pre, const uint64_t*
   // 1,000 sites 10.5 / 6.3, x 5,000 15 / 22, 128 (61,976) x 4,000 49 / 39, x 20,011
   // 135 / 153; weighted: 24 (1,812) x 5,000 6.5 / 26 (runs of 1), 50 (8,856) x 1,000
   // 10.8 / 9.5 (of 4), x 2,500 14.5 / 20 (4), x 5,000 22 / 27 (8), 64 x 2,500 23 / 22
-  // (7), x 5,000 37 / 34 (14), 24 x 50,000 35 / 34 (11), 64 x 20,000 139 / 63 (35).
+  // (7), x 5,000 37 / 34 (14), 43 x 14,085 31 / 32 (12), 40 x 20,000 50 / 37 (13),
+  // 64 x 20,000 139 / 63 (35).
   // PHY_FITCH_INSERT=0|1 takes the one or the other.
   const char* e = getenv("PHY_FITCH_INSERT");
-  const bool runs = e ? e[0] != '0' : wt ? run >= (chunks > 1 ? 11 : 3 + bs / 64) : chunks == 1;
+  const bool runs = e ? e[0] != '0' : wt ? run >= (chunks > 1 ? 13 : 3 + bs / 64) : chunks == 1;
   if (!runs) {
     hipLaunchKernelGGL(k_fitch_insert_each, dim3((unsigned)n_q), dim3(256), 0, ctx->stream, pre, fin, stride, W, n_sites,
                        wt, d_q, (unsigned long long*)d_costs);
