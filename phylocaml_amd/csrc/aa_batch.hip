@@ -27,7 +27,7 @@
 // taxa and 1,000-20,000 patterns take 9.1 ms against 17.1 at 8 groups per tile and
 // 9.8 against 16.2 at 4.  Bound: the node's LDS reads and barrier, with the VALU
 // held 59% and the matrix cores 29% of the time.  The pairs of figures at the rules
-// below compare forms of one earlier state on one box, 8.0 and 8.3 ms there.)
+// below compare forms of one earlier state of the code on one card, 8.0 and 8.3 ms there.)
 // Combining the two children, per-pattern power-of-two rescaling and the root
 // sum are FP32 / FP64 VALU work on 4R + 4 values per lane.  A wave may own G
 // groups of 16 patterns, which share each P operand it reads from LDS.
